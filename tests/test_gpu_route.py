@@ -51,6 +51,63 @@ def test_route_from_x_matches_oracle(gpu, T, d, E, k, x_dtype, r_dtype):
     np.testing.assert_allclose(w.cpu().numpy(), want_w, rtol=2e-6, atol=1e-7)
 
 
+@pytest.mark.parametrize("T,d,E,k,x_dtype,r_dtype,shift", [
+    (220, 7168, 256, 8, "bf16", "f32", 0),    # 128-token tiles, last one ragged
+    (2049, 7168, 256, 8, "f16", "f32", 0),    # 256-token tiles, one token over
+    (1500, 2080, 130, 6, "f32", "f32", 0),    # two experts in the last tile, 65 steps of 32 rows
+    (4096, 2048, 64, 6, "bf16", "bf16", 0),
+    (300, 1408, 1000, 64, "bf16", "f32", 0),  # 16 experts a lane in the selection
+    (1300, 1280, 257, 8, "f16", "bf16", 1),   # x rows not 16-byte aligned
+    (12600, 32, 1000, 1, "f32", "bf16", 1),   # a slice is one step
+])
+def test_route_long_batches_against_float64(gpu, T, d, E, k, x_dtype, r_dtype, shift):
+    """The split-operand logits: fp32 sums of exact bf16 products, so the error
+    of a logit stays a few 2^-24 of sum |x w| (|x| |w| sqrt(d) here), and the
+    selection is the oracle's on the same logits."""
+    import torch
+
+    tdt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+    gen = torch.Generator(device="cuda").manual_seed(T + E)
+    x = torch.randn(T * d + shift, generator=gen, device="cuda").to(tdt[x_dtype])[shift:].view(T, d)
+    W = (torch.randn((d, E), generator=gen, device="cuda") / d ** 0.5).to(tdt[r_dtype])
+    logits = torch.empty((T, E), dtype=torch.float32, device="cuda")
+    ids, w = gpu.route(k, x=x, router=W, logits_out=logits)
+    want = x.double() @ W.double()
+    scale = x.double().abs() @ W.double().abs()
+    assert float(((logits.double() - want).abs() / scale).max()) <= 8 * 2.0 ** -24
+    assert float((logits.double() - want).norm() / want.norm()) <= 3e-7
+    want_ids, want_w = routing.softmax_topk(logits.cpu().numpy(), k)
+    assert np.array_equal(ids.cpu().numpy(), want_ids)
+    np.testing.assert_allclose(w.cpu().numpy(), want_w, rtol=2e-6, atol=1e-7)
+
+
+def test_route_long_batches_non_finite(gpu):
+    """A non-finite operand spoils its own tokens or experts only, as a plain
+    fp32 sum has it: inf stays inf, inf - inf and NaN are NaN and never chosen."""
+    import torch
+
+    T, d, E, k = 230, 7168, 256, 8
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn((T, d), generator=gen, device="cuda")
+    W = torch.randn((d, E), generator=gen, device="cuda") / d ** 0.5
+    W[:, 17] = W[:, 17].abs()
+    x[5, 100] = float("inf")
+    x[7, 3] = float("nan")
+    W[9, 40] = float("-inf")
+    logits = torch.empty((T, E), dtype=torch.float32, device="cuda")
+    ids, _ = gpu.route(k, x=x, router=W, logits_out=logits)
+    want = x.double() @ W.double()
+    nan = torch.isnan(want)
+    assert torch.equal(torch.isnan(logits), nan) and float(logits[5, 17]) == float("inf")
+    fin = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(logits), fin)
+    assert float((logits.double() - want)[fin].abs().max()) <= 1e-5
+    got = ids.cpu().numpy()
+    chosen = torch.gather(nan, 1, ids.long().clamp(min=0)).cpu().numpy()
+    rows = nan.sum(1).cpu().numpy() < E - k
+    assert not chosen[rows].any() and (got[rows] >= 0).all()
+
+
 @pytest.mark.parametrize("drop,param", [("none", 0.0), ("below", 0.05), ("below", 0.2), ("inclusive", 0.95),
                                         ("inclusive", 0.5)])
 def test_route_from_logits_drop_rules(gpu, drop, param):
