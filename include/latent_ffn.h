@@ -226,8 +226,8 @@ int latent_moe_check(void* workspace, size_t workspace_bytes, latent_stream_t st
  *       factor has INT8 groups: at least 16 routed pairs, max_rank <= 512,
  *       16-byte aligned x (per-expert ranks allowed); factors decoded into
  *       LDS chunk by chunk;
- *   1 = single persistent fp32 decode kernel: row layout, 32 to 512 routed
- *       pairs, 2 * max_rank <= 1024, 16-byte aligned x (INT8 groups allowed);
+ *   1 = fp32 matrix-core chain: row layout, 32 to 512 routed pairs, at most
+ *       512 experts, 16-byte aligned x (INT8 groups allowed); bit-reproducible;
  *   4 = as above, for the pure-NF4 calls path 1 does not take;
  *   0 = multi-kernel fp32 GEMV path: any call on the row layout.
  * A call in the tile layout that neither path 2 nor 3 takes is

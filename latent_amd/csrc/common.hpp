@@ -15,6 +15,13 @@ constexpr int kGroup = 32;     // elements per quantization group (one row segme
 constexpr int kGroupBytes = 16; // NF4 bytes of a group: one 128-bit load
 constexpr int kWave = 64;
 
+// Workspace bytes at the start of every workspace that are zero between calls
+// (the small-batch streaming chain's counters), and the byte offset in them of
+// the int error word a timed-out bounded wait sets (read and cleared by
+// latent_moe_check).
+constexpr size_t kControlBytes = 256 * 1024;
+constexpr size_t kErrorOffset = 36;
+
 // The 16 NF4 levels, loader/latent_loader.py:28-48.  Identical float literals,
 // so each rounds to the same binary32 value as np.float32(literal).
 __host__ __device__ constexpr float nf4_level(int c) {

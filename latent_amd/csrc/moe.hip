@@ -19,8 +19,8 @@
 // by the group scale once and then by 32 codebook levels read from a 16-entry
 // LDS table.  Lanes sharing a group are combined with wave shuffles, waves
 // through LDS, workgroups with fp32 atomics.  All arithmetic is fp32.
+#include "chain32.hpp"
 #include "common.hpp"
-#include "fused.hpp"
 #include "prefill.hpp"
 #include "rows.hpp"
 #include "stream.hpp"
@@ -67,9 +67,10 @@ struct MoeParams {
   float* pair_w;
   float* gu;  // [P][2R]
   float* dl;  // [P][R]
-  int4* unit_info;  // streaming path work units {expert, first pair, pairs, 0} (NULL: not built)
-  int* unit_tok;    // [units][16] token of each unit row (0 past the unit's pairs)
-  int* pos_of;      // [T*K] grouped position of each routed slot (streaming path)
+  int4* unit_info;  // work units {expert, first pair, pairs, 0} (NULL: not built)
+  int unit_shift;   // a unit holds at most 1 << unit_shift pairs of one expert
+  int* unit_tok;    // [units][1 << unit_shift] token of each unit row (0 past the unit's pairs)
+  int* pos_of;      // [T*K] grouped position of each routed slot (with units)
   _Float16* xh;     // streaming path: x as fp16 rows * 2^xexp (NULL: not converted)
   int* xexp;        // [T] row exponents
   int x_dtype, w_dtype;
@@ -121,8 +122,7 @@ __device__ __forceinline__ void place_pair(const MoeParams& p, const int* start,
   p.pair_w[pos] = w;
   if (p.unit_info) {
     const int rel = pos - start[e];
-    const int row = (ubase[e] + rel / stream::kMaxM) * stream::kMaxM + rel % stream::kMaxM;
-    p.unit_tok[row] = tok;
+    p.unit_tok[(ubase[e] << p.unit_shift) + rel] = tok;
     p.pos_of[i] = pos;
   }
 }
@@ -179,11 +179,12 @@ __device__ void route_block(const MoeParams& p) {
   // Block scan over experts: each thread owns a contiguous run of experts.
   const int per = (p.E + kRouteThreads - 1) / kRouteThreads;
   const int e0 = min(p.E, tid * per), e1 = min(p.E, e0 + per);
+  const int um = 1 << p.unit_shift;
   int sc = 0, sa = 0, su = 0;
   for (int e = e0; e < e1; ++e) {
     sc += cnt[e];
     sa += cnt[e] > 0;
-    su += (cnt[e] + stream::kMaxM - 1) / stream::kMaxM;
+    su += (cnt[e] + um - 1) >> p.unit_shift;
   }
   // Inclusive scan: within the wave by shuffles, then across the waves'
   // totals.
@@ -219,12 +220,12 @@ __device__ void route_block(const MoeParams& p) {
       p.act_expert[act] = e;
       p.act_start[act] = start;
       p.act_count[act] = c;
-      if (p.unit_info) {  // units of at most kMaxM pairs of one expert; rows past the pairs are padding
-        for (int j = 0; j < c; j += stream::kMaxM, ++unit) {
-          const int m = min(stream::kMaxM, c - j);
+      if (p.unit_info) {  // units of one expert; rows past the pairs are padding
+        for (int j = 0; j < c; j += um, ++unit) {
+          const int m = min(um, c - j);
           p.unit_info[unit] = make_int4(e, start + j, m, 0);
-          for (int r = m; r < stream::kMaxM; ++r) {
-            p.unit_tok[unit * stream::kMaxM + r] = 0;
+          for (int r = m; r < um; ++r) {
+            p.unit_tok[unit * um + r] = 0;
           }
         }
       }
@@ -236,7 +237,7 @@ __device__ void route_block(const MoeParams& p) {
     p.meta[0] = ia;
     p.meta[1] = bad;
     p.meta[3] = ic;  // routed pairs
-    p.meta[4] = iu;  // streaming work units
+    p.meta[4] = iu;  // work units
   }
   __syncthreads();
   const int words = (P + 31) / 32;
@@ -952,7 +953,7 @@ enum { kPathGeneral = 0, kPathFused = 1, kPathPrefill = 2, kPathStream = 3, kPat
 // comparisons; the default is the measured fastest supported path.  A layer
 // in the tile layout has only the two MFMA paths (LATENT_E_UNSUPPORTED when
 // neither takes the call).
-int choose_path(const latent_moe_args& a, fused::Plan& pl) {
+int choose_path(const latent_moe_args& a) {
   if (a.layout == LATENT_LAYOUT_TILES) {
     const bool prefill_ok = prefill::supported(a), stream_ok = stream::supported(a);
     const char* env = std::getenv("LATENT_MOE_PATH");
@@ -961,7 +962,7 @@ int choose_path(const latent_moe_args& a, fused::Plan& pl) {
     if (stream_ok) return kPathStream;
     return LATENT_E_UNSUPPORTED;
   }
-  const bool fused_ok = fused::supported(a) && fused::make_plan(a, pl);
+  const bool fused_ok = chain32::supported(a);
   const bool prefill_ok = prefill::supported(a);
   const bool stream_ok = stream::supported(a);
   const bool rows_ok = rows::supported(a);
@@ -976,16 +977,17 @@ int choose_path(const latent_moe_args& a, fused::Plan& pl) {
   // Measured on MI355X at the DeepSeek-V3 shape (d 7168, ff 2048, 256
   // experts, top-8): below the prefill threshold the streaming MFMA path is
   // the fastest wherever it applies (batch 1: 49 vs 52 us for the
-  // multi-kernel path; batch 8: 100 vs 144 us and batch 64: 270 vs 370 us
-  // for the persistent kernel).  On the row layout:
+  // multi-kernel path; batch 8 85 and batch 64 208 us against 109 and 361 us
+  // for the fp32 chain on the row layout of the same layer).  On the row layout:
   //   * with INT8 groups (ranks 64..512, 10 % INT8 groups): the row-layout
   //     MFMA phases from 16 routed pairs (batch 16 / 32 / 64 / 256: 382 /
-  //     567 / 704 / 840 us against 400 / 577 / 830 us for the persistent
-  //     fp32 kernel and 632 / 977 / 1,549 / 3,633 us for the multi-kernel
-  //     path; batch 1: 160 against 134 us, so below 16 pairs the latter);
-  //   * pure NF4 (rank 256): the persistent fp32 kernel where it applies
-  //     (batch 16 / 32 / 64: 189 / 268 / 381 us against 246 / 362 / 495 us
-  //     for the row-layout MFMA phases; batch 8 151 against 154 us).
+  //     567 / 704 / 840 us against 632 / 977 / 1,549 / 3,633 us for the
+  //     multi-kernel path; batch 1: 160 against 134 us, so below 16 pairs the
+  //     latter);
+  //   * pure NF4: the fp32 chain where it applies (rank 256, batch 16 / 32 /
+  //     64: 182 / 272 / 361 us against 246 / 362 / 495 us for the row-layout
+  //     MFMA phases; 64 experts, d 2048, ff 1408, rank 128, top-6, 24 tokens:
+  //     45 us against 177 us for the persistent fp32 kernel it replaced).
   const bool int8 = a.gate_a.int8_bitmap || a.gate_b.int8_bitmap || a.up_a.int8_bitmap || a.up_b.int8_bitmap ||
                     a.down_a.int8_bitmap || a.down_b.int8_bitmap;
   const bool rows_pairs = rows_ok && a.n_tokens * a.n_expert_used >= 16;
@@ -1089,11 +1091,9 @@ extern "C" int latent_moe_workspace_size(const latent_moe_args* args, size_t* by
   const Layout L = layout_for(args->n_tokens, args->n_expert_used, args->n_expert, args->max_rank, xh_cols(*args));
   size_t scratch = L.total;
   if (prefill::supported(*args)) scratch = std::max(scratch, L.gu + prefill::layout_for(*args).total);
-  fused::Plan pl;
-  if (args->layout == LATENT_LAYOUT_ROWS && fused::supported(*args) && fused::make_plan(*args, pl))
-    scratch = std::max(scratch, pl.scratch_bytes);
+  if (chain32::supported(*args)) scratch = std::max(scratch, L.gu + chain32::layout_for(*args).total);
   if (stream::supported(*args)) scratch = std::max(scratch, L.gu + stream::layout_for(*args).total);
-  *bytes = fused::kReserved + align_up(scratch) + int8_word_offset_bytes(*args);
+  *bytes = kControlBytes + align_up(scratch) + int8_word_offset_bytes(*args);
   return LATENT_OK;
 }
 
@@ -1122,15 +1122,15 @@ extern "C" int latent_moe_check(void* workspace, size_t workspace_bytes, latent_
     (void)hipGetLastError();
     const int st = noalloc_scratch(s, &workspace);
     if (st != LATENT_OK) return st;
-  } else if (workspace_bytes < fused::kReserved) {
+  } else if (workspace_bytes < kControlBytes) {
     return LATENT_E_WORKSPACE;
   }
-  int* word = reinterpret_cast<int*>(static_cast<char*>(workspace) + fused::kErrorOffset);
+  int* word = reinterpret_cast<int*>(static_cast<char*>(workspace) + kErrorOffset);
   int h = 0;
   if (hipMemcpyAsync(&h, word, sizeof h, hipMemcpyDeviceToHost, s) != hipSuccess) return LATENT_E_HIP;
   if (hipStreamSynchronize(s) != hipSuccess) return LATENT_E_HIP;
   if (h == 0) return LATENT_OK;
-  const size_t n16 = fused::kReserved / 16;
+  const size_t n16 = kControlBytes / 16;
   hipLaunchKernelGGL(clear_control_kernel, dim3(static_cast<unsigned>((n16 + 255) / 256)), dim3(256), 0, s,
                      static_cast<uint4*>(workspace), n16);
   if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) return LATENT_E_HIP;
@@ -1141,16 +1141,14 @@ extern "C" int latent_moe_path(const latent_moe_args* args) {
   if (!args) return LATENT_E_INVALID;
   const int st = validate(*args);
   if (st != LATENT_OK) return st;
-  fused::Plan pl;
-  return choose_path(*args, pl);
+  return choose_path(*args);
 }
 
 extern "C" int latent_stream_launch(const latent_moe_args* args) {
   if (!args) return LATENT_E_INVALID;
   const int st = validate(*args);
   if (st != LATENT_OK) return st;
-  fused::Plan pl;
-  if (choose_path(*args, pl) != kPathStream) return LATENT_E_UNSUPPORTED;
+  if (choose_path(*args) != kPathStream) return LATENT_E_UNSUPPORTED;
   return stream::lite_applies(*args) ? 2 : 0;
 }
 
@@ -1168,8 +1166,7 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
   if ((reinterpret_cast<uintptr_t>(a.workspace) & (kAlign - 1)) != 0) return LATENT_E_WORKSPACE;
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   (void)hipGetLastError();  // clear a stale error so the checks below see only ours
-  fused::Plan pl;
-  const int path = choose_path(a, pl);
+  const int path = choose_path(a);
   if (path < 0) return path;
   MoeParams p{};
   const latent_factor* fs[6] = {&a.gate_a, &a.gate_b, &a.up_a, &a.up_b, &a.down_a, &a.down_b};
@@ -1186,9 +1183,8 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
     st = set_int8_word_offsets(a, tail, p.fac, s);
     if (st != LATENT_OK) return st;
   }
-  if (path == kPathFused) return fused::forward(a, s, static_cast<char*>(a.workspace), pl, p.fac);
   const Layout L = layout_for(a.n_tokens, a.n_expert_used, a.n_expert, a.max_rank, xh_cols(a));
-  char* ws = static_cast<char*>(a.workspace) + fused::kReserved;
+  char* ws = static_cast<char*>(a.workspace) + kControlBytes;
   p.x = a.x;
   p.ids = a.ids;
   p.weights = a.weights;
@@ -1218,12 +1214,26 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
   const bool use_prefill = path == kPathPrefill;
   const bool use_stream = path == kPathStream;
   if (use_stream && stream::lite_applies(a)) {
-    static_assert(stream::kLiteCtrlOffset + stream::kLiteCtrlBytes <= fused::kReserved, "control block");
+    static_assert(stream::kLiteCtrlOffset + stream::kLiteCtrlBytes <= kControlBytes, "control block");
     return stream::lite_forward(a, static_cast<char*>(a.workspace), ws + L.gu,
-                                reinterpret_cast<int*>(static_cast<char*>(a.workspace) + fused::kErrorOffset), s);
+                                reinterpret_cast<int*>(static_cast<char*>(a.workspace) + kErrorOffset), s);
+  }
+  if (path == kPathFused) {
+    const chain32::Layout CL = chain32::layout_for(a);
+    static_assert(chain32::kUnitPairs == 4, "unit_shift");
+    p.unit_shift = 2;
+    p.unit_info = reinterpret_cast<int4*>(ws + L.gu + CL.units);
+    p.unit_tok = reinterpret_cast<int*>(p.unit_info + chain32::max_units(a));
+    p.pos_of = reinterpret_cast<int*>(ws + L.gu + CL.pos_of);
+    hipLaunchKernelGGL(prep_kernel, dim3(1), dim3(kRouteThreads), 0, s, p);
+    if (hipGetLastError() != hipSuccess) return LATENT_E_HIP;
+    const chain32::Grouping g{p.meta, p.unit_info, p.unit_tok, p.pos_of, p.pair_w};
+    return chain32::forward(a, p.fac, g, ws + L.gu, s);
   }
   if (use_stream) {
     const int64_t mu = stream::max_units(P, a.n_expert);
+    static_assert(stream::kMaxM == 16, "unit_shift");
+    p.unit_shift = 4;
     p.unit_info = reinterpret_cast<int4*>(ws + L.units);
     p.unit_tok = reinterpret_cast<int*>(p.unit_info + mu);
     const stream::Layout SL = stream::layout_for(a);
@@ -1279,7 +1289,7 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
   }
   if (use_stream) {
     const stream::Grouping g{p.meta,      p.unit_info, p.unit_tok, p.pair_tok, p.pair_slot, p.pair_w,
-                             reinterpret_cast<int*>(static_cast<char*>(a.workspace) + fused::kErrorOffset)};
+                             reinterpret_cast<int*>(static_cast<char*>(a.workspace) + kErrorOffset)};
     return stream::forward(a, g, ws + L.gu, s);
   }
   if (use_rows) {

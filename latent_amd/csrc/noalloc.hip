@@ -13,14 +13,13 @@
 // array, so calls that overlap on one GPU (several streams or host threads)
 // race; calls issued in order on one stream do not.
 #include "common.hpp"
-#include "fused.hpp"
 
 #include <mutex>
 
 namespace latent {
 namespace {
 
-static_assert(LATENT_NOALLOC_CONTROL_BYTES == fused::kReserved, "control block size");
+static_assert(LATENT_NOALLOC_CONTROL_BYTES == kControlBytes, "control block size");
 
 constexpr int kMaxDevices = 64;
 
