@@ -82,6 +82,7 @@ struct MoeParams {
   int cd, n_d;           // phase D: d columns per item, items per expert
   int64_t zero_floats;   // accumulator floats cleared by prep
   int zero_out;          // reduced mode: prep clears out (the phase kernels accumulate into it)
+  int longest_first;     // active experts in descending order of work
   int clear;             // prep clears the accumulators (and out) also where it converts x
 };
 
@@ -211,6 +212,25 @@ __device__ void route_block(const MoeParams& p) {
   int start = ic - sc;
   int act = ia - sa;
   int unit = iu - su;
+  if (p.longest_first && per == 1) {
+    // The row-layout MFMA phases launch an expert's items together: experts in
+    // descending order of their work (passes x true ranks), ties by id, so the
+    // long items are not the last to start.  One expert per thread here;
+    // `fill` holds the works until the insert positions replace them.
+    if (sa) {
+      const int work = ((sc + 15) / 16) * (rank_of(p, e0, 0) + rank_of(p, e0, 1) + rank_of(p, e0, 2));
+      fill[act] = work;
+    }
+    __syncthreads();
+    if (sa) {
+      const int mine = fill[act];
+      int pos = 0, total = 0;
+      for (int w = 0; w < kRouteWaves; ++w) total += wave_sum[1][w];
+      for (int j = 0; j < total; ++j) pos += fill[j] > mine || (fill[j] == mine && j < act);
+      act = pos;
+    }
+    __syncthreads();
+  }
   for (int e = e0; e < e1; ++e) {
     const int c = cnt[e];
     fill[e] = start;  // reuse as the running insert position
@@ -942,13 +962,10 @@ int choose_path(const latent_moe_args& a) {
   // multi-kernel path; batch 8 85 and batch 64 208 us against 109 and 361 us
   // for the fp32 chain on the row layout of the same layer).  On the row layout:
   //   * with INT8 groups (ranks 64..512, 10 % INT8 groups): the row-layout
-  //     MFMA phases from 16 routed pairs (batch 16 / 32 / 64 / 256: 382 /
-  //     567 / 704 / 840 us against 632 / 977 / 1,549 / 3,633 us for the
-  //     multi-kernel path; batch 1: 160 against 134 us, so below 16 pairs the
-  //     latter);
+  //     MFMA phases from 16 routed pairs (batch 16 / 64 / 256: 219 / 442 /
+  //     509 us against 632 / 1,549 / 3,633 us for the multi-kernel path);
   //   * pure NF4: the fp32 chain where it applies (rank 256, batch 16 / 32 /
-  //     64: 182 / 272 / 361 us against 246 / 362 / 495 us for the row-layout
-  //     MFMA phases; 64 experts, d 2048, ff 1408, rank 128, top-6, 24 tokens:
+  //     64: 182 / 272 / 361 us; 64 experts, d 2048, ff 1408, rank 128, top-6, 24 tokens:
   //     45 us against 177 us for the persistent fp32 kernel it replaced).
   const bool int8 = a.gate_a.int8_bitmap || a.gate_b.int8_bitmap || a.up_a.int8_bitmap || a.up_b.int8_bitmap ||
                     a.down_a.int8_bitmap || a.down_b.int8_bitmap;
@@ -1207,6 +1224,7 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
   if (use_rows) {
     p.xh = reinterpret_cast<_Float16*>(ws + L.xh);
     p.xexp = reinterpret_cast<int*>(ws + L.xexp);
+    p.longest_first = 1;
   }
   // The MFMA paths write their intermediates whole, and every output row
   // (per-token combine); the row-layout MFMA phases accumulate like the fp32 ones.

@@ -11,26 +11,34 @@
 // kernels/latent_fused_expert_ffn.cu:27-108 for the routed pairs of each
 // active expert; only an expert's true-rank rows and columns are read.
 //
-// Every factor is row-major [K][N] with 32-column groups along N (16 bytes
-// of NF4 codes, low nibble first, or 32 INT8 bytes, and one fp16 scale),
-// while an MFMA operand holds 8 consecutive K values per lane.  So a
-// workgroup decodes a chunk of rows at a time into LDS, transposed: thread
-// (group, row pair) turns its two rows' groups into fp16 values (level x
-// scale or q x scale, one rounding) and stores each column's pair of rows as
-// one dword; the MFMA then reads 16 bytes of one column per lane.  A chunk is
-// 256 such units: ngp groups (the item's groups rounded up to a power of
-// two, 2..16) by 512 / ngp rows, so a chunk is about 8 KB of codes whatever
-// the rank.  The codes, scales, bitmap words and word offsets of chunk c + 2
-// are in flight in registers while chunk c is decoded, and the INT8 bytes of
-// chunk c + 1 (their offsets known one chunk earlier).
+// The factors go from HBM to the matrix cores in rowblock.hpp's blocks of 32
+// rows: a lane holds eight rows of CPL adjacent columns, and the eight values
+// of a column are one operand.  Two rows' nibbles of a column meet in one byte
+// (two shifts and two bit selects per eight columns), a byte table in LDS gives
+// both levels as fp16, one packed product scales them.  An INT8 group's lanes
+// take a zero NF4 scale and add q x scale (one rounding either way).  A lane
+// reloads its rows from the next block as it uses them; the INT8 bytes of the
+// next block are found through bitmap words loaded one block earlier still.
+// No LDS round trip for a factor and no barrier in the loop: decoding chunks
+// transposed through LDS, as this file once did, spent two barriers and 64
+// scattered LDS stores a thread on every 8 KB.  DeepSeek-V3 shape, ranks 64 to
+// 512, 10 % INT8 groups: batch 16 328 -> 219 us, batch 256 751 -> 509 us.
+//
+// What bounds it with INT8 groups: the decode's VALU (about 390 instructions a
+// block of 32 x 128, half of them for the INT8 bytes, which nearly every wave
+// has some of) at three waves per SIMD.  Items of one expert are as long as its
+// rank; the prep kernel lists the experts longest first and phase A cuts an
+// expert's rows into pieces in proportion to its rank, which took batch 16 from
+// 258 to 221 us (a late rank-512 item ran on alone).
 //
 // Activations (x rows, latents, h) enter the MFMA as fp16 rows scaled by a
 // power of two per row (the row maximum into [2^14, 2^15)); products are
 // scaled back in fp32 and summed into the fp32 accumulators of the
 // multi-kernel path with atomics (gu, dl; out for the reduced output), which
-// its prep kernel zeroes.  A pass takes 16 pairs of one expert (one MFMA row
-// block); an expert with more pairs takes several passes.
+// its prep kernel zeroes.  A pass takes MB blocks of 16 pairs of one expert;
+// an expert with more pairs takes several passes.
 #include "common.hpp"
+#include "rowblock.hpp"
 #include "rows.hpp"
 
 #include <algorithm>
@@ -39,55 +47,25 @@ namespace latent {
 namespace rows {
 namespace {
 
+using namespace rowblock;
+
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 enum { F_GATE_A = 0, F_GATE_B, F_UP_A, F_UP_B, F_DOWN_A, F_DOWN_B };
 
 constexpr int kT = 256;            // threads per workgroup (4 waves)
-constexpr int kPass = 16;          // pairs per pass: one MFMA row block
-constexpr int kMaxGroups = 16;     // groups per chunk (512 columns)
 constexpr int kCB = 256;           // BC: ff columns per item
 constexpr int kCD = 512;           // D: d columns per item
-constexpr int kHDw = kCB / 2 + 4;  // BC: dwords per h row (256 halves + 8 pad)
-// Decoded chunk: group blocks of 32 columns of (rows / 2 + 4) dwords; at
-// most 16 x (32 x 20 + 4) dwords (ngp = 16, 32 rows).
-constexpr int kBtDw = kMaxGroups * (32 * 20 + 4);
-constexpr int kActDw = kPass * (256 / 2 + 4);  // activation rows of a chunk of at most 256 rows
-
-// LDS byte address of a __shared__ object and raw LDS accesses.
-template <typename T>
-__device__ __forceinline__ uint32_t lds_addr(T& obj) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)(&obj)));
-}
-template <typename T>
-__device__ __forceinline__ T lds_ld(uint32_t addr) {
-  return *reinterpret_cast<const __attribute__((address_space(3))) T*>(static_cast<uintptr_t>(addr));
-}
-template <typename T>
-__device__ __forceinline__ void lds_st(uint32_t addr, const T& v) {
-  *reinterpret_cast<__attribute__((address_space(3))) T*>(static_cast<uintptr_t>(addr)) = v;
-}
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-
-// Workgroup barrier over LDS only: waits for this wave's LDS accesses, then
-// s_barrier.  (__syncthreads() would also wait for every outstanding global
-// load and drain the chunks loaded ahead.)  Workgroups of these kernels
-// share data through LDS only.
-__device__ __forceinline__ void lds_barrier() {
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0); vmcnt and expcnt left at their maxima
-  __builtin_amdgcn_s_barrier();
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
-// Raw buffer resource over `bytes` bytes (loads beyond them return zero).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), static_cast<short>(0), static_cast<int>(bytes),
-                                           0x00020000);
-}
+constexpr int kHStr = kCB + 8;     // halves per h row
+constexpr int kTileStr = 128 + 4;  // floats per row of a wave's products
+constexpr int kHalfSlot = 8 * kTileStr * 4;  // LDS bytes of eight rows of them
+constexpr int kRedBytes = 4 * kHalfSlot;     // of every wave
+constexpr int kCopies = 16;               // of the level table, by lane
+constexpr int kLutBytes = 256 * kCopies * 4;
+constexpr int kMetaSlot = 256 + 256;         // a block's scales [group][row]; its INT8 words, then offsets
+constexpr int kMetaBytes = 2 * kMetaSlot;    // per wave
+constexpr int kFixBytes = kLutBytes + 4 * kMetaBytes;  // the table, then the waves' meta slots
 
 __device__ __forceinline__ int rank_of(const Params& p, int e, int kind) {
   if (!p.ranks) return p.R;
@@ -104,527 +82,442 @@ __device__ __forceinline__ bool map_item(int b, int n_items, int n_active, int& 
   return a < n_active;
 }
 
-// Level-pair table: entry b = (level(b & 15), level(b >> 4)) as two fp16.
-__device__ __forceinline__ void lut_fill(uint32_t* lut, int tid) {
+// Level-pair table: entry b = (level(b & 15), level(b >> 4)) as two fp16, in
+// kCopies copies so that a wave's random lookups spread over the banks.
+__device__ __forceinline__ void lut_fill(uint32_t lut, int tid) {
   const half2v lv = {static_cast<_Float16>(nf4_level(tid & 15)), static_cast<_Float16>(nf4_level(tid >> 4))};
-  lut[tid] = __builtin_bit_cast(uint32_t, lv);
-}
-
-// Chunk shape for ng groups (a compile-time type, so every LDS offset of a
-// chunk is an immediate): ngp = ng rounded up to a power of two in [2, 16],
-// rows = 512 / ngp; dwords per decoded column cstr = rows / 2 + 4 (16-byte
-// MFMA reads of 8 consecutive columns fall on distinct banks), per group
-// block gstr = 32 cstr + 64 / ngp (the 64 stores of a wave, 64 / ngp row
-// pairs of ngp groups, fall on distinct banks).
-template <int NGP>
-struct Shape {
-  static constexpr int ngp = NGP, rows = 512 / NGP, cstr = rows / 2 + 4, gstr = 32 * cstr + 64 / NGP;
-};
-// The same shape as run-time values (one code path for every shape).
-struct DynShape {
-  int ngp, rows, cstr, gstr;
-};
-__device__ __forceinline__ DynShape dyn_shape(int ng) {
-  int ngp = 2;
-  while (ngp < ng) ngp <<= 1;
-  const int rows = 512 / ngp, cstr = rows / 2 + 4;
-  return DynShape{ngp, rows, cstr, 32 * cstr + 64 / ngp};
-}
-// f(Shape<ngp>{}) for the chunk shape of ng groups.
-template <typename F>
-__device__ __forceinline__ void with_shape(int ng, F&& f) {
-  if (ng <= 2)
-    f(Shape<2>{});
-  else if (ng <= 4)
-    f(Shape<4>{});
-  else if (ng <= 8)
-    f(Shape<8>{});
-  else
-    f(Shape<16>{});
-}
-
-// One thread's decode unit of a chunk: rows r, r + 1 of one group.
-struct Unit {
-  u32x4 c[2];     // codes
-  uint32_t s;     // scales (fp16 bits; row r in the low half)
-  uint32_t w[2];  // INT8 bitmap words
-  int o[2];       // their word offsets
-};
-struct Q {  // the INT8 bytes of the unit's rows (zero where NF4)
-  u32x4 v[2][2];
-};
-
-// One thread's view of a decode source: rows below row_end of groups
-// [g0, g0 + ng) of one expert's factor, in chunks of sh.rows rows from row
-// `base`; the thread's unit is group gi and row pair rp of each chunk.  The
-// expert's codes, scales, bitmap words and word offsets through buffer
-// resources (wave-uniform; 32-bit offsets, zeros past the expert's rows or
-// for a factor without INT8 groups), the INT8 bytes through one over the
-// factor's side buffer.
-struct Src {
-  __amdgpu_buffer_rsrc_t rc, rs, rb, ro, rd;
-  int cs, ss, words;
-  int base, row_end, g0, ng, gi, rp;
-};
-__device__ __forceinline__ Src make_src(const Factor& f, int e, int base, int row_end, int g0, int ng, int gi,
-                                        int rp) {
-  const int64_t er = static_cast<int64_t>(e) * f.rows;
-  const int cs = static_cast<int>(f.code_stride()), ss = static_cast<int>(f.scale_stride()), words = f.words();
-  const bool has8 = f.ext.bitmap != nullptr;
-  const uint32_t rows = static_cast<uint32_t>(f.rows);
-  Src s;
-  s.rc = buffer_rsrc(f.codes + er * cs, rows * cs);
-  s.rs = buffer_rsrc(f.scales + er * ss, rows * ss * 2u);
-  s.rb = buffer_rsrc(has8 ? f.ext.bitmap + er * words : nullptr, has8 ? rows * words * 4u : 0u);
-  s.ro = buffer_rsrc(has8 ? f.ext.word_offset + er * words : nullptr, has8 ? rows * words * 4u : 0u);
-  s.rd = buffer_rsrc(f.ext.data, has8 ? 0x7FFFFFF0u : 0u);
-  s.cs = cs;
-  s.ss = ss;
-  s.words = words;
-  s.base = base;
-  s.row_end = row_end;
-  s.g0 = g0;
-  s.ng = ng;
-  s.gi = gi;
-  s.rp = rp;
-  return s;
-}
-
-// Loads of rows r, r + 1 of group g.
-template <bool kInt8>
-__device__ __forceinline__ void unit_load(const Src& s, int r, int g, Unit& u) {
-  const uint32_t r0 = static_cast<uint32_t>(r), r1 = r0 + 1u;
-  u.c[0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(s.rc, r0 * s.cs + g * kGroupBytes, 0, 0));
-  u.c[1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(s.rc, r1 * s.cs + g * kGroupBytes, 0, 0));
-  const uint32_t s0 = __builtin_amdgcn_raw_buffer_load_b16(s.rs, (r0 * s.ss + g) * 2u, 0, 0);
-  const uint32_t s1 = __builtin_amdgcn_raw_buffer_load_b16(s.rs, (r1 * s.ss + g) * 2u, 0, 0);
-  u.s = s0 | (s1 << 16);
-  if (kInt8) {
-    const uint32_t ws = static_cast<uint32_t>(g >> 5);
-    u.w[0] = __builtin_amdgcn_raw_buffer_load_b32(s.rb, (r0 * s.words + ws) * 4u, 0, 0);
-    u.w[1] = __builtin_amdgcn_raw_buffer_load_b32(s.rb, (r1 * s.words + ws) * 4u, 0, 0);
-    u.o[0] = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(s.ro, (r0 * s.words + ws) * 4u, 0, 0));
-    u.o[1] = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(s.ro, (r1 * s.words + ws) * 4u, 0, 0));
-  }
-}
-
-// The INT8 bytes of a unit's flagged rows (an unflagged row reads past the
-// range and gets zeros: no branch).
-template <bool kInt8>
-__device__ __forceinline__ void q_load(const Src& s, const Unit& u, int g, Q& q) {
-  if (!kInt8) return;
-  const uint32_t bit = 1u << (g & 31);
+  const uint32_t v = __builtin_bit_cast(uint32_t, lv);
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const bool is8 = (u.w[h] & bit) != 0u;
-    const uint32_t off = is8 ? static_cast<uint32_t>(u.o[h] + popc(u.w[h] & (bit - 1u))) * kGroup : 0x80000000u;
-    q.v[h][0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(s.rd, off, 0, 0));
-    q.v[h][1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(s.rd, off + 16u, 0, 0));
-  }
+  for (int i = 0; i < kCopies / 4; ++i) lds_st<u32x4>(lut + tid * (kCopies * 4) + i * 16, u32x4{v, v, v, v});
 }
 
-// Row h of a unit as 16 fp16 pairs (columns 2i, 2i + 1): level x scale or
-// q x scale, rounded once; zeros for a dead row (scale 0: every level and q
-// is finite).  INT8 bytes become fp16 exactly through 0x6400 | (q ^ 0x80) =
-// 1024 + q + 128, less 1152.
-template <bool kInt8>
-__device__ __forceinline__ void unit_row(const Unit& u, const Q& q, int h, int g, bool live, uint32_t lut,
-                                         half2v (&v)[16]) {
-  const _Float16 s = live ? __builtin_bit_cast(_Float16, static_cast<uint16_t>(u.s >> (16 * h)))
-                          : static_cast<_Float16>(0.f);
-  const half2v s2 = {s, s};
-  const bool is8 = kInt8 && ((u.w[h] >> (g & 31)) & 1u);
-  if (is8) {
-    const half2v bias = {static_cast<_Float16>(-1152.f), static_cast<_Float16>(-1152.f)};
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint32_t d = q.v[h][i >> 2][i & 3] ^ 0x80808080u;
-      const uint32_t lo = __builtin_amdgcn_perm(0x64646464u, d, 0x04010400u);  // bytes (d0, 0x64, d1, 0x64)
-      const uint32_t hi = __builtin_amdgcn_perm(0x64646464u, d, 0x04030402u);  // bytes (d2, 0x64, d3, 0x64)
-      v[2 * i] = (__builtin_bit_cast(half2v, lo) + bias) * s2;
-      v[2 * i + 1] = (__builtin_bit_cast(half2v, hi) + bias) * s2;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const uint32_t b = (u.c[h][i >> 2] >> (8 * (i & 3))) & 0xFFu;
-      v[i] = __builtin_bit_cast(half2v, lds_ld<uint32_t>(lut + b * 4)) * s2;
+// A wave's walk over blocks [b0, b1) of 32 rows from `row0` of a factor and
+// 16 CPL columns from col0, times MB blocks of 16 pairs.  start() issues the
+// first loads (as early as the caller can), run() does the rest.
+// act.load(b) issues the loads of block b's activations, act.get(b, mb) gives
+// the lane's eight of pair block mb (zero for rows that do not count).
+//
+// Per block a lane loads the codes of its eight rows and, for INT8 factors,
+// the bytes of its flagged rows; the scales, bitmap words and word offsets,
+// which lanes share, are loaded once per wave, two blocks ahead, and go
+// through wave-private LDS slots (a lane then reads its eight rows' scales as
+// one 16-byte word): loading them per lane and row made two thirds of all
+// load instructions.
+template <int CPL, int MB, bool kInt8, class Act>
+struct Walk {
+  static constexpr int kG = CPL / 4;  // groups a lane loads the scale of
+  static constexpr int kQ = kInt8 ? CPL / 4 : 1;
+  int row0, b0, b1, lane;
+  uint32_t meta;  // LDS address of the wave's meta slots
+  Src<CPL> src;
+  __amdgpu_buffer_rsrc_t rb, ro, rd;  // INT8 bitmap words, word offsets, bytes
+  uint32_t vm, vw, bit, byte, gsc;
+  int wstride;
+  Act act;
+  uint32_t c[8][(CPL + 7) / 8];  // codes of the block
+  uint32_t q[kInt8 ? 8 : 1][kQ];  // its INT8 bytes
+  uint32_t flags;                 // bit i: row i is INT8
+  uint32_t msc[kG], mw, mo;       // meta of the block after the next
+  __device__ __forceinline__ Walk(const Factor& f, int e, int col0, int row0_, int b0_, int b1_, int lane_,
+                                  uint32_t meta_, const Act& act_)
+      : row0(row0_), b0(b0_), b1(b1_), lane(lane_), meta(meta_), src(make_src<CPL>(f, e, col0, lane_)), act(act_),
+        flags(0u) {
+    // Scales: lane -> row lane / 2, half lane & 1 of the tile's groups (groups
+    // past the factor's last belong to columns that are not stored).
+    const int g0 = col0 / kGroup;
+    vm = static_cast<uint32_t>((lane >> 1) * src.ss + (g0 + (lane & 1) * kG) * 2);
+    gsc = static_cast<uint32_t>(src.group - g0) * 64u + static_cast<uint32_t>(lane >> 4) * 16u;
+    if (kInt8) {
+      const int words = f.words();
+      const int64_t er = static_cast<int64_t>(e) * f.rows * words;
+      const bool has = f.ext.bitmap != nullptr;
+      const uint32_t bytes = has ? static_cast<uint32_t>(f.rows) * words * 4u : 0u;
+      rb = buffer_rsrc(has ? f.ext.bitmap + er : nullptr, bytes);
+      ro = buffer_rsrc(has ? f.ext.word_offset + er : nullptr, bytes);
+      rd = buffer_rsrc(f.ext.data, has ? 0x7FFFFFF0u : 0u);
+      wstride = words * 4;
+      vw = static_cast<uint32_t>((lane & 31) * wstride + (g0 >> 5) * 4);
+      bit = 1u << (src.group & 31);
+      byte = static_cast<uint32_t>(min(col0 + CPL * (lane & 15), static_cast<int>(f.cols) - CPL) % kGroup);
     }
   }
-}
-
-// Decode a unit and store it transposed: column j's dword at dst + j cstr
-// holds (row r, row r + 1).
-template <bool kInt8>
-__device__ __forceinline__ void unit_store(const Unit& u, const Q& q, int g, bool live0, bool live1, uint32_t lut,
-                                           uint32_t dst, int cstr) {
-  half2v v0[16], v1[16];
-  unit_row<kInt8>(u, q, 0, g, live0, lut, v0);
-  unit_row<kInt8>(u, q, 1, g, live1, lut, v1);
-  const uint32_t step = static_cast<uint32_t>(cstr) * 4u;
+  __device__ __forceinline__ int row_of(int b) const { return row0 + 32 * max(0, min(b, b1 - 1)); }  // the same loads on every path
+  __device__ __forceinline__ void load_codes(int row, int h) {
+    const int oc = row * src.cs;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const uint32_t a = __builtin_bit_cast(uint32_t, v0[i]), b = __builtin_bit_cast(uint32_t, v1[i]);
-    lds_st<uint32_t>(dst + (2 * i) * step, __builtin_amdgcn_perm(b, a, 0x05040100u));
-    lds_st<uint32_t>(dst + (2 * i + 1) * step, __builtin_amdgcn_perm(b, a, 0x07060302u));
-  }
-}
-
-// The decode ring: units of chunks c .. c + 3 (slots c % 4) and INT8 bytes
-// of chunks c, c + 1 (slots c % 2).  Every chunk issues the same loads
-// (clamped past the last chunk), so the compiler's wait counts hold on every
-// path.
-template <bool kInt8>
-struct Ring {
-  Unit u[4];
-  Q q[2];
-};
-
-template <bool kInt8, class SH>
-__device__ __forceinline__ void ring_issue(const Src& s, SH sh, int c, int nc, Unit& u) {
-  const int g = s.g0 + min(s.gi, s.ng - 1);
-  unit_load<kInt8>(s, s.base + min(c, nc - 1) * sh.rows + 2 * s.rp, g, u);
-}
-template <bool kInt8, class SH>
-__device__ __forceinline__ void ring_store(const Src& s, SH sh, int c, const Unit& u, const Q& q,
-                                           uint32_t lut, uint32_t bt, int block) {
-  if (s.gi >= s.ng) return;
-  const int r = s.base + c * sh.rows + 2 * s.rp;
-  const uint32_t dst = bt + static_cast<uint32_t>(block * sh.gstr + s.rp) * 4u;
-  unit_store<kInt8>(u, q, s.g0 + s.gi, r < s.row_end, r + 1 < s.row_end, lut, dst, sh.cstr);
-}
-
-// MFMA steps of a chunk: acc[j] += act rows . decoded columns of column block
-// cb = cb0 + j * cbs (j < kNcb, cb < ncb), rows / 32 steps of K.  act: LDS
-// byte address of the activation rows (astr dwords apart) at the chunk's
-// first K value.
-template <int kNcb, class SH>
-__device__ __forceinline__ void chunk_mfma(uint32_t act, int astr, uint32_t bt, SH sh, int cb0, int cbs,
-                                           int ncb, int n, int kq, float4v (&acc)[kNcb]) {
-  const int steps = sh.rows / 32;
-  for (int s = 0; s < steps; ++s) {
-    const half8 a = lds_ld<half8>(act + static_cast<uint32_t>(n * astr + s * 16 + kq * 4) * 4u);
-#pragma unroll
-    for (int j = 0; j < kNcb; ++j) {
-      const int cb = cb0 + j * cbs;
-      if (cb < ncb) {
-        const uint32_t col = (cb & 1) * 16 + n;
-        const half8 b = lds_ld<half8>(bt + static_cast<uint32_t>((cb >> 1) * sh.gstr + col * sh.cstr + s * 16 + kq * 4) * 4u);
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc[j], 0, 0, 0);
+    for (int i = 2 * h; i < 2 * h + 2; ++i) {
+      if (CPL == 16) {
+        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(src.rc, src.vc, oc + i * src.cs, 0));
+        c[i][0] = v[0];
+        c[i][(CPL + 7) / 8 - 1] = v[1];
+      } else if (CPL == 8) {
+        c[i][0] = __builtin_amdgcn_raw_buffer_load_b32(src.rc, src.vc, oc + i * src.cs, 0);
+      } else {
+        c[i][0] = __builtin_amdgcn_raw_buffer_load_b16(src.rc, src.vc, oc + i * src.cs, 0);
       }
     }
   }
+  __device__ __forceinline__ void load_meta(int row) {
+#pragma unroll
+    for (int j = 0; j < kG; ++j) msc[j] = __builtin_amdgcn_raw_buffer_load_b16(src.rs, vm + 2 * j, row * src.ss, 0);
+    if (kInt8) {
+      mw = __builtin_amdgcn_raw_buffer_load_b32(rb, vw, row * wstride, 0);
+      mo = __builtin_amdgcn_raw_buffer_load_b32(ro, vw, row * wstride, 0);
+    }
+  }
+  // Slot of block b: scales [group][row], then 32 words, 32 offsets.
+  __device__ __forceinline__ void store_meta(int b) {
+    const uint32_t slot = meta + static_cast<uint32_t>(b & 1) * kMetaSlot;
+#pragma unroll
+    for (int j = 0; j < kG; ++j)
+      lds_st<uint16_t>(slot + static_cast<uint32_t>(((lane & 1) * kG + j) * 64 + (lane >> 1) * 2),
+                       static_cast<uint16_t>(msc[j]));
+    if (kInt8) lds_st<uint32_t>(slot + 256u + 4u * lane, lane < 32 ? mw : mo);
+    __builtin_amdgcn_wave_barrier();
+  }
+  // The INT8 bytes of rows 2 h, 2 h + 1 of block b (its meta stored); an NF4
+  // row reads past the range and gets zeros.
+  __device__ __forceinline__ void load_int8(int b, int h, uint32_t& fl) {
+    if (!kInt8) return;
+    const uint32_t at = meta + static_cast<uint32_t>(b & 1) * kMetaSlot + 256u + 32u * (lane >> 4) + 8u * h;
+    const u32x2 w = lds_ld<u32x2>(at), o = lds_ld<u32x2>(at + 128u);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int i = kInt8 ? 2 * h + j : 0;
+      const bool is8 = (w[j] & bit) != 0u;
+      const uint32_t off = is8 ? (o[j] + popc(w[j] & (bit - 1u))) * kGroup + byte : 0x80000000u;
+      fl |= is8 ? 1u << (2 * h + j) : 0u;
+      if (CPL == 16) {
+        const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rd, off, 0, 0));
+#pragma unroll
+        for (int t = 0; t < kQ; ++t) q[i][t] = v[t & 3];
+      } else if (CPL == 8) {
+        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rd, off, 0, 0));
+#pragma unroll
+        for (int t = 0; t < kQ; ++t) q[i][t] = v[t & 1];
+      } else {
+        q[i][0] = __builtin_amdgcn_raw_buffer_load_b32(rd, off, 0, 0);
+      }
+    }
+  }
+  __device__ __forceinline__ void start() {
+    load_meta(row_of(b0));
+    act.load(max(0, min(b0, b1 - 1)));
+#pragma unroll
+    for (int h = 0; h < 4; ++h) load_codes(row_of(b0), h);
+    store_meta(b0);
+    load_meta(row_of(b0 + 1));
+#pragma unroll
+    for (int h = 0; h < 4; ++h) load_int8(b0, h, flags);
+  }
+  __device__ __forceinline__ void run(uint32_t lut, float4v (&acc)[MB][CPL]) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int j = 0; j < CPL; ++j) acc[mb][j] = float4v{0.f, 0.f, 0.f, 0.f};
+    for (int b = b0; b < b1; ++b) {
+      store_meta(b + 1);
+      load_meta(row_of(b + 2));
+      const u32x4 sc = lds_ld<u32x4>(meta + static_cast<uint32_t>(b & 1) * kMetaSlot + gsc);
+      half8 a[MB];
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) a[mb] = act.get(b, mb);
+      act.load(max(0, min(b + 1, b1 - 1)));
+      uint32_t fl = 0u;
+      constexpr int kHalf = CPL < 8 ? CPL : 8;
+#pragma unroll
+      for (int hc = 0; hc < CPL; hc += kHalf) {  // eight columns at a time
+        // Every level pair of the block first (the scheduling fence keeps the
+        // reads together: left alone, the compiler waited for each one).
+        uint32_t v[4][kHalf];
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const uint32_t d0 = c[2 * h][hc / 8], d1 = c[2 * h + 1][hc / 8];
+          // Bytes of (row 2h, row 2h + 1) nibbles: even columns, odd columns.
+          const uint32_t even = (d0 & 0x0F0F0F0Fu) | ((d1 << 4) & 0xF0F0F0F0u);
+          const uint32_t odd = ((d0 >> 4) & 0x0F0F0F0Fu) | (d1 & 0xF0F0F0F0u);
+#pragma unroll
+          for (int j = 0; j < kHalf; ++j)
+            v[h][j] = lds_ld<uint32_t>(lut + ((((j & 1) ? odd : even) >> (8 * (j >> 1))) & 0xFFu) * (kCopies * 4));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          half2v s = __builtin_bit_cast(half2v, static_cast<uint32_t>(sc[h])), s8 = {};
+          if (kInt8) {
+            const uint32_t m = ((flags >> (2 * h)) & 1u ? 0xFFFFu : 0u) | ((flags >> (2 * h)) & 2u ? 0xFFFF0000u : 0u);
+            s8 = __builtin_bit_cast(half2v, __builtin_bit_cast(uint32_t, s) & m);
+            s = __builtin_bit_cast(half2v, __builtin_bit_cast(uint32_t, s) & ~m);
+          }
+#pragma unroll
+          for (int j = 0; j < kHalf; ++j) {
+            half2v x = __builtin_bit_cast(half2v, v[h][j]);
+            if (kInt8) {
+              // q ^ 0x80 under 0x64: 1024 + q + 128 as fp16, exactly.
+              const int t = kInt8 ? (hc + j) >> 2 : 0;
+              const uint32_t q0 = q[kInt8 ? 2 * h : 0][t] ^ 0x80808080u;
+              const uint32_t q1 = q[kInt8 ? 2 * h + 1 : 0][t] ^ 0x80808080u;
+              const uint32_t pr = __builtin_amdgcn_perm(q1, q0, (j & 2) ? 0x07030602u : 0x05010400u);
+              const half2v bias = {static_cast<_Float16>(-1152.f), static_cast<_Float16>(-1152.f)};
+              const half2v y = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, pr, (j & 1) ? 0x04030402u : 0x04010400u));
+              x = __builtin_elementwise_fma(x, s, (y + bias) * s8);  // one of the two is zero
+            } else {
+              x = x * s;
+            }
+            v[h][j] = __builtin_bit_cast(uint32_t, x);
+          }
+          if (hc + kHalf == CPL) {  // the rows are used: reload them from the next block
+            load_codes(row_of(b + 1), h);
+            load_int8(b + 1, h, fl);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < kHalf; ++j) {
+          const half8 bv = __builtin_bit_cast(half8, u32x4{v[0][j], v[1][j], v[2][j], v[3][j]});
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb)
+            acc[mb][hc + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[mb], bv, acc[mb][hc + j], 0, 0, 0);
+        }
+      }
+      flags = fl;
+    }
+  }
+};
+
+// x rows (fp16, global): the lane's row of each pair block at the item's first
+// column + 8 kq.
+template <int MB>
+struct ActX {
+  const _Float16* src[MB];
+  half8 r[MB];
+  __device__ __forceinline__ void load(int b) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) r[mb] = *reinterpret_cast<const half8*>(src[mb] + 32 * b);
+  }
+  __device__ __forceinline__ half8 get(int, int mb) const { return r[mb]; }
+};
+// fp16 rows in LDS, `block` bytes between pair blocks: at = the lane's row of
+// the first, column 8 kq.
+struct ActLds {
+  uint32_t at, block;
+  __device__ __forceinline__ void load(int) const {}
+  __device__ __forceinline__ half8 get(int b, int mb) const { return lds_ld<half8>(at + mb * block + b * 64); }
+};
+
+// f(columns per lane, column tiles) for N columns.
+template <typename F>
+__device__ __forceinline__ void with_columns(int n, F&& f) {
+  using std::integral_constant;
+  if (n <= 64)
+    f(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+  else if (n <= 128)
+    f(integral_constant<int, 8>{}, integral_constant<int, 1>{});
+  else if (n <= 256)
+    f(integral_constant<int, 8>{}, integral_constant<int, 2>{});
+  else
+    f(integral_constant<int, 8>{}, integral_constant<int, 4>{});
 }
 
-// The chunk loop of one decode source.  Step c issues the activation loads
-// of chunk c + 1 (issue(c + 1, slot)), the INT8 bytes of chunk c + 1 (whose
-// units were issued two steps earlier) and the units of chunk c + 3, then
-// stores chunk c's activations (store(c, slot)) and decoded units to LDS
-// and runs its MFMA steps (mfma(c)).  Loads complete in issue order, so the
-// decode of chunk c leaves the units of chunks c + 2 and c + 3 in flight.
-// Two barriers per chunk: the decoded chunk and the activations are
-// complete, then every wave is done with them (LDS barriers: the loads
-// issued ahead stay in flight).  block: the thread's group block in the
-// decoded chunk.
-template <bool kInt8, class SH, typename Issue, typename Store, typename Mfma>
-__device__ __forceinline__ void run_chunks(const Src& s, SH sh, int nc, int block, uint32_t lut,
-                                           uint32_t bt, Ring<kInt8>& rg, Issue&& issue, Store&& store,
-                                           Mfma&& mfma) {
-  const int g = s.g0 + min(s.gi, s.ng - 1);
-  ring_issue<kInt8>(s, sh, 0, nc, rg.u[0]);
-  ring_issue<kInt8>(s, sh, 1, nc, rg.u[1]);
-  ring_issue<kInt8>(s, sh, 2, nc, rg.u[2]);
-  q_load<kInt8>(s, rg.u[0], g, rg.q[0]);
-  issue(0, std::integral_constant<int, 0>{});
-  auto step = [&](int c, auto us) __attribute__((always_inline)) {
-    constexpr int U = decltype(us)::value, Qs = U & 1;
-    issue(c + 1, std::integral_constant<int, Qs ^ 1>{});
-    q_load<kInt8>(s, rg.u[(U + 1) & 3], g, rg.q[Qs ^ 1]);
-    ring_issue<kInt8>(s, sh, c + 3, nc, rg.u[(U + 3) & 3]);
-    store(c, std::integral_constant<int, Qs>{});
-    ring_store<kInt8>(s, sh, c, rg.u[U], rg.q[Qs], lut, bt, block);
-    lds_barrier();
-    mfma(c);
-    lds_barrier();
-  };
-  for (int c = 0; c < nc; c += 4) {
-    step(c, std::integral_constant<int, 0>{});
-    if (c + 1 >= nc) break;
-    step(c + 1, std::integral_constant<int, 1>{});
-    if (c + 2 >= nc) break;
-    step(c + 2, std::integral_constant<int, 2>{});
-    if (c + 3 >= nc) break;
-    step(c + 3, std::integral_constant<int, 3>{});
+// A lane's products of a 16 x 16 CPL tile in LDS (at: its first row, column CPL n).
+template <int CPL>
+__device__ __forceinline__ void store_tile(uint32_t at, const float4v (&acc)[CPL]) {
+#pragma unroll
+  for (int v = 0; v < 4; ++v)
+#pragma unroll
+    for (int c = 0; c < CPL; c += 4)
+      lds_st<float4v>(at + static_cast<uint32_t>(v * kTileStr + c) * 4u,
+                      float4v{acc[c][v], acc[c + 1][v], acc[c + 2][v], acc[c + 3][v]});
+}
+// Products of 32 nblk rows (from row0 of the factor) with `cols` columns for
+// m pairs, times 2^-exp of their rows, added to dst[row][0 .. cols) (rows
+// `stride` floats apart).  The waves share K where the columns are fewer than
+// four tiles.  ready(): the level table and the activations are in LDS (the
+// first factor loads are issued before it).  red: LDS address of kRedBytes the
+// table, the meta slots and the activations may overlap.
+template <int MB, bool kInt8, class Act, typename Ready>
+__device__ __forceinline__ void rank_gemm(const Factor& f, int e, int row0, int nblk, int cols, int m, uint32_t lut,
+                                          uint32_t meta, uint32_t red, const int* rexp, const Act& act, Ready&& ready,
+                                          float* dst, int stride) {
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform(tid >> 6);
+  const int n = lane & 15, kq = lane >> 4;
+  with_columns(cols, [&](auto cpl, auto nt) __attribute__((always_inline)) {
+    constexpr int CPL = decltype(cpl)::value, NT = decltype(nt)::value, KP = 4 / NT;
+    const int tile = wave % NT, kp = wave / NT;
+    Walk<CPL, MB, kInt8, Act> walk(f, e, tile * 16 * CPL, row0, kp * nblk / KP, (kp + 1) * nblk / KP, lane, meta, act);
+    walk.start();
+    ready();
+    float4v acc[MB][CPL];
+    walk.run(lut, acc);
+    const uint32_t at = red + wave * kHalfSlot + static_cast<uint32_t>((kq & 1) * 4 * kTileStr + n * CPL) * 4u;
+#pragma unroll
+    for (int half = 0; half < 2 * MB; ++half) {
+      if (half * 8 >= m) break;
+      lds_barrier();  // every wave is done with the activations, or with the last rows' sums
+      if ((kq >> 1) == (half & 1)) store_tile(at, acc[half >> 1]);
+      lds_barrier();
+      const int rows = min(8, m - half * 8);
+      for (int i = tid; i < rows * cols; i += kT) {
+        const int r = i / cols, c = i - r * cols, t = c / (16 * CPL);
+        const uint32_t src = red + t * kHalfSlot + static_cast<uint32_t>(r * kTileStr + c - t * 16 * CPL) * 4u;
+        float s = lds_ld<float>(src);
+#pragma unroll
+        for (int k = 1; k < KP; ++k) s += lds_ld<float>(src + k * NT * kHalfSlot);
+        atomic_add_f32(dst + static_cast<int64_t>(half * 8 + r) * stride + c, ldexpf(s, -rexp[half * 8 + r]));
+      }
+    }
+  });
+}
+
+// fp32 latent rows [m][.] (rank values of each, `stride` floats apart) as fp16
+// rows times a power of two in LDS (dst, dst_str bytes apart), zero past the
+// rank and past m up to `rows`; the exponents to rexp.  16 lanes per row.
+__device__ __forceinline__ void stage_rows(const float* src, int64_t stride, int rows, int m, int rank, int width,
+                                           uint32_t dst, uint32_t dst_str, int* rexp) {
+  const int t = threadIdx.x & 15;
+  for (int r = threadIdx.x >> 4; r < rows; r += kT / 16) {
+    const float* row = src + static_cast<int64_t>(min(r, m - 1)) * stride;
+    const int n4 = r < m ? (rank + 3) / 4 : 0;
+    float mx = 0.f;
+    for (int c = t; c < n4; c += 16) {
+      const float4v v = *reinterpret_cast<const float4v*>(row + 4 * c);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) mx = 4 * c + q < rank ? fmaxf(mx, fabsf(v[q])) : mx;
+    }
+    mx = op_over(mx, 1, 16, OpMax{});
+    const int ex = pow2_row_exponent(mx);
+    if (t == 0) rexp[r] = ex;
+    for (int c = t; c < width / 4; c += 16) {
+      const float4v v = c < n4 ? *reinterpret_cast<const float4v*>(row + 4 * c) : float4v{0.f, 0.f, 0.f, 0.f};
+      typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+      half4 h;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) h[q] = static_cast<_Float16>(4 * c + q < rank ? ldexpf(v[q], ex) : 0.f);
+      lds_st<half4>(dst + r * dst_str + c * 8, h);
+    }
   }
 }
 
-__device__ __forceinline__ half2v to_h2(float a, float b, int ex) {
-  return half2v{static_cast<_Float16>(ldexpf(a, ex)), static_cast<_Float16>(ldexpf(b, ex))};
-}
+// Waves per SIMD the kernels are compiled for (four pair blocks take 128
+// accumulators).
+constexpr int waves_for(int mb) { return mb == 1 ? 3 : 2; }
 
 // ---------------------------------------------------------------------------
 // Phase A: x . A_g, x . A_u over a range of d rows
 // ---------------------------------------------------------------------------
-struct alignas(16) SmemA {
-  uint32_t bt[kBtDw];
-  uint32_t act[2][kActDw];  // x rows of the chunk (by ring slot parity of the stage)
-  uint32_t lut[256];
-  int rtok[kPass];
-  int rexp[kPass];
-};
-
-template <bool kInt8>
-__global__ void __launch_bounds__(kT, 2) a_kernel(Params p) {
-  __shared__ SmemA sm;
+template <int MB, bool kInt8>
+__global__ void __launch_bounds__(kT, waves_for(MB)) a_kernel(Params p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __shared__ int rexp[16 * MB];
   int a, item;
   if (!map_item(blockIdx.x, p.n_a, p.meta[0], a, item)) return;
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform(tid >> 6);
-  const int n = lane & 15, kq = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int kind = item & 1, split = item >> 1;
-  const Factor& f = p.fac[kind ? F_UP_A : F_GATE_A];
   const int e = p.act_expert[a], s0 = p.act_start[a], mtot = p.act_count[a];
-  const int rank = rank_of(p, e, kind), ng = (rank + kGroup - 1) / kGroup;
-  if (ng == 0 || mtot == 0) return;
-  with_shape(ng, [&](auto sh) __attribute__((always_inline)) {
-    // The item's share of the expert's chunks of d (chunks of sh.rows rows:
-    // about 8 KB of codes each, so an expert's chunk count grows with its rank).
-    const int nct = (p.d + sh.rows - 1) / sh.rows;
-    const int c_lo = split * nct / p.na_split, c_hi = (split + 1) * nct / p.na_split;
-    const int nc = c_hi - c_lo;
-    if (nc <= 0) return;
-    const int r_lo = c_lo * sh.rows, r_end = min(p.d, c_hi * sh.rows);
-    lut_fill(sm.lut, tid);
-    const uint32_t L_lut = lds_addr(sm.lut), L_bt = lds_addr(sm.bt);
-    const uint32_t L_act[2] = {lds_addr(sm.act[0]), lds_addr(sm.act[1])};
-    const Src src = make_src(f, e, r_lo, r_end, 0, ng, tid & (sh.ngp - 1), tid / sh.ngp);
-    const int ncb = 2 * ng;  // 16-column blocks of the rank
-    const int astr = sh.cstr;
-    // x staging: 16 rows x sh.rows halves in 16-byte pieces; piece i of this
-    // thread is tid + 256 i (i < 2; sh.rows <= 256).
-    const int pieces = kPass * sh.rows / 8, ppr = sh.rows / 8;
-    for (int tb = 0; tb < mtot; tb += kPass) {
-      const int m = min(kPass, mtot - tb);
-      if (tid < kPass) {
-        const int tok = tid < m ? p.pair_tok[s0 + tb + tid] : -1;
-        sm.rtok[tid] = tok;
-        sm.rexp[tid] = tok >= 0 ? p.xexp[tok] : 0;
-      }
-      lds_barrier();
-      u32x4 xr[2][2];
-      auto load_x = [&](int c, u32x4 (&x)[2]) __attribute__((always_inline)) {
-  #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int pc = tid + kT * i;
-          const int row = min(pc / ppr, kPass - 1), k8 = pc % ppr;
-          const int tok = sm.rtok[row];
-          const int col = r_lo + min(c, nc - 1) * sh.rows + k8 * 8;
-          const bool ok = pc < pieces && tok >= 0 && col < r_end;
-          const int64_t off = static_cast<int64_t>(max(tok, 0)) * p.d + min(col, p.d - 8);
-          const u32x4 v = *reinterpret_cast<const u32x4*>(p.xh + off);
-          x[i] = ok ? v : u32x4{0u, 0u, 0u, 0u};
-        }
-      };
-      float4v acc[8];
-  #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[j] = float4v{0.f, 0.f, 0.f, 0.f};
-      Ring<kInt8> rg;
-      auto issue = [&](int c, auto slot) __attribute__((always_inline)) { load_x(c, xr[decltype(slot)::value]); };
-      auto store = [&](int c, auto slot) __attribute__((always_inline)) {
-        constexpr int S = decltype(slot)::value;
-  #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int pc = tid + kT * i;
-          if (pc < pieces)
-            lds_st<u32x4>(L_act[S] + static_cast<uint32_t>((pc / ppr) * astr + (pc % ppr) * 4) * 4u, xr[S][i]);
-        }
-      };
-      auto mfma = [&](int c) __attribute__((always_inline)) {
-        // The stage of chunk c wrote act[c % 2] (the ring's slot order).
-        chunk_mfma<8>(L_act[c & 1], astr, L_bt, sh, wave, 4, ncb, n, kq, acc);
-      };
-      run_chunks<kInt8>(src, sh, nc, src.gi, L_lut, L_bt, rg, issue, store, mfma);
-      // Partial latents of the pass: scaled back, summed into gu.
-  #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int cb = wave + 4 * j;
-        const int col = cb * 16 + n;
-        if (cb < ncb && col < rank) {
-  #pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int row = kq * 4 + v;
-            if (row < m) {
-              const float sc = ldexpf(1.0f, -sm.rexp[row]);
-              atomic_add_f32(p.gu + static_cast<int64_t>(s0 + tb + row) * (2 * p.R) + kind * p.R + col, acc[j][v] * sc);
-            }
-          }
-        }
-      }
-      lds_barrier();  // rtok / rexp of the next pass
+  const int cols = (rank_of(p, e, kind) + kGroup - 1) / kGroup * kGroup;
+  // Ranges of d in proportion to the expert's rank, so that items are alike.
+  const int pieces = (p.na_split * max(cols, 128) + p.R - 1) / max(p.R, 128), nblk = p.d / 32;
+  if (split >= pieces) return;
+  const int blk0 = split * nblk / pieces, blk1 = (split + 1) * nblk / pieces;
+  if (blk0 == blk1) return;
+  const uint32_t lut0 = lds_addr(smem), lut = lut0 + (lane & (kCopies - 1)) * 4;
+  const uint32_t meta = lut0 + kLutBytes + uniform(tid >> 6) * kMetaBytes;
+  for (int tb = 0; tb < mtot; tb += 16 * MB) {
+    const int m = min(16 * MB, mtot - tb);
+    ActX<MB> act;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {  // rows past m repeat the last: their results are not stored
+      const int tok = p.pair_tok[s0 + tb + min(16 * mb + (lane & 15), m - 1)];
+      act.src[mb] = p.xh + static_cast<int64_t>(tok) * p.d + 32 * blk0 + 8 * (lane >> 4);
     }
-  });
+    auto ready = [&]() __attribute__((always_inline)) {
+      if (tid < 16 * MB) rexp[tid] = p.xexp[p.pair_tok[s0 + tb + min(tid, m - 1)]];
+      lut_fill(lut0, tid);  // the sums take the table's place
+      lds_barrier();
+    };
+    rank_gemm<MB, kInt8>(p.fac[kind ? F_UP_A : F_GATE_A], e, 32 * blk0, blk1 - blk0, cols, m, lut, meta, lut0, rexp,
+                         act, ready, p.gu + static_cast<int64_t>(s0 + tb) * (2 * p.R) + kind * p.R, 2 * p.R);
+    lds_barrier();  // the sums and exponents are read
+  }
 }
 
 // ---------------------------------------------------------------------------
 // Phase BC: g . B_g and u . B_u over 256 columns of ff, h = SiLU(g) u in
 // LDS, then h . A_d (those 256 rows of A_d)
 // ---------------------------------------------------------------------------
-struct alignas(16) SmemBC {
-  uint32_t bt[kBtDw];
-  uint32_t act[2][2][kPass * 20];  // [slot][gate, up] latent rows of a 32-row chunk
-  uint32_t h[kPass * kHDw];        // h rows (fp16 x 2^hexp)
-  uint32_t lut[256];
-  int rexp[2][kPass];              // gate, up latent exponents
-  int hexp[kPass];
-  float hmax[4][kPass];
-};
-
-template <bool kInt8>
-__global__ void __launch_bounds__(kT, 2) bc_kernel(Params p) {
-  __shared__ SmemBC sm;
+template <int MB, bool kInt8>
+__global__ void __launch_bounds__(kT, waves_for(MB)) bc_kernel(Params p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __shared__ int rexp[2][16 * MB], hexp[16 * MB];
   int a, item;
   if (!map_item(blockIdx.x, p.n_bc, p.meta[0], a, item)) return;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform(tid >> 6);
   const int n = lane & 15, kq = lane >> 4;
   const int e = p.act_expert[a], s0 = p.act_start[a], mtot = p.act_count[a];
-  const int rg_ = rank_of(p, e, 0), ru = rank_of(p, e, 1), rd = rank_of(p, e, 2);
-  const int c0 = item * kCB, ncol = min(kCB, p.ff - c0), ngc = ncol / kGroup;
-  if (mtot == 0) return;
-  lut_fill(sm.lut, tid);
-  const uint32_t L_lut = lds_addr(sm.lut), L_bt = lds_addr(sm.bt), L_h = lds_addr(sm.h);
-  const Factor& fbg = p.fac[F_GATE_B];
-  const Factor& fbu = p.fac[F_UP_B];
-  const Factor& fad = p.fac[F_DOWN_A];
-  // Stage 1: 16 groups per chunk (8 of B_g, 8 of B_u), 32 rows of the rank.
-  constexpr Shape<16> sh1{};
-  const int kb = max(rg_, ru);
-  const int nc1 = (kb + 31) / 32;
-  // Stage 2: the 256 rows of A_d at c0, rd columns.
-  const int ngd = (rd + kGroup - 1) / kGroup;
-  for (int tb = 0; tb < mtot; tb += kPass) {
-    const int m = min(kPass, mtot - tb);
-    // Latent row exponents: max |g|, then max |u|, over the rank (16 lanes per row).
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int r = tid >> 4, t = tid & 15;
-      const int rk = k ? ru : rg_;
-      float mx = 0.f;
-      if (r < m) {
-        const float* row = p.gu + static_cast<int64_t>(s0 + tb + r) * (2 * p.R) + k * p.R;
-        for (int c = t; c < rk; c += 16) mx = fmaxf(mx, fabsf(row[c]));
-      }
-      mx = op_over(mx, 1, 16, OpMax{});
-      if (t == 0) sm.rexp[k][r] = pow2_row_exponent(mx);
-    }
+  const int rg = rank_of(p, e, 0), ru = rank_of(p, e, 1), rd = rank_of(p, e, 2);
+  const int c0 = item * kCB, ncol = min(kCB, p.ff - c0);
+  // LDS: level table and meta slots, then the latents (gate and up halves of a
+  // row); their place the h rows take, and behind those the waves' products,
+  // eight rows at a time (three workgroups per CU at any rank).
+  const uint32_t lstr = (2 * p.R + 8) * 2;
+  const uint32_t lut0 = lds_addr(smem), L_lat = lut0 + kFixBytes, L_h = L_lat, L_red = L_h + 16 * MB * kHStr * 2;
+  const uint32_t lut = lut0 + (lane & (kCopies - 1)) * 4, meta = lut0 + kLutBytes + wave * kMetaBytes;
+  lut_fill(lut0, tid);
+  // Waves: (gate, up) x (columns 0-127, 128-255).
+  const int kind = wave & 1, tile = wave >> 1;
+  const int nb = tile * 128 < ncol ? ((kind ? ru : rg) + 31) / 32 : 0;
+  const int cols = (rd + kGroup - 1) / kGroup * kGroup;
+  for (int tb = 0; tb < mtot; tb += 16 * MB) {
+    const int m = min(16 * MB, mtot - tb);
+    Walk<8, MB, kInt8, ActLds> walk(
+        p.fac[kind ? F_UP_B : F_GATE_B], e, min(c0 + tile * 128, p.ff - 32), 0, 0, nb, lane, meta,
+        ActLds{L_lat + n * lstr + static_cast<uint32_t>(kind * p.R + 8 * kq) * 2u, 16u * lstr});
+    walk.start();
+    const float* gu = p.gu + static_cast<int64_t>(s0 + tb) * (2 * p.R);
+    stage_rows(gu, 2 * p.R, 16 * MB, m, rg, p.R, L_lat, lstr, rexp[0]);
+    stage_rows(gu + p.R, 2 * p.R, 16 * MB, m, ru, p.R, L_lat + 2u * p.R, lstr, rexp[1]);
     lds_barrier();
-    float4v accg[4], accu[4];
+    float4v acc[MB][8];
+    walk.run(lut, acc);
+    const uint32_t at = L_red + (2 * kind + tile) * kHalfSlot + static_cast<uint32_t>((kq & 1) * 4 * kTileStr + n * 8) * 4u;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) accg[j] = accu[j] = float4v{0.f, 0.f, 0.f, 0.f};
-    if (nc1 > 0) {
-      // Two sources in one chunk: waves 0-1 decode the item's groups of B_g
-      // into group blocks 0-7, waves 2-3 those of B_u into blocks 8-15
-      // (thread: group tid % 8, row pair (tid % 128) / 8).  Rows past a
-      // factor's own rank decode as zeros.
-      const bool up = uniform(tid >> 7) != 0;
-      const Src mine = make_src(up ? fbu : fbg, e, 0, up ? ru : rg_, c0 / kGroup, ngc, tid & 7, (tid & 127) >> 3);
-      const int block = (up ? 8 : 0) + (tid & 7);
-      // act staging: gate and up latent rows of chunk c (32 rank rows), fp16 x 2^rexp.
-      u32x4 lr[2];
-      auto load_l = [&](int c, u32x4& x) __attribute__((always_inline)) {
-        // Thread: row r = tid >> 4, factor k = (tid >> 3) & 1, 4 values at 4 (tid & 7).
-        const int r = tid >> 4, k = (tid >> 3) & 1, q4 = (tid & 7) * 4;
-        const int col = min(c, nc1 - 1) * 32 + q4;
-        const int rk = k ? ru : rg_;
-        const bool ok = r < m && col < rk;
-        const float* src = p.gu + static_cast<int64_t>(s0 + tb + min(r, m - 1)) * (2 * p.R) + k * p.R + min(col, p.R - 4);
-        const float4 v = *reinterpret_cast<const float4*>(src);
-        x = ok ? u32x4{__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)}
-               : u32x4{0u, 0u, 0u, 0u};
-      };
-      auto issue = [&](int c, auto slot) __attribute__((always_inline)) { load_l(c, lr[decltype(slot)::value]); };
-      auto store = [&](int c, auto slot) __attribute__((always_inline)) {
-        constexpr int S = decltype(slot)::value;
-        const int r = tid >> 4, k = (tid >> 3) & 1, q4 = (tid & 7) * 4;
-        const int ex = sm.rexp[k][r];
-        const half2v h0 = to_h2(__uint_as_float(lr[S][0]), __uint_as_float(lr[S][1]), ex);
-        const half2v h1 = to_h2(__uint_as_float(lr[S][2]), __uint_as_float(lr[S][3]), ex);
-        typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-        const u32x2 w = {__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1)};
-        lds_st<u32x2>(lds_addr(sm.act[S][k]) + static_cast<uint32_t>(r * 20 + q4 / 2) * 4u, w);
-      };
-      Ring<kInt8> rg;
-      auto mfma = [&](int c) __attribute__((always_inline)) {
-        const int S = c & 1;
-        // Wave w: columns [64w, 64w + 64) of the item for both factors
-        // (groups 2w, 2w + 1 of B_g and 8 + 2w, 9 + 2w of B_u).
-        chunk_mfma<4>(lds_addr(sm.act[S][0]), 20, L_bt, sh1, 4 * wave, 1, 2 * ngc, n, kq, accg);
-        chunk_mfma<4>(lds_addr(sm.act[S][1]), 20, L_bt, sh1, 16 + 4 * wave, 1, 16 + 2 * ngc, n, kq, accu);
-      };
-      run_chunks<kInt8>(mine, sh1, nc1, block, L_lut, L_bt, rg, issue, store, mfma);
-    }
-    // h = SiLU(g) u (x router weight before down) of the wave's 64 columns,
-    // fp16 with one exponent per row (the maximum over the item's columns).
-    float hv[4][4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = kq * 4 + v;
-      const float sg = ldexpf(1.0f, -sm.rexp[0][row]), su = ldexpf(1.0f, -sm.rexp[1][row]);
-      const float wr = p.wbd && row < m ? p.pair_w[s0 + tb + row] : 1.0f;
+    for (int half = 0; half < 2 * MB; ++half) {
+      lds_barrier();  // the latents (or the last rows' products) are read
+      if ((kq >> 1) == (half & 1)) store_tile(at, acc[half >> 1]);
+      lds_barrier();
+      // h = SiLU(g) u (x router weight before down), fp16 with one exponent
+      // per row (the maximum over the item's columns); 32 lanes per row.
+      const int r = half * 8 + (tid >> 5), t = tid & 31;
+      const float sg = ldexpf(1.0f, -rexp[0][r]), su = ldexpf(1.0f, -rexp[1][r]);
+      const float wr = p.wbd && r < m ? p.pair_w[s0 + tb + r] : 1.0f;
+      float4v h[2];
       float mx = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int col = 64 * wave + 16 * j + n;
-        const float g = accg[j][v] * sg, u = accu[j][v] * su;
-        hv[j][v] = col < ncol && row < m ? g / (1.0f + expf(-g)) * u * wr : 0.f;
-        mx = fmaxf(mx, fabsf(hv[j][v]));
-      }
-      mx = op_over(mx, 1, 16, OpMax{});
-      if (n == 0) sm.hmax[wave][row] = mx;
-    }
-    lds_barrier();
+      for (int j = 0; j < 2; ++j) {
+        const int col = 128 * j + 4 * t;
+        const uint32_t src = L_red + j * kHalfSlot + static_cast<uint32_t>((tid >> 5) * kTileStr + 4 * t) * 4u;
+        const float4v g = lds_ld<float4v>(src) * sg, u = lds_ld<float4v>(src + 2 * kHalfSlot) * su;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = kq * 4 + v;
-      const float mx = fmaxf(fmaxf(sm.hmax[0][row], sm.hmax[1][row]), fmaxf(sm.hmax[2][row], sm.hmax[3][row]));
-      const int ex = pow2_row_exponent(mx);
-      if (wave == 0 && n == 0) sm.hexp[row] = ex;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int col = 64 * wave + 16 * j + n;
-        const _Float16 hh = static_cast<_Float16>(ldexpf(hv[j][v], ex));
-        lds_st<_Float16>(L_h + static_cast<uint32_t>(row * kHDw * 4 + col * 2), hh);
-      }
-    }
-    lds_barrier();
-    // Stage 2: d latent partial of these 256 rows of A_d.
-    // (One run-time shape: a compile-time one per group count spilled.)
-    if (ngd > 0) {
-      const DynShape sh2 = dyn_shape(ngd);
-      const int nc2 = (ncol + sh2.rows - 1) / sh2.rows;
-      float4v accd[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) accd[j] = float4v{0.f, 0.f, 0.f, 0.f};
-      const Src sd = make_src(fad, e, c0, c0 + ncol, 0, ngd, tid & (sh2.ngp - 1), tid / sh2.ngp);
-      auto none = [&](int, auto) __attribute__((always_inline)) {};
-      Ring<kInt8> rg;
-      auto mfma = [&](int c) __attribute__((always_inline)) {
-        chunk_mfma<8>(L_h + static_cast<uint32_t>(c * sh2.rows) * 2u, kHDw, L_bt, sh2, wave, 4, 2 * ngd, n, kq, accd);
-      };
-      run_chunks<kInt8>(sd, sh2, nc2, sd.gi, L_lut, L_bt, rg, none, none, mfma);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int cb = wave + 4 * j;
-        const int col = cb * 16 + n;
-        if (cb < 2 * ngd && col < rd) {
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const int row = kq * 4 + v;
-            if (row < m)
-              atomic_add_f32(p.dl + static_cast<int64_t>(s0 + tb + row) * p.R + col,
-                             accd[j][v] * ldexpf(1.0f, -sm.hexp[row]));
-          }
+        for (int q = 0; q < 4; ++q) {
+          h[j][q] = col < ncol && r < m ? g[q] / (1.0f + expf(-g[q])) * u[q] * wr : 0.f;
+          mx = fmaxf(mx, fabsf(h[j][q]));
         }
       }
+      mx = op_over(mx, 1, 32, OpMax{});
+      const int ex = pow2_row_exponent(mx);
+      if (t == 0) hexp[r] = ex;
+      typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        half4 v;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] = static_cast<_Float16>(ldexpf(h[j][q], ex));
+        lds_st<half4>(L_h + static_cast<uint32_t>(r * kHStr + 128 * j + 4 * t) * 2u, v);
+      }
     }
+    if (cols != 0)
+      rank_gemm<MB, kInt8>(p.fac[F_DOWN_A], e, c0, ncol / 32, cols, m, lut, meta, L_red, hexp,
+                           ActLds{L_h + static_cast<uint32_t>(n * kHStr + 8 * kq) * 2u, 16u * kHStr * 2},
+                           [] { lds_barrier(); }, p.dl + static_cast<int64_t>(s0 + tb) * p.R, p.R);
     lds_barrier();
   }
 }
@@ -632,99 +525,83 @@ __global__ void __launch_bounds__(kT, 2) bc_kernel(Params p) {
 // ---------------------------------------------------------------------------
 // Phase D: d_lat . B_d over 512 columns of d, weighted into out
 // ---------------------------------------------------------------------------
-struct alignas(16) SmemD {
-  uint32_t bt[kBtDw];
-  uint32_t act[2][kPass * 20];  // d latent rows of a 32-row chunk
-  uint32_t lut[256];
-  int rexp[kPass];
-  int rtok[kPass];
-  float rw[kPass];
-};
-
-template <bool kInt8>
-__global__ void __launch_bounds__(kT, 2) d_kernel(Params p) {
-  __shared__ SmemD sm;
+template <int MB, bool kInt8>
+__global__ void __launch_bounds__(kT, waves_for(MB)) d_kernel(Params p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  __shared__ int rexp[16 * MB];
   int a, item;
   if (!map_item(blockIdx.x, p.n_d, p.meta[0], a, item)) return;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform(tid >> 6);
   const int n = lane & 15, kq = lane >> 4;
   const int e = p.act_expert[a], s0 = p.act_start[a], mtot = p.act_count[a];
   const int rd = rank_of(p, e, 2);
-  const int c0 = item * kCD, ncol = min(kCD, p.d - c0), ngc = ncol / kGroup;
-  const Factor& f = p.fac[F_DOWN_B];
-  if (mtot == 0) return;
-  lut_fill(sm.lut, tid);
-  const uint32_t L_lut = lds_addr(sm.lut), L_bt = lds_addr(sm.bt);
-  constexpr Shape<16> sh{};  // 32 rows of the rank per chunk
-  const int nc = (rd + 31) / 32;
-  const Src src = make_src(f, e, 0, rd, c0 / kGroup, ngc, tid & (sh.ngp - 1), tid / sh.ngp);
-  for (int tb = 0; tb < mtot; tb += kPass) {
-    const int m = min(kPass, mtot - tb);
-    {
-      const int r = tid >> 4, t = tid & 15;
-      float mx = 0.f;
-      if (r < m) {
-        const float* row = p.dl + static_cast<int64_t>(s0 + tb + r) * p.R;
-        for (int c = t; c < rd; c += 16) mx = fmaxf(mx, fabsf(row[c]));
-      }
-      mx = op_over(mx, 1, 16, OpMax{});
-      if (t == 0) {
-        sm.rexp[r] = pow2_row_exponent(mx);
-        const int pair = s0 + tb + min(r, m - 1);
-        sm.rtok[r] = r < m ? p.pair_tok[pair] * p.K + p.pair_slot[pair] : -1;
-        sm.rw[r] = p.wbd ? 1.0f : p.pair_w[pair];
-      }
-    }
+  const int c0 = item * kCD, ct = c0 + wave * 128;  // a tile of 128 columns per wave
+  const int nb = ct < p.d ? (rd + 31) / 32 : 0;
+  const uint32_t lstr = (p.R + 8) * 2;
+  const uint32_t lut0 = lds_addr(smem), L_lat = lut0 + kFixBytes, lut = lut0 + (lane & (kCopies - 1)) * 4;
+  const uint32_t meta = lut0 + kLutBytes + wave * kMetaBytes;
+  lut_fill(lut0, tid);
+  for (int tb = 0; tb < mtot; tb += 16 * MB) {
+    const int m = min(16 * MB, mtot - tb);
+    Walk<8, MB, kInt8, ActLds> walk(p.fac[F_DOWN_B], e, min(ct, p.d - 32), 0, 0, nb, lane, meta,
+                                    ActLds{L_lat + n * lstr + 16u * kq, 16u * lstr});
+    walk.start();
+    stage_rows(p.dl + static_cast<int64_t>(s0 + tb) * p.R, p.R, 16 * MB, m, rd, p.R, L_lat, lstr, rexp);
     lds_barrier();
-    float4v acc[8];
+    float4v acc[MB][8];
+    walk.run(lut, acc);
+    // Eight rows of every wave's products at a time.
+    const uint32_t at = L_lat + wave * kHalfSlot + static_cast<uint32_t>((kq & 1) * 4 * kTileStr + n * 8) * 4u;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[j] = float4v{0.f, 0.f, 0.f, 0.f};
-    if (nc > 0) {
-      u32x4 lr[2];
-      // Thread: row r = tid >> 4 (16 rows), 2 values at 2 (tid & 15) of the chunk's 32.
-      auto load_l = [&](int c, u32x4& x) __attribute__((always_inline)) {
-        const int r = tid >> 4, q2 = (tid & 15) * 2;
-        const int col = min(c, nc - 1) * 32 + q2;
-        const bool ok = r < m && col < rd;
-        const float* s = p.dl + static_cast<int64_t>(s0 + tb + min(r, m - 1)) * p.R + min(col, p.R - 2);
-        const float2 v = *reinterpret_cast<const float2*>(s);
-        x = ok ? u32x4{__float_as_uint(v.x), __float_as_uint(v.y), 0u, 0u} : u32x4{0u, 0u, 0u, 0u};
-      };
-      auto issue = [&](int c, auto slot) __attribute__((always_inline)) { load_l(c, lr[decltype(slot)::value]); };
-      auto store = [&](int c, auto slot) __attribute__((always_inline)) {
-        constexpr int S = decltype(slot)::value;
-        const int r = tid >> 4, q2 = (tid & 15) * 2;
-        const half2v h = to_h2(__uint_as_float(lr[S][0]), __uint_as_float(lr[S][1]), sm.rexp[r]);
-        lds_st<uint32_t>(lds_addr(sm.act[S]) + static_cast<uint32_t>(r * 20 + q2 / 2) * 4u,
-                         __builtin_bit_cast(uint32_t, h));
-      };
-      Ring<kInt8> rg;
-      auto mfma = [&](int c) __attribute__((always_inline)) {
-        chunk_mfma<8>(lds_addr(sm.act[c & 1]), 20, L_bt, sh, wave, 4, 2 * ngc, n, kq, acc);
-      };
-      run_chunks<kInt8>(src, sh, nc, src.gi, L_lut, L_bt, rg, issue, store, mfma);
-    }
+    for (int half = 0; half < 2 * MB; ++half) {
+      if (half * 8 >= m) break;
+      lds_barrier();  // the latents (or the last rows' products) are read
+      if ((kq >> 1) == (half & 1)) store_tile(at, acc[half >> 1]);
+      lds_barrier();
+      // One row at a time over the workgroup: a wave's stores and atomics
+      // cover consecutive columns.
+      const int rows = min(8, m - half * 8);
+      for (int r = 0; r < rows; ++r) {
+        const int pair = s0 + tb + half * 8 + r, tok = p.pair_tok[pair];
+        const float sc = ldexpf(1.0f, -rexp[half * 8 + r]);
+        const float w = p.out_mode == LATENT_OUT_REDUCED && !p.wbd ? p.pair_w[pair] * sc : sc;
+        float* dst = p.out + (p.out_mode == LATENT_OUT_REDUCED ? static_cast<int64_t>(tok)
+                                                               : static_cast<int64_t>(tok) * p.K + p.pair_slot[pair]) * p.d;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int cb = wave + 4 * j;
-      const int col = cb * 16 + n;
-      if (cb < 2 * ngc) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int row = kq * 4 + v;
-          if (row < m) {
-            const float y = acc[j][v] * ldexpf(1.0f, -sm.rexp[row]);
-            const int ts = sm.rtok[row];  // token * K + slot
-            if (p.out_mode == LATENT_OUT_REDUCED)
-              atomic_add_f32(p.out + static_cast<int64_t>(ts / p.K) * p.d + c0 + col, sm.rw[row] * y);
-            else
-              p.out[static_cast<int64_t>(ts) * p.d + c0 + col] = y;
-          }
+        for (int t = 0; t < 2; ++t) {
+          const int col = c0 + t * 256 + tid;
+          if (col >= p.d) continue;
+          const float y = w * lds_ld<float>(L_lat + (2 * t + (tid >> 7)) * kHalfSlot +
+                                            static_cast<uint32_t>(r * kTileStr + (tid & 127)) * 4u);
+          if (p.out_mode == LATENT_OUT_REDUCED)
+            atomic_add_f32(dst + col, y);
+          else
+            dst[col] = y;
         }
       }
     }
-    lds_barrier();
+    lds_barrier();  // the products are read
   }
+}
+
+// Dynamic LDS bytes of the phases.
+constexpr size_t lds_a() { return std::max(kFixBytes, kRedBytes); }
+template <int MB>
+size_t lds_bc(int R) {
+  return static_cast<size_t>(kFixBytes + std::max(16 * MB * (2 * R + 8) * 2, 16 * MB * kHStr * 2 + kRedBytes));
+}
+template <int MB>
+size_t lds_d(int R) {
+  return static_cast<size_t>(kFixBytes + std::max(16 * MB * (R + 8) * 2, kRedBytes));
+}
+
+template <int MB, bool kInt8>
+int launch_phases(const Params& p, hipStream_t s) {
+  const unsigned groups = static_cast<unsigned>((p.a_max + 7) / 8);
+  hipLaunchKernelGGL((a_kernel<MB, kInt8>), dim3(8 * groups * p.n_a), dim3(kT), lds_a(), s, p);
+  hipLaunchKernelGGL((bc_kernel<MB, kInt8>), dim3(8 * groups * p.n_bc), dim3(kT), lds_bc<MB>(p.R), s, p);
+  hipLaunchKernelGGL((d_kernel<MB, kInt8>), dim3(8 * groups * p.n_d), dim3(kT), lds_d<MB>(p.R), s, p);
+  return hipGetLastError() == hipSuccess ? LATENT_OK : LATENT_E_HIP;
 }
 
 }  // namespace
@@ -743,12 +620,10 @@ bool supported(const latent_moe_args& a) {
 }
 
 void plan(Params& p) {
-  // Phase A items per expert and factor: about 4096 items in all, 4 to 16
-  // per factor (measured at the DeepSeek-V3 shape with ranks 64..512: 8 at
-  // 16, 64 and 256 tokens within 3 % of the best; 2 took 17 % longer, 32 up
-  // to 14 %).
+  // Phase A ranges per expert and factor at the full rank (a smaller rank has
+  // fewer): about 4096 items in all, of eight blocks of 32 rows or more.
   int s = 4;
-  while (s < 16 && 2ll * p.a_max * s < 4096) s *= 2;
+  while (s < 32 && 2ll * p.a_max * s < 4096 && p.d / 32 >= 16 * s) s *= 2;
   p.na_split = s;
   p.n_a = 2 * s;
   p.n_bc = (p.ff + kCB - 1) / kCB;
@@ -756,17 +631,16 @@ void plan(Params& p) {
 }
 
 int launch(const Params& p, bool int8, hipStream_t s) {
-  const unsigned groups = static_cast<unsigned>((p.a_max + 7) / 8);
-  if (int8) {
-    hipLaunchKernelGGL(a_kernel<true>, dim3(8 * groups * p.n_a), dim3(kT), 0, s, p);
-    hipLaunchKernelGGL(bc_kernel<true>, dim3(8 * groups * p.n_bc), dim3(kT), 0, s, p);
-    hipLaunchKernelGGL(d_kernel<true>, dim3(8 * groups * p.n_d), dim3(kT), 0, s, p);
-  } else {
-    hipLaunchKernelGGL(a_kernel<false>, dim3(8 * groups * p.n_a), dim3(kT), 0, s, p);
-    hipLaunchKernelGGL(bc_kernel<false>, dim3(8 * groups * p.n_bc), dim3(kT), 0, s, p);
-    hipLaunchKernelGGL(d_kernel<false>, dim3(8 * groups * p.n_d), dim3(kT), 0, s, p);
-  }
-  return hipGetLastError() == hipSuccess ? LATENT_OK : LATENT_E_HIP;
+  // Pair blocks a decoded block of the factor is multiplied with: an expert of
+  // many pairs then decodes its factors once per 64 (or 32) of them.  E 128, d
+  // 4096, ff 1408, rank 64, top-8: 200 tokens (12 pairs an expert) 99 us at
+  // one block and 110 at two, 2000 tokens 674 at one and 568 at four; E 64, d
+  // 2048, rank 192, 200 tokens (19 pairs): 124 at one, 116 at two.
+  if (int8) return launch_phases<1, true>(p, s);
+  const int64_t per = static_cast<int64_t>(p.T) * p.K / p.a_max;
+  if (per >= 24) return launch_phases<4, false>(p, s);
+  if (per >= 16) return launch_phases<2, false>(p, s);
+  return launch_phases<1, false>(p, s);
 }
 
 }  // namespace rows

@@ -108,3 +108,19 @@ def test_rows_dtypes_weighting_and_drops(gpu, layers, x_dtype, wbd):
             assert not got[1, 2].any() and not got[2, 3].any() and not got[5].any()
         else:
             assert not got[5].any()
+
+
+@pytest.mark.parametrize("T,k,mode,wbd", [(70, 4, 0, False), (100, 4, 1, True), (9, 3, 0, True)])
+def test_rows_pair_blocks(gpu, T, k, mode, wbd):
+    """Passes of one, two and four blocks of 16 pairs (the pairs per expert
+    decide), with experts far below and above the average, ranks 192 (a tile of
+    128 columns and half of one), ff and d that end inside an item."""
+    host = synth.make_layer(seed=91, n_expert=9, d=1056, ff=1184, max_rank=192,
+                            ranks=[192, 64, 32, 160, 192, 128, 191, 96, 0])
+    dev = _rows_layer(host)
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T, host.d)).astype(np.float32)
+    ids, w = routing.softmax_topk(rng.standard_normal((T, host.n_expert)) + np.linspace(2, 0, host.n_expert), k)
+    ids[rng.random(ids.shape) < 0.05] = -1
+    got, want = _run(gpu, host, dev, x, ids, w, wbd=wbd, mode=mode)
+    assert ref.rel_l2(want, got) <= TOL
