@@ -219,7 +219,8 @@ int latent_moe_check(void* workspace, size_t workspace_bytes, latent_stream_t st
  *       path 3 takes), no INT8 groups, 16-byte aligned x; on the tile layout
  *       it streams 64-pair units of one expert, on the row layout (n_embd /
  *       n_ff / max_rank multiples of 128, n_ff and max_rank <= 2048, 16-byte
- *       aligned codes) it runs grouped GEMMs;
+ *       aligned codes) it runs grouped GEMMs, or the kernels of path 4 where
+ *       the GEMMs' 128-pair tiles would not fill the chip;
  *   3 = streaming fp16-MFMA decode: the factors are in the tile layout, 1 to
  *       4096 routed pairs, 16-byte aligned x;
  *   4 = multi-kernel fp16-MFMA path on the row layout, taken here when a

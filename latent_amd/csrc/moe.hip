@@ -51,8 +51,19 @@ constexpr int kMaxRank = 512;
 constexpr int kRouteThreads = 1024;
 enum { F_GATE_A = 0, F_GATE_B, F_UP_A, F_UP_B, F_DOWN_A, F_DOWN_B };
 
+// INT8 word offsets to fill: out[row][word] for rows of `words` bitmap words.
+struct WordOffsets {
+  const uint32_t* bitmap;
+  const int32_t* row_offset;
+  int32_t* out;
+  int64_t rows;
+  int words;
+};
+
 struct MoeParams {
   Factor fac[6];
+  WordOffsets off[6];
+  int n_off;
   const void* x;
   const int32_t* ids;
   const void* weights;
@@ -124,8 +135,8 @@ __device__ __forceinline__ void place_pair(const MoeParams& p, const int* start,
   if (p.unit_info) {
     const int rel = pos - start[e];
     p.unit_tok[(ubase[e] << p.unit_shift) + rel] = tok;
-    p.pos_of[i] = pos;
   }
+  if (p.pos_of) p.pos_of[i] = pos;
 }
 
 // Same, at the expert's next free position (the order among one expert's
@@ -320,6 +331,79 @@ __device__ void route_block(const MoeParams& p) {
   }
 }
 
+// What the workgroups beside the grouping do: word offsets of INT8 factors, x
+// as fp16 rows, cleared accumulators.
+__device__ void prep_rest(const MoeParams& p, int64_t blk, int64_t nblk) {
+  const int64_t t0 = blk * static_cast<int64_t>(kRouteThreads) + threadIdx.x;
+  const int64_t stride = nblk * kRouteThreads;
+  for (int f = 0; f < p.n_off; ++f) {  // index of each bitmap word's first INT8 group
+    const WordOffsets& w = p.off[f];
+    for (int64_t r = t0; r < w.rows; r += stride) {
+      int run = w.row_offset[r];
+      for (int i = 0; i < w.words; ++i) {
+        w.out[r * w.words + i] = run;
+        run += popc(w.bitmap[r * w.words + i]);
+      }
+    }
+  }
+  if (p.xh) {
+    // One workgroup per token, 8 elements per thread and step: the row maximum
+    // picks the exponent that brings it into [2^14, 2^15), then the row is
+    // stored as fp16 * 2^exponent (the streaming path requires d % 8 == 0 and
+    // a 16-byte aligned x).
+    __shared__ float wmax[kRouteThreads / kWave];
+    for (int64_t t = blk; t < p.T; t += nblk) {
+      const int64_t row = t * p.d;
+      float mx = 0.f;
+      for (int i = threadIdx.x * 8; i < p.d; i += kRouteThreads * 8) {
+        float v[8];
+        load_act8(p.x, p.x_dtype, row + i, v);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mx = fmaxf(mx, fabsf(v[j]));
+      }
+      mx = op_over(mx, 1, kWave, OpMax{});
+      if (threadIdx.x % kWave == 0) wmax[threadIdx.x / kWave] = mx;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < kRouteThreads / kWave; ++w) mx = fmaxf(mx, wmax[w]);
+      __syncthreads();  // wmax is reused by the next token
+      const int ex = pow2_row_exponent(mx);
+      for (int i = threadIdx.x * 8; i < p.d; i += kRouteThreads * 8) {
+        float v[8];
+        load_act8(p.x, p.x_dtype, row + i, v);
+        typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+        half8_t h;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) h[j] = static_cast<_Float16>(ldexpf(v[j], ex));
+        *reinterpret_cast<half8_t*>(p.xh + row + i) = h;
+      }
+      if (threadIdx.x == 0) p.xexp[t] = ex;
+    }
+    // The streaming path clears nothing (its kernels write every output); the
+    // row-layout MFMA phases accumulate like the fp32 ones.
+    if (!p.clear) return;
+  }
+  // Accumulators gu and dl are contiguous: zero_floats covers both.
+  float4* acc4 = reinterpret_cast<float4*>(p.gu);
+  const int64_t n4 = p.zero_floats / 4;
+  for (int64_t i = t0; i < n4; i += stride) acc4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (p.out_mode == LATENT_OUT_REDUCED) {
+    if (!p.zero_out) return;
+    float4* o4 = reinterpret_cast<float4*>(p.out);
+    const int64_t no = static_cast<int64_t>(p.T) * p.d / 4;
+    for (int64_t i = t0; i < no; i += stride) o4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  } else {
+    // Per-slot output: only dropped slots are never written by phase D.
+    const int64_t rows = static_cast<int64_t>(p.T) * p.K;
+    const int64_t d4 = p.d / 4;
+    for (int64_t i = t0; i < rows * d4; i += stride) {
+      const int64_t r = i / d4;
+      const int e = p.ids[r];
+      if (e < 0 || e >= p.E) reinterpret_cast<float4*>(p.out)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  }
+}
+
 // Multi-workgroup grouping for large batches (the single-workgroup route_block
 // serializes on its LDS counters): per-chunk histograms, one scan over
 // (expert, chunk), then a scatter.  hist is [E + 1][nchunk] (the last row
@@ -329,7 +413,11 @@ __device__ void route_block(const MoeParams& p) {
 // its expert, so results do not depend on it.
 constexpr int kHistInts = 16384;  // (E + 1) * nchunk bound: the scan holds the histograms in LDS
 
-__global__ void __launch_bounds__(kRouteThreads) group_count_kernel(MoeParams p, int* hist, int chunk) {
+__global__ void __launch_bounds__(kRouteThreads) group_count_kernel(MoeParams p, int* hist, int chunk, int nchunk) {
+  if (static_cast<int>(blockIdx.x) >= nchunk) {
+    prep_rest(p, blockIdx.x - nchunk, gridDim.x - nchunk);
+    return;
+  }
   __shared__ int cnt[kMaxExperts + 1];
   const int tid = threadIdx.x, E = p.E, P = p.T * p.K;
   for (int e = tid; e <= E; e += kRouteThreads) cnt[e] = 0;
@@ -343,7 +431,7 @@ __global__ void __launch_bounds__(kRouteThreads) group_count_kernel(MoeParams p,
       atomicAdd(&cnt[E], 1);
   }
   __syncthreads();
-  for (int e = tid; e <= E; e += kRouteThreads) hist[e * gridDim.x + blockIdx.x] = cnt[e];
+  for (int e = tid; e <= E; e += kRouteThreads) hist[e * nchunk + blockIdx.x] = cnt[e];
 }
 
 __global__ void __launch_bounds__(kRouteThreads) group_scan_kernel(MoeParams p, int* hist, int nchunk) {
@@ -416,74 +504,16 @@ __global__ void __launch_bounds__(kRouteThreads) group_scatter_kernel(MoeParams 
       p.pair_tok[pos] = i / p.K;
       p.pair_slot[pos] = i - (i / p.K) * p.K;
       p.pair_w[pos] = load_act(p.weights, p.w_dtype, i);
+      if (p.pos_of) p.pos_of[i] = pos;
     }
   }
 }
 
 __global__ void __launch_bounds__(kRouteThreads) prep_kernel(MoeParams p) {
-  if (blockIdx.x == 0) {
+  if (blockIdx.x == 0)
     route_block(p);
-    return;
-  }
-  const int64_t nblk = gridDim.x - 1;
-  const int64_t t0 = (blockIdx.x - 1) * static_cast<int64_t>(kRouteThreads) + threadIdx.x;
-  const int64_t stride = nblk * kRouteThreads;
-  if (p.xh) {
-    // One workgroup per token, 8 elements per thread and step: the row maximum
-    // picks the exponent that brings it into [2^14, 2^15), then the row is
-    // stored as fp16 * 2^exponent (the streaming path requires d % 8 == 0 and
-    // a 16-byte aligned x).
-    __shared__ float wmax[kRouteThreads / kWave];
-    for (int64_t t = blockIdx.x - 1; t < p.T; t += nblk) {
-      const int64_t row = t * p.d;
-      float mx = 0.f;
-      for (int i = threadIdx.x * 8; i < p.d; i += kRouteThreads * 8) {
-        float v[8];
-        load_act8(p.x, p.x_dtype, row + i, v);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) mx = fmaxf(mx, fabsf(v[j]));
-      }
-      mx = op_over(mx, 1, kWave, OpMax{});
-      if (threadIdx.x % kWave == 0) wmax[threadIdx.x / kWave] = mx;
-      __syncthreads();
-#pragma unroll
-      for (int w = 0; w < kRouteThreads / kWave; ++w) mx = fmaxf(mx, wmax[w]);
-      __syncthreads();  // wmax is reused by the next token
-      const int ex = pow2_row_exponent(mx);
-      for (int i = threadIdx.x * 8; i < p.d; i += kRouteThreads * 8) {
-        float v[8];
-        load_act8(p.x, p.x_dtype, row + i, v);
-        typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-        half8_t h;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) h[j] = static_cast<_Float16>(ldexpf(v[j], ex));
-        *reinterpret_cast<half8_t*>(p.xh + row + i) = h;
-      }
-      if (threadIdx.x == 0) p.xexp[t] = ex;
-    }
-    // The streaming path clears nothing (its kernels write every output); the
-    // row-layout MFMA phases accumulate like the fp32 ones.
-    if (!p.clear) return;
-  }
-  // Accumulators gu and dl are contiguous: zero_floats covers both.
-  float4* acc4 = reinterpret_cast<float4*>(p.gu);
-  const int64_t n4 = p.zero_floats / 4;
-  for (int64_t i = t0; i < n4; i += stride) acc4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (p.out_mode == LATENT_OUT_REDUCED) {
-    if (!p.zero_out) return;
-    float4* o4 = reinterpret_cast<float4*>(p.out);
-    const int64_t no = static_cast<int64_t>(p.T) * p.d / 4;
-    for (int64_t i = t0; i < no; i += stride) o4[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-  } else {
-    // Per-slot output: only dropped slots are never written by phase D.
-    const int64_t rows = static_cast<int64_t>(p.T) * p.K;
-    const int64_t d4 = p.d / 4;
-    for (int64_t i = t0; i < rows * d4; i += stride) {
-      const int64_t r = i / d4;
-      const int e = p.ids[r];
-      if (e < 0 || e >= p.E) reinterpret_cast<float4*>(p.out)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-  }
+  else
+    prep_rest(p, blockIdx.x - 1, gridDim.x - 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -856,8 +886,11 @@ __global__ void __launch_bounds__(kThreads) phase_d_kernel(MoeParams p) {
 constexpr size_t kAlign = 256;
 inline size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
+// Scratch of the library's own array (latent_moe_ffn_forward_noalloc).
+constexpr size_t kOwn = LATENT_NOALLOC_SCRATCH_BYTES - LATENT_NOALLOC_CONTROL_BYTES;
+
 struct Layout {
-  size_t meta, act_expert, act_start, act_count, pair_tok, pair_slot, pair_w, hist, units, gu, dl, xh, xexp, total;
+  size_t meta, act_expert, act_start, act_count, pair_tok, pair_slot, pair_w, hist, units, gu, dl, xh, xexp, pos_of, y, total;
 };
 
 // Pairs per chunk of the multi-workgroup grouping: multiples of the block
@@ -876,7 +909,7 @@ int64_t xh_cols(const latent_moe_args& a) {
   return a.layout == LATENT_LAYOUT_ROWS && a.max_rank <= 512 ? a.n_embd : 0;
 }
 
-Layout layout_for(int64_t T, int64_t K, int64_t E, int64_t R, int64_t d) {
+Layout layout_for(int64_t T, int64_t K, int64_t E, int64_t R, int64_t d, bool roomy) {
   Layout L{};
   const int64_t P = T * K;
   const int64_t amax = std::max<int64_t>(1, std::min(E, P));
@@ -895,8 +928,23 @@ Layout layout_for(int64_t T, int64_t K, int64_t E, int64_t R, int64_t d) {
   // x as fp16 rows x 2^xexp for the row-layout MFMA phases (d = 0: none).
   L.xh = off;         off = align_up(off + T * d * 2);
   L.xexp = off;       off = align_up(off + T * sizeof(int));
+  // Their y rows, summed per token at the end, from 2048 pairs (25 M fp32
+  // atomics into out took 75 us of a call's 113 in phase D); not where they
+  // alone (another path of the call needing no more: not roomy) would take it
+  // past the library's own scratch array.
+  L.pos_of = L.y = 0;
+  const size_t with_y = align_up(off + P * sizeof(int)) + align_up(static_cast<size_t>(P) * d * sizeof(float));
+  if (d > 0 && P >= 2048 && (with_y <= kOwn || off > kOwn || roomy)) {
+    L.pos_of = off;   off = align_up(off + P * sizeof(int));
+    L.y = off;        off = align_up(off + static_cast<size_t>(P) * d * sizeof(float));
+  }
   L.total = off;
   return L;
+}
+
+Layout layout_for(const latent_moe_args& a) {
+  const bool roomy = a.layout == LATENT_LAYOUT_ROWS && prefill::supported(a) && prefill::layout_for(a).total > kOwn;
+  return layout_for(a.n_tokens, a.n_expert_used, a.n_expert, a.max_rank, xh_cols(a), roomy);
 }
 
 int validate(const latent_moe_args& a) {
@@ -978,6 +1026,20 @@ int choose_path(const latent_moe_args& a) {
   return kPathGeneral;
 }
 
+// Whether a prefill call on the row layout takes the row-layout MFMA phases
+// rather than the grouped GEMMs, whose 128-pair tiles need a tile on every CU
+// (us, phases / GEMMs): E 64, d 2048, ff 1408, rank 128, top-6: 200 tokens 89
+// / 221, 1999 tokens (128 tiles) 252 / 291; E 16, d 4096, ff 2048, rank 128:
+// 2000 tokens 261 / 424; DeepSeek-V3 shape: 512 tokens 481 / 866, 1280 (208
+// tiles) 822 / 875, 1536 (224) 1,010 / 897, 4096 (384) 2,186 / 1,510.
+// LATENT_MOE_PATH=prefill keeps the GEMMs.
+bool rows_prefill(const latent_moe_args& a) {
+  if (a.layout != LATENT_LAYOUT_ROWS || !rows::supported(a)) return false;
+  const char* env = std::getenv("LATENT_MOE_PATH");
+  if (env && !std::strcmp(env, "prefill")) return false;
+  return a.n_tokens * a.n_expert_used / 128 + std::min(a.n_expert, a.n_tokens * a.n_expert_used) / 2 < 212;
+}
+
 template <int MB, bool kInt8>
 int launch_phases(const MoeParams& p, hipStream_t s) {
   const unsigned a_groups = static_cast<unsigned>((p.a_max + 7) / 8);
@@ -993,20 +1055,6 @@ int launch_phases(const MoeParams& p, hipStream_t s) {
   return LATENT_OK;
 }
 
-// Index of each bitmap word's first INT8 group: row_offset plus the set bits
-// of the row's earlier words (one thread per expert row).
-__global__ void __launch_bounds__(kThreads) int8_word_offset_kernel(const uint32_t* bitmap, const int32_t* row_offset,
-                                                                   int32_t* out, int64_t rows_total, int words) {
-  for (int64_t r = blockIdx.x * static_cast<int64_t>(kThreads) + threadIdx.x; r < rows_total;
-       r += static_cast<int64_t>(gridDim.x) * kThreads) {
-    int run = row_offset[r];
-    for (int w = 0; w < words; ++w) {
-      out[r * words + w] = run;
-      run += popc(bitmap[r * words + w]);
-    }
-  }
-}
-
 // Workspace tail holding the per-word INT8 offsets of the factors whose rows
 // span more than one bitmap word (factors of one word use row_offset).
 size_t int8_word_offset_bytes(const latent_moe_args& a) {
@@ -1019,9 +1067,10 @@ size_t int8_word_offset_bytes(const latent_moe_args& a) {
   return n;
 }
 
-// Fill `word_offset` of every INT8 factor: the workspace tail for factors of
-// more than one bitmap word (a kernel per factor), row_offset for the others.
-int set_int8_word_offsets(const latent_moe_args& a, char* tail, Factor (&fac)[6], hipStream_t s) {
+// Set `word_offset` of every INT8 factor: the workspace tail for factors of
+// more than one bitmap word (filled beside the grouping, see prep_rest),
+// row_offset for the others.
+void set_int8_word_offsets(const latent_moe_args& a, char* tail, MoeParams& p) {
   const latent_factor* fs[6] = {&a.gate_a, &a.gate_b, &a.up_a, &a.up_b, &a.down_a, &a.down_b};
   size_t off = 0;
   for (int i = 0; i < 6; ++i) {
@@ -1029,18 +1078,15 @@ int set_int8_word_offsets(const latent_moe_args& a, char* tail, Factor (&fac)[6]
     if (!f.int8_bitmap) continue;
     const int64_t words = (f.cols / kGroup + 31) / 32;
     if (words == 1) {
-      fac[i].ext.word_offset = f.int8_row_offset;
+      p.fac[i].ext.word_offset = f.int8_row_offset;
       continue;
     }
     int32_t* dst = reinterpret_cast<int32_t*>(tail + off);
-    const int64_t rows_total = a.n_expert * f.rows;
-    const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(1024, (rows_total + kThreads - 1) / kThreads));
-    hipLaunchKernelGGL(int8_word_offset_kernel, dim3(blocks), dim3(kThreads), 0, s, f.int8_bitmap, f.int8_row_offset,
-                       dst, rows_total, static_cast<int>(words));
-    fac[i].ext.word_offset = dst;
-    off += align_up(static_cast<size_t>(rows_total * words) * sizeof(int32_t));
+    const int64_t rows = a.n_expert * f.rows;
+    p.off[p.n_off++] = WordOffsets{f.int8_bitmap, f.int8_row_offset, dst, rows, static_cast<int>(words)};
+    p.fac[i].ext.word_offset = dst;
+    off += align_up(static_cast<size_t>(rows * words) * sizeof(int32_t));
   }
-  return hipGetLastError() == hipSuccess ? LATENT_OK : LATENT_E_HIP;
 }
 
 }  // namespace
@@ -1067,7 +1113,7 @@ extern "C" int latent_moe_workspace_size(const latent_moe_args* args, size_t* by
   if (!args || !bytes) return LATENT_E_INVALID;
   const int st = validate(*args);
   if (st != LATENT_OK) return st;
-  const Layout L = layout_for(args->n_tokens, args->n_expert_used, args->n_expert, args->max_rank, xh_cols(*args));
+  const Layout L = layout_for(*args);
   size_t scratch = L.total;
   if (prefill::supported(*args)) scratch = std::max(scratch, L.gu + prefill::layout_for(*args).total);
   if (chain32::supported(*args)) scratch = std::max(scratch, L.gu + chain32::layout_for(*args).total);
@@ -1159,10 +1205,9 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
     size_t total = 0;
     latent_moe_workspace_size(&a, &total);
     char* tail = static_cast<char*>(a.workspace) + total - int8_word_offset_bytes(a);
-    st = set_int8_word_offsets(a, tail, p.fac, s);
-    if (st != LATENT_OK) return st;
+    set_int8_word_offsets(a, tail, p);
   }
-  const Layout L = layout_for(a.n_tokens, a.n_expert_used, a.n_expert, a.max_rank, xh_cols(a));
+  const Layout L = layout_for(a);
   char* ws = static_cast<char*>(a.workspace) + kControlBytes;
   p.x = a.x;
   p.ids = a.ids;
@@ -1190,7 +1235,7 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
   p.out_mode = a.out_mode;
   const int64_t P = a.n_tokens * a.n_expert_used;
   p.a_max = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(a.n_expert, P)));
-  const bool use_prefill = path == kPathPrefill;
+  const bool use_prefill = path == kPathPrefill && !rows_prefill(a);
   const bool use_stream = path == kPathStream;
   if (use_stream && stream::lite_applies(a)) {
     static_assert(stream::kLiteCtrlOffset + stream::kLiteCtrlBytes <= kControlBytes, "control block");
@@ -1204,7 +1249,7 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
     p.unit_info = reinterpret_cast<int4*>(ws + L.gu + CL.units);
     p.unit_tok = reinterpret_cast<int*>(p.unit_info + chain32::max_units(a));
     p.pos_of = reinterpret_cast<int*>(ws + L.gu + CL.pos_of);
-    hipLaunchKernelGGL(prep_kernel, dim3(1), dim3(kRouteThreads), 0, s, p);
+    hipLaunchKernelGGL(prep_kernel, dim3(p.n_off ? 257 : 1), dim3(kRouteThreads), 0, s, p);
     if (hipGetLastError() != hipSuccess) return LATENT_E_HIP;
     const chain32::Grouping g{p.meta, p.unit_info, p.unit_tok, p.pos_of, p.pair_w};
     return chain32::forward(a, p.fac, g, ws + L.gu, s);
@@ -1220,16 +1265,18 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
     p.xh = reinterpret_cast<_Float16*>(ws + L.gu + SL.xh);
     p.xexp = reinterpret_cast<int*>(ws + L.gu + SL.xexp);
   }
-  const bool use_rows = path == kPathRows;
+  const bool use_rows = path == kPathRows || (path == kPathPrefill && !use_prefill);
   if (use_rows) {
     p.xh = reinterpret_cast<_Float16*>(ws + L.xh);
     p.xexp = reinterpret_cast<int*>(ws + L.xexp);
     p.longest_first = 1;
   }
+  const bool y_rows = use_rows && L.y != 0 && a.out_mode == LATENT_OUT_REDUCED;
+  if (y_rows) p.pos_of = reinterpret_cast<int*>(ws + L.pos_of);
   // The MFMA paths write their intermediates whole, and every output row
   // (per-token combine); the row-layout MFMA phases accumulate like the fp32 ones.
   p.zero_floats = use_prefill || use_stream ? 0 : P * 3 * a.max_rank;
-  p.zero_out = use_prefill || use_stream ? 0 : 1;
+  p.zero_out = use_prefill || use_stream || y_rows ? 0 : 1;
   p.clear = use_stream ? 0 : 1;
 
   // Work split: enough items to fill 256 CUs even when few experts are routed.
@@ -1249,14 +1296,17 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
   // The streaming path and the row-layout MFMA phases also convert x, one
   // workgroup per token.
   const int64_t conv_blocks = use_stream || use_rows ? a.n_tokens : 1;
-  const int zero_blocks = static_cast<int>(
-      std::min<int64_t>(512, std::max<int64_t>(conv_blocks, zero_work / (kRouteThreads * 8))));
-  if (use_prefill) {
-    // Large batch: the multi-workgroup grouping; nothing to clear.
+  const int zero_blocks = static_cast<int>(std::min<int64_t>(
+      512, std::max<int64_t>(std::max<int64_t>(conv_blocks, p.n_off ? 256 : 0), zero_work / (kRouteThreads * 8))));
+  // Large batches: the multi-workgroup grouping, for the row-layout MFMA phases
+  // from 4096 pairs (64 experts, 11,994 pairs: 37 us in one workgroup), with
+  // the other preparations beside its first kernel; prefill has none.
+  if (use_prefill || (use_rows && P >= 4096)) {
     int* hist = reinterpret_cast<int*>(ws + L.hist);
     const int chunk = static_cast<int>(group_chunk(P, a.n_expert));
     const int nchunk = static_cast<int>(group_chunks(P, a.n_expert));
-    hipLaunchKernelGGL(group_count_kernel, dim3(nchunk), dim3(kRouteThreads), 0, s, p, hist, chunk);
+    hipLaunchKernelGGL(group_count_kernel, dim3(nchunk + (use_rows ? zero_blocks : 0)), dim3(kRouteThreads), 0, s, p, hist,
+                       chunk, nchunk);
     hipLaunchKernelGGL(group_scan_kernel, dim3(1), dim3(kRouteThreads), 0, s, p, hist, nchunk);
     hipLaunchKernelGGL(group_scatter_kernel, dim3(nchunk), dim3(kRouteThreads), 0, s, p, hist, chunk);
   } else {
@@ -1288,6 +1338,12 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
     rp.gu = p.gu;
     rp.dl = p.dl;
     rp.out = p.out;
+    rp.y = y_rows ? reinterpret_cast<float*>(ws + L.y) : nullptr;
+    rp.pos_of = p.pos_of;
+    rp.ids = p.ids;
+    rp.weights = p.weights;
+    rp.w_dtype = p.w_dtype;
+    rp.E = p.E;
     rp.T = p.T;
     rp.d = p.d;
     rp.ff = p.ff;
@@ -1296,7 +1352,7 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
     rp.wbd = p.wbd;
     rp.out_mode = p.out_mode;
     rp.a_max = p.a_max;
-    rows::plan(rp);
+    rows::plan(rp, any_int8);
     return rows::launch(rp, any_int8, s);
   }
   if (MB == 1)

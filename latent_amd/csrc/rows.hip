@@ -370,31 +370,63 @@ __device__ __forceinline__ void rank_gemm(const Factor& f, int e, int row0, int 
 
 // fp32 latent rows [m][.] (rank values of each, `stride` floats apart) as fp16
 // rows times a power of two in LDS (dst, dst_str bytes apart), zero past the
-// rank and past m up to `rows`; the exponents to rexp.  16 lanes per row.
-__device__ __forceinline__ void stage_rows(const float* src, int64_t stride, int rows, int m, int rank, int width,
-                                           uint32_t dst, uint32_t dst_str, int* rexp) {
+// rank (to `width`) and past m up to 16 MB rows; the exponents to rexp.  16
+// lanes per row; a row's values stay in registers between its maximum and the
+// conversion, and up to 16 loads of a lane are in flight (a second pass over
+// the rows, one row at a time, was half of phase BC's time at 64 pairs).
+template <int MB, int NV>
+__device__ __forceinline__ void stage_rows_n(const float* src, int stride, int m, int rank, int width,
+                                             uint32_t dst, uint32_t dst_str, int* rexp) {
+  typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+  constexpr int kRows = NV * MB <= 16 ? MB : 16 / NV;  // rows at a time
   const int t = threadIdx.x & 15;
-  for (int r = threadIdx.x >> 4; r < rows; r += kT / 16) {
-    const float* row = src + static_cast<int64_t>(min(r, m - 1)) * stride;
-    const int n4 = r < m ? (rank + 3) / 4 : 0;
-    float mx = 0.f;
-    for (int c = t; c < n4; c += 16) {
-      const float4v v = *reinterpret_cast<const float4v*>(row + 4 * c);
+  // Loads past row m read zeros: no branch and no mask per load.
+  const __amdgpu_buffer_rsrc_t rows = buffer_rsrc(src, static_cast<uint32_t>(m * stride - (stride - width)) * 4u);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) mx = 4 * c + q < rank ? fmaxf(mx, fabsf(v[q])) : mx;
+  for (int i0 = 0; i0 < MB; i0 += kRows) {
+    float4v v[kRows][NV];
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+      const int r = (threadIdx.x >> 4) + 16 * (i0 + i);
+#pragma unroll
+      for (int j = 0; j < NV; ++j)
+        v[i][j] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(
+                                                  rows, static_cast<uint32_t>(r * stride + 4 * t) * 4u, 256 * j, 0));
     }
-    mx = op_over(mx, 1, 16, OpMax{});
-    const int ex = pow2_row_exponent(mx);
-    if (t == 0) rexp[r] = ex;
-    for (int c = t; c < width / 4; c += 16) {
-      const float4v v = c < n4 ? *reinterpret_cast<const float4v*>(row + 4 * c) : float4v{0.f, 0.f, 0.f, 0.f};
-      typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-      half4 h;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) h[q] = static_cast<_Float16>(4 * c + q < rank ? ldexpf(v[q], ex) : 0.f);
-      lds_st<half4>(dst + r * dst_str + c * 8, h);
+    for (int i = 0; i < kRows; ++i) {
+      const int r = (threadIdx.x >> 4) + 16 * (i0 + i);
+      float mx = 0.f;
+#pragma unroll
+      for (int j = 0; j < NV; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          v[i][j][q] = 4 * (t + 16 * j) + q < rank ? v[i][j][q] : 0.f;
+          mx = fmaxf(mx, fabsf(v[i][j][q]));
+        }
+      mx = op_over(mx, 1, 16, OpMax{});
+      const int ex = pow2_row_exponent(mx);
+      if (t == 0) rexp[r] = ex;
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        if (4 * (t + 16 * j) >= width) continue;
+        half4 h;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) h[q] = static_cast<_Float16>(ldexpf(v[i][j][q], ex));
+        lds_st<half4>(dst + r * dst_str + (t + 16 * j) * 8, h);
+      }
     }
   }
+}
+template <int MB>
+__device__ __forceinline__ void stage_rows(const float* src, int stride, int m, int rank, int width, uint32_t dst,
+                                           uint32_t dst_str, int* rexp) {
+  if (width <= 128)
+    stage_rows_n<MB, 2>(src, stride, m, rank, width, dst, dst_str, rexp);
+  else if (width <= 256)
+    stage_rows_n<MB, 4>(src, stride, m, rank, width, dst, dst_str, rexp);
+  else
+    stage_rows_n<MB, 8>(src, stride, m, rank, width, dst, dst_str, rexp);
 }
 
 // Waves per SIMD the kernels are compiled for (four pair blocks take 128
@@ -409,7 +441,9 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) a_kernel(Params p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ int rexp[16 * MB];
   int a, item;
-  if (!map_item(blockIdx.x, p.n_a, p.meta[0], a, item)) return;
+  if (!map_item(blockIdx.x, p.n_a * p.n_pass, p.meta[0], a, item)) return;
+  const int pass = item / p.n_a;
+  item -= pass * p.n_a;
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int kind = item & 1, split = item >> 1;
   const int e = p.act_expert[a], s0 = p.act_start[a], mtot = p.act_count[a];
@@ -421,7 +455,7 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) a_kernel(Params p) {
   if (blk0 == blk1) return;
   const uint32_t lut0 = lds_addr(smem), lut = lut0 + (lane & (kCopies - 1)) * 4;
   const uint32_t meta = lut0 + kLutBytes + uniform(tid >> 6) * kMetaBytes;
-  for (int tb = 0; tb < mtot; tb += 16 * MB) {
+  for (int tb = 16 * MB * pass; tb < mtot; tb += 16 * MB * p.n_pass) {
     const int m = min(16 * MB, mtot - tb);
     ActX<MB> act;
 #pragma unroll
@@ -449,7 +483,9 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) bc_kernel(Params p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ int rexp[2][16 * MB], hexp[16 * MB];
   int a, item;
-  if (!map_item(blockIdx.x, p.n_bc, p.meta[0], a, item)) return;
+  if (!map_item(blockIdx.x, p.n_bc * p.n_pass, p.meta[0], a, item)) return;
+  const int pass = item / p.n_bc;
+  item -= pass * p.n_bc;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform(tid >> 6);
   const int n = lane & 15, kq = lane >> 4;
   const int e = p.act_expert[a], s0 = p.act_start[a], mtot = p.act_count[a];
@@ -466,15 +502,15 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) bc_kernel(Params p) {
   const int kind = wave & 1, tile = wave >> 1;
   const int nb = tile * 128 < ncol ? ((kind ? ru : rg) + 31) / 32 : 0;
   const int cols = (rd + kGroup - 1) / kGroup * kGroup;
-  for (int tb = 0; tb < mtot; tb += 16 * MB) {
+  for (int tb = 16 * MB * pass; tb < mtot; tb += 16 * MB * p.n_pass) {
     const int m = min(16 * MB, mtot - tb);
     Walk<8, MB, kInt8, ActLds> walk(
         p.fac[kind ? F_UP_B : F_GATE_B], e, min(c0 + tile * 128, p.ff - 32), 0, 0, nb, lane, meta,
         ActLds{L_lat + n * lstr + static_cast<uint32_t>(kind * p.R + 8 * kq) * 2u, 16u * lstr});
     walk.start();
     const float* gu = p.gu + static_cast<int64_t>(s0 + tb) * (2 * p.R);
-    stage_rows(gu, 2 * p.R, 16 * MB, m, rg, p.R, L_lat, lstr, rexp[0]);
-    stage_rows(gu + p.R, 2 * p.R, 16 * MB, m, ru, p.R, L_lat + 2u * p.R, lstr, rexp[1]);
+    stage_rows<MB>(gu, 2 * p.R, m, rg, p.R, L_lat, lstr, rexp[0]);
+    stage_rows<MB>(gu + p.R, 2 * p.R, m, ru, p.R, L_lat + 2u * p.R, lstr, rexp[1]);
     lds_barrier();
     float4v acc[MB][8];
     walk.run(lut, acc);
@@ -530,7 +566,9 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) d_kernel(Params p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ int rexp[16 * MB];
   int a, item;
-  if (!map_item(blockIdx.x, p.n_d, p.meta[0], a, item)) return;
+  if (!map_item(blockIdx.x, p.n_d * p.n_pass, p.meta[0], a, item)) return;
+  const int pass = item / p.n_d;
+  item -= pass * p.n_d;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform(tid >> 6);
   const int n = lane & 15, kq = lane >> 4;
   const int e = p.act_expert[a], s0 = p.act_start[a], mtot = p.act_count[a];
@@ -541,12 +579,12 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) d_kernel(Params p) {
   const uint32_t lut0 = lds_addr(smem), L_lat = lut0 + kFixBytes, lut = lut0 + (lane & (kCopies - 1)) * 4;
   const uint32_t meta = lut0 + kLutBytes + wave * kMetaBytes;
   lut_fill(lut0, tid);
-  for (int tb = 0; tb < mtot; tb += 16 * MB) {
+  for (int tb = 16 * MB * pass; tb < mtot; tb += 16 * MB * p.n_pass) {
     const int m = min(16 * MB, mtot - tb);
     Walk<8, MB, kInt8, ActLds> walk(p.fac[F_DOWN_B], e, min(ct, p.d - 32), 0, 0, nb, lane, meta,
                                     ActLds{L_lat + n * lstr + 16u * kq, 16u * lstr});
     walk.start();
-    stage_rows(p.dl + static_cast<int64_t>(s0 + tb) * p.R, p.R, 16 * MB, m, rd, p.R, L_lat, lstr, rexp);
+    stage_rows<MB>(p.dl + static_cast<int64_t>(s0 + tb) * p.R, p.R, m, rd, p.R, L_lat, lstr, rexp);
     lds_barrier();
     float4v acc[MB][8];
     walk.run(lut, acc);
@@ -564,16 +602,18 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) d_kernel(Params p) {
       for (int r = 0; r < rows; ++r) {
         const int pair = s0 + tb + half * 8 + r, tok = p.pair_tok[pair];
         const float sc = ldexpf(1.0f, -rexp[half * 8 + r]);
-        const float w = p.out_mode == LATENT_OUT_REDUCED && !p.wbd ? p.pair_w[pair] * sc : sc;
-        float* dst = p.out + (p.out_mode == LATENT_OUT_REDUCED ? static_cast<int64_t>(tok)
-                                                               : static_cast<int64_t>(tok) * p.K + p.pair_slot[pair]) * p.d;
+        const bool add = p.out_mode == LATENT_OUT_REDUCED && !p.y;
+        const float w = add && !p.wbd ? p.pair_w[pair] * sc : sc;
+        float* dst = p.y ? p.y + static_cast<int64_t>(pair) * p.d
+                   : add ? p.out + static_cast<int64_t>(tok) * p.d
+                         : p.out + (static_cast<int64_t>(tok) * p.K + p.pair_slot[pair]) * p.d;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const int col = c0 + t * 256 + tid;
           if (col >= p.d) continue;
           const float y = w * lds_ld<float>(L_lat + (2 * t + (tid >> 7)) * kHalfSlot +
                                             static_cast<uint32_t>(r * kTileStr + (tid & 127)) * 4u);
-          if (p.out_mode == LATENT_OUT_REDUCED)
+          if (add)
             atomic_add_f32(dst + col, y);
           else
             dst[col] = y;
@@ -582,6 +622,22 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) d_kernel(Params p) {
     }
     lds_barrier();  // the products are read
   }
+}
+
+// Reduced output from y rows: the weighted sum over a token's slots in slot
+// order, one float4 per thread.
+__global__ void __launch_bounds__(kT) combine_kernel(Params p) {
+  const int d4 = p.d / 4, t = blockIdx.y, c = blockIdx.x * kT + threadIdx.x;
+  if (c >= d4) return;
+  float4v s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int k = 0; k < p.K; ++k) {
+    const int slot = t * p.K + k, e = p.ids[slot];
+    if (e < 0 || e >= p.E) continue;
+    const float w = p.wbd ? 1.0f : load_act(p.weights, p.w_dtype, slot);
+    s += w * reinterpret_cast<const float4v*>(p.y + static_cast<int64_t>(p.pos_of[slot]) * p.d)[c];
+  }
+  reinterpret_cast<float4v*>(p.out + static_cast<int64_t>(t) * p.d)[c] = s;
 }
 
 // Dynamic LDS bytes of the phases.
@@ -597,10 +653,11 @@ size_t lds_d(int R) {
 
 template <int MB, bool kInt8>
 int launch_phases(const Params& p, hipStream_t s) {
-  const unsigned groups = static_cast<unsigned>((p.a_max + 7) / 8);
+  const unsigned groups = static_cast<unsigned>((p.a_max + 7) / 8 * p.n_pass);
   hipLaunchKernelGGL((a_kernel<MB, kInt8>), dim3(8 * groups * p.n_a), dim3(kT), lds_a(), s, p);
   hipLaunchKernelGGL((bc_kernel<MB, kInt8>), dim3(8 * groups * p.n_bc), dim3(kT), lds_bc<MB>(p.R), s, p);
   hipLaunchKernelGGL((d_kernel<MB, kInt8>), dim3(8 * groups * p.n_d), dim3(kT), lds_d<MB>(p.R), s, p);
+  if (p.y) hipLaunchKernelGGL(combine_kernel, dim3((p.d / 4 + kT - 1) / kT, p.T), dim3(kT), 0, s, p);
   return hipGetLastError() == hipSuccess ? LATENT_OK : LATENT_E_HIP;
 }
 
@@ -619,28 +676,41 @@ bool supported(const latent_moe_args& a) {
   return true;
 }
 
-void plan(Params& p) {
-  // Phase A ranges per expert and factor at the full rank (a smaller rank has
-  // fewer): about 4096 items in all, of eight blocks of 32 rows or more.
-  int s = 4;
-  while (s < 32 && 2ll * p.a_max * s < 4096 && p.d / 32 >= 16 * s) s *= 2;
-  p.na_split = s;
-  p.n_a = 2 * s;
+// Pair blocks a decoded block of the factor is multiplied with: an expert of
+// many pairs then decodes its factors once per 64 (or 32) of them.  E 128, d
+// 4096, ff 1408, rank 64, top-8: 200 tokens (12 pairs an expert) 99 us at one
+// block and 110 at two, 2000 tokens 674 at one and 568 at four; E 64, d 2048,
+// rank 192, 200 tokens (19 pairs): 124 at one, 116 at two.
+int pair_blocks(const Params& p, bool int8) {
+  const int64_t per = static_cast<int64_t>(p.T) * p.K / p.a_max;
+  return int8 || per < 16 ? 1 : per < 24 ? 2 : 4;
+}
+
+void plan(Params& p, bool int8) {
+  // Workgroups that share an expert's passes, up to four rounds of phase D's items.
+  const int64_t step = 16 * pair_blocks(p, int8);
+  const int64_t passes = (3 * static_cast<int64_t>(p.T) * p.K / (2 * p.a_max) + step - 1) / step;  // half over the mean
   p.n_bc = (p.ff + kCB - 1) / kCB;
   p.n_d = (p.d + kCD - 1) / kCD;
+  p.n_pass = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(passes, 2048 / (static_cast<int64_t>(p.a_max) * p.n_d))));
+  // Phase A ranges per expert and factor at the full rank (a smaller rank has
+  // fewer): about 4096 items in all, of eight blocks of 32 rows or more; with
+  // 64 pairs a pass the items are eight times as long, and their sums cost as
+  // many atomics per range.
+  const int64_t want = step == 64 ? 512 : 4096;
+  int s = step == 64 ? 1 : 4;
+  while (s < 32 && 2ll * p.a_max * p.n_pass * s < want && p.d / 32 >= 16 * s) s *= 2;
+  p.na_split = s;
+  p.n_a = 2 * s;
 }
 
 int launch(const Params& p, bool int8, hipStream_t s) {
-  // Pair blocks a decoded block of the factor is multiplied with: an expert of
-  // many pairs then decodes its factors once per 64 (or 32) of them.  E 128, d
-  // 4096, ff 1408, rank 64, top-8: 200 tokens (12 pairs an expert) 99 us at
-  // one block and 110 at two, 2000 tokens 674 at one and 568 at four; E 64, d
-  // 2048, rank 192, 200 tokens (19 pairs): 124 at one, 116 at two.
   if (int8) return launch_phases<1, true>(p, s);
-  const int64_t per = static_cast<int64_t>(p.T) * p.K / p.a_max;
-  if (per >= 24) return launch_phases<4, false>(p, s);
-  if (per >= 16) return launch_phases<2, false>(p, s);
-  return launch_phases<1, false>(p, s);
+  switch (pair_blocks(p, false)) {
+    case 4: return launch_phases<4, false>(p, s);
+    case 2: return launch_phases<2, false>(p, s);
+    default: return launch_phases<1, false>(p, s);
+  }
 }
 
 }  // namespace rows

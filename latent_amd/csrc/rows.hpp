@@ -27,18 +27,24 @@ struct Params {
   const int* xexp;     // [T]
   float* gu;           // [P][2R] gate and up latents (accumulated)
   float* dl;           // [P][R] down latents (accumulated)
+  float* y;            // [P][d] rows of the routed pairs, combined at the end (NULL: summed into out)
+  const int* pos_of;   // [T*K] grouped position of each routed slot (with y)
+  const int32_t* ids;  // with y
+  const void* weights;
+  int w_dtype, E;
   float* out;
   int T, d, ff, K, R, wbd, out_mode;
   int a_max;     // upper bound of the active experts (grid)
   int na_split;  // phase A: K ranges per factor
   int n_a, n_bc, n_d;  // items per active expert
+  int n_pass;          // workgroups that share an item's passes
 };
 
 // The row-layout shapes the kernels take (d, ff multiples of 32, max_rank at
 // most 512, x 16-byte aligned for the fp16 conversion).
 bool supported(const latent_moe_args& a);
-// Sets the work split (na_split, n_a, n_bc, n_d) of p from its shape.
-void plan(Params& p);
+// Sets the work split (na_split, n_a, n_bc, n_d, n_pass) of p from its shape.
+void plan(Params& p, bool int8);
 int launch(const Params& p, bool int8, hipStream_t s);
 
 }  // namespace rows

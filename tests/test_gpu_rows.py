@@ -124,3 +124,38 @@ def test_rows_pair_blocks(gpu, T, k, mode, wbd):
     ids[rng.random(ids.shape) < 0.05] = -1
     got, want = _run(gpu, host, dev, x, ids, w, wbd=wbd, mode=mode)
     assert ref.rel_l2(want, got) <= TOL
+
+
+@pytest.mark.parametrize("T,E,d,ff,R,mode", [
+    (2050, 7, 288, 544, 128, 0),   # y rows and the per-token combine; passes shared by workgroups
+    (2050, 7, 384, 640, 128, 1),   # also a shape of the GEMMs
+    (1400, 5, 1056, 256, 64, 0),   # three pairs a token: 4200 pairs, the multi-workgroup grouping
+])
+def test_rows_large_batches(gpu, monkeypatch, T, E, d, ff, R, mode):
+    """Batches from 2048 pairs (y rows) and 4096 (grouping in several
+    workgroups), one hot expert; a sample of the tokens against the oracle,
+    every token of the two output modes and of the GEMM engine (where the rank
+    allows it) against each other."""
+    import torch
+
+    host = synth.make_layer(seed=95, n_expert=E, d=d, ff=ff, max_rank=R)
+    dev = _rows_layer(host)
+    rng = np.random.default_rng(T + R)
+    k = 3 if R == 64 else 2
+    x = torch.from_numpy(rng.standard_normal((T, d)).astype(np.float32)).cuda()
+    logits = rng.standard_normal((T, E))
+    logits[:, 3] += 1.5
+    ids, w = routing.softmax_topk(logits, k)
+    ids[rng.random(ids.shape) < 0.03] = -1
+    it, wt = torch.from_numpy(ids.astype(np.int32)).cuda(), torch.from_numpy(w.astype(np.float32)).cuda()
+    got = gpu.moe_forward(x, it, wt, dev, out_mode=mode).cpu().numpy()
+    pick = np.array(sorted(set(range(0, T, T // 40)) | {T - 1}))
+    want = ref.moe_forward(x.cpu().numpy()[pick], ids[pick], w[pick], host, out_mode=mode)
+    assert ref.rel_l2(want, got[pick]) <= TOL
+    other = gpu.moe_forward(x, it, wt, dev, out_mode=1 - mode).cpu().numpy().astype(np.float64)
+    slots, red = (other, got) if mode == 0 else (got.astype(np.float64), other)
+    assert ref.rel_l2((slots * np.where(ids >= 0, w, 0.0)[..., None]).sum(1), red) <= 1e-4
+    if R % 128 == 0 and d % 128 == 0:
+        monkeypatch.setenv("LATENT_MOE_PATH", "prefill")
+        gemm = gpu.moe_forward(x, it, wt, dev, out_mode=mode).cpu().numpy()
+        assert ref.rel_l2(gemm, got) <= TOL
