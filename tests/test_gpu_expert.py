@@ -129,3 +129,31 @@ def test_weight_ignored_without_weight_before_down(gpu):
     assert np.array_equal(g1, g2)
     _, gw = _both(arrays, x, weight=0.1, wbd=True)
     assert ref.rel_l2(0.1 * g1, gw) <= 1e-5
+
+
+@pytest.mark.parametrize("T,d,ff,ranks,kind", [
+    (1, 2048, 64, (256, 1, 255), "nf4"),    # one column of ff tiles, the largest rank beside the smallest
+    (9, 33, 4096, (3, 64, 65), "nf4"),      # two token tiles, 64 column tiles in 32 ranges, a slice of one row
+    (8, 100, 129, (64, 37, 200), "int8"),
+    (4, 2049, 70, (40, 40, 40), "nf4"),     # one past the chain's d, ff and rank: a launch per product
+    (5, 64, 4100, (40, 33, 40), "int8"),
+    (3, 70, 96, (40, 40, 257), "nf4"),
+])
+def test_chain_limits(gpu, T, d, ff, ranks, kind):
+    """Both sides of the three-launch chain's limits, against fp32 sums of the
+    same decoded factors: a sum of K terms rounds to about sqrt(K) 2^-24 (4e-6 at
+    4096), four of them in a chain."""
+    rng = np.random.default_rng(T * 100 + d)
+    arrays = {}
+    dims = {"gate": (d, ranks[0], ff), "up": (d, ranks[1], ff), "down": (ff, ranks[2], d)}
+    for name, (n_in, r, n_out) in dims.items():
+        for side, shape in (("a", (n_in, r)), ("b", (r, n_out))):
+            m = (rng.standard_normal(shape) / np.sqrt(shape[0])).astype(np.float32)
+            data, scales, _ = ref.quantize_nf4(m) if kind == "nf4" else ref.quantize_int8(m)
+            arrays[f"{name}.{side}.{kind}"] = data
+            arrays[f"{name}.{side}.scales"] = scales
+            arrays[f"{name}.{side}.shape"] = np.array(shape)
+    x = rng.standard_normal((T, d)).astype(np.float32)
+    want, got = _both(arrays, x, weight=0.7, wbd=True)
+    assert ref.rel_l2(want, got) <= 1e-5
+    assert np.array_equal(got, _both(arrays, x, weight=0.7, wbd=True)[1])
