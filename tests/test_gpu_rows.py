@@ -126,6 +126,30 @@ def test_rows_pair_blocks(gpu, T, k, mode, wbd):
     assert ref.rel_l2(want, got) <= TOL
 
 
+@pytest.mark.parametrize("E,T,k", [
+    (512, 700, 3),   # rounds of 1024 pairs: two and a part, the most experts they take
+    (513, 260, 4),   # rounds of 512 pairs: two and 16 pairs
+    (1024, 128, 4),  # one whole round, the most experts placed in order
+    (1025, 129, 4),  # more experts: placed as the threads come
+])
+def test_rows_grouping_rounds(gpu, E, T, k):
+    """The grouping's placement rounds at their edges, a hot expert over every
+    round, dropped slots, ids past the last expert and a repeated expert."""
+    host = synth.make_layer(seed=E, n_expert=E, d=64, ff=64, max_rank=32)
+    dev = _rows_layer(host)
+    rng = np.random.default_rng(E + T)
+    x = rng.standard_normal((T, host.d)).astype(np.float32)
+    ids = rng.integers(0, E, (T, k)).astype(np.int32)
+    w = rng.random((T, k)).astype(np.float32)
+    ids[::3, 0] = E - 1
+    ids[1::7, 1] = -1
+    ids[2::11, 1] = E
+    ids[5::13, 1] = ids[5::13, 0]
+    for mode in (0, 1):
+        got, want = _run(gpu, host, dev, x, ids, w, mode=mode)
+        assert ref.rel_l2(want, got) <= TOL
+
+
 @pytest.mark.parametrize("T,E,d,ff,R,mode", [
     (2050, 7, 288, 544, 128, 0),   # y rows and the per-token combine; passes shared by workgroups
     (2050, 7, 384, 640, 128, 1),   # also a shape of the GEMMs
