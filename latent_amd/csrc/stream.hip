@@ -120,11 +120,12 @@ struct Params {
   int* dexp;           // [P]
   float* ybuf;         // [P][d]
   int T, K, E, d, ff, P, wbd, out_mode;
+  int direct;            // phase D writes the per-slot output itself
   int nka, nb, nkc, nd;  // tiles per unit and factor: A (d/256), B (ff/128), C (ff/256), D (d/256)
   int G;                 // workgroups the tile ranges are cut for
-  // Bulk (prefill) launches only.
-  const int* pair_tok;    // [P] token of each grouped pair
+  const int* pair_tok;    // [P] token of each grouped pair (bulk launches, direct)
   const int* pair_slot;   // [P] slot of each grouped pair
+  // Bulk (prefill) launches only.
   const float* pair_w;    // [P] router weight of each grouped pair
   const int* nunits;      // number of units (reduce kernels; the decode launches set meta + 4)
   _Float16* yh;           // reduced output: [P][d] fp16 y rows * 2^yexp
@@ -417,7 +418,11 @@ __device__ __forceinline__ int part_slot(int b, int key, int chunk, int per_key,
   return b * maxj + key - (b * chunk) / per_key;
 }
 
-template <int kPhase>
+// kSlots (phase D of a per-slot call that weights after the down projection): a
+// pair's exponent word also holds its output row (reduce_kernel), and y goes
+// there: with the copy from y rows to slots 289 us, without it 263 (301 tokens,
+// top-8 of 256 experts, d 7168).
+template <int kPhase, bool kSlots = false>
 __global__ void __launch_bounds__(kT, kGroupsPerCU) item_kernel(Params p) {
   static_assert(kPhase == kPhaseA || kPhase == kPhaseD, "phases B and C run in bc_kernel");
   __shared__ ItemLds sm;
@@ -517,8 +522,10 @@ __global__ void __launch_bounds__(kT, kGroupsPerCU) item_kernel(Params p) {
       for (int v = 0; v < 4; ++v) {
         const int row = kq * 4 + v;
         if (row < tr.m) {
-          const float sc = ldexpf(1.0f, -lds_ld<int>(L + item_st(kStExp + (buf * 16 + row) * 4)));
-          float* dst = p.ybuf + static_cast<int64_t>(tr.start + row) * p.d + tr.r * kN + wave * 64 + n * 4;
+          const int ex = lds_ld<int>(L + item_st(kStExp + (buf * 16 + row) * 4));
+          const float sc = ldexpf(1.0f, kSlots ? -((ex << 24) >> 24) : -ex);
+          float* dst = (kSlots ? p.out + static_cast<int64_t>(ex >> 8) * p.d : p.ybuf + static_cast<int64_t>(tr.start + row) * p.d) +
+                       tr.r * kN + wave * 64 + n * 4;
           *reinterpret_cast<float4*>(dst) = make_float4(acc[0][v] * sc, acc[1][v] * sc, acc[2][v] * sc, acc[3][v] * sc);
         }
       }
@@ -773,8 +780,9 @@ __global__ void __launch_bounds__(kT, kGroupsPerCU) bc_kernel(Params p) {
   }
 }
 
-// A row of 256 sums -> fp16 row * 2^e and e (one wave, 4 columns per lane).
-__device__ __forceinline__ void finish_row(float4 s, _Float16* dst, int* dexp, int lane) {
+// A row of 256 sums -> fp16 row * 2^e and e (one wave, 4 columns per lane); with
+// a tag, e's word is tag * 256 + e.
+__device__ __forceinline__ void finish_row(float4 s, _Float16* dst, int* dexp, int lane, int tag = -1) {
   const float mx = op_over(fmaxf(fmaxf(fabsf(s.x), fabsf(s.y)), fmaxf(fabsf(s.z), fabsf(s.w))), 1, kWave, OpMax{});
   const int ex = pow2_row_exponent(mx);
   half4v h;
@@ -783,7 +791,7 @@ __device__ __forceinline__ void finish_row(float4 s, _Float16* dst, int* dexp, i
   h[2] = static_cast<_Float16>(ldexpf(s.z, ex));
   h[3] = static_cast<_Float16>(ldexpf(s.w, ex));
   reinterpret_cast<half4v*>(dst)[lane] = h;
-  if (lane == 0) *dexp = ex;
+  if (lane == 0) *dexp = tag < 0 ? ex : (tag << 8) | (ex & 255);
 }
 
 // How a bulk launch deals its keys (runs of `per_key` consecutive tiles that
@@ -937,13 +945,22 @@ __global__ void __launch_bounds__(kT) reduce_kernel(Params p) {
     if (kPhase == kPhaseA)
       finish_row(s, p.lat + (static_cast<int64_t>(f) * p.P + pair) * kK, p.lexp + f * p.P + pair, lane);
     else
-      finish_row(s, p.dlat + pair * kK, p.dexp + pair, lane);
+      finish_row(s, p.dlat + pair * kK, p.dexp + pair, lane, p.direct ? p.pair_tok[pair] * p.K + p.pair_slot[pair] : -1);
+  }
+  if constexpr (kPhase == kPhaseC && kPerItem) {
+    // Phase D writes no dropped slot's row.
+    for (int r = blockIdx.x; p.direct && r < p.P; r += gridDim.x) {
+      const int e = p.ids[r];
+      if (e >= 0 && e < p.E) continue;
+      float4* o = reinterpret_cast<float4*>(p.out + static_cast<int64_t>(r) * p.d);
+      for (int i = threadIdx.x; i < p.d / 4; i += kT) o[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
   }
 }
 
 // out from the y rows of the routed slots, in slot order: reduced mode sums
-// w * y over the token's slots; per-slot mode writes y (times w when the weight
-// goes before the down projection: y is linear in h) and zero for a dropped slot.
+// w * y over the token's slots; per-slot mode with the weight before
+// the down projection writes w * y (y is linear in h) and zero for a dropped slot.
 // d % 256 == 0, so the 64 float4 columns of a wave lie in one output row: the
 // slot's id, weight and grouped position are wave-uniform (scalar loads), and
 // the y rows of kCombineBatch slots are loaded before any is added.
@@ -980,10 +997,8 @@ __global__ void __launch_bounds__(kT) combine_kernel(Params p) {
       const int e = p.ids[r];
       if (e >= 0 && e < p.E) {
         s = reinterpret_cast<const float4*>(p.ybuf + static_cast<int64_t>(p.pos_of[r]) * p.d)[c4];
-        if (p.wbd) {
-          const float w = load_act(p.weights, p.w_dtype, r);
-          s.x *= w; s.y *= w; s.z *= w; s.w *= w;
-        }
+        const float w = load_act(p.weights, p.w_dtype, r);
+        s.x *= w; s.y *= w; s.z *= w; s.w *= w;
       }
     }
     reinterpret_cast<float4*>(p.out)[i] = s;
@@ -2757,6 +2772,11 @@ int forward(const latent_moe_args& a, const Grouping& g, char* scratch, hipStrea
   p.P = p.T * p.K;
   p.wbd = a.weight_before_down ? 1 : 0;
   p.out_mode = a.out_mode;
+  // reduce_kernel tags a pair's exponent with its output row (T * K rows).
+  static_assert(kMaxPairs < (1 << 23), "output row in 23 bits");
+  p.direct = p.out_mode == LATENT_OUT_PER_SLOT && !p.wbd ? 1 : 0;
+  p.pair_tok = g.pair_tok;
+  p.pair_slot = g.pair_slot;
   p.nka = p.d / kK;
   p.nb = p.ff / kHBlock;
   p.nkc = p.ff / kK;
@@ -2774,6 +2794,10 @@ int forward(const latent_moe_args& a, const Grouping& g, char* scratch, hipStrea
   hipLaunchKernelGGL(bc_kernel, dim3(item_grid(p.nkc)), dim3(kT), 0, s, p);
   hipLaunchKernelGGL((reduce_kernel<kPhaseC, kMaxM, true>), dim3(blocks((U * kMaxM + rows_per_block - 1) / rows_per_block)),
                      dim3(kT), 0, s, p);
+  if (p.direct) {
+    hipLaunchKernelGGL((item_kernel<kPhaseD, true>), dim3(item_grid(p.nd)), dim3(kT), 0, s, p);
+    return hipGetLastError() == hipSuccess ? LATENT_OK : LATENT_E_HIP;
+  }
   hipLaunchKernelGGL(item_kernel<kPhaseD>, dim3(item_grid(p.nd)), dim3(kT), 0, s, p);
   const int64_t out4 = (a.out_mode == LATENT_OUT_REDUCED ? p.T : static_cast<int64_t>(p.P)) * p.d / 4;
   hipLaunchKernelGGL(combine_kernel, dim3(blocks((out4 + kT - 1) / kT)), dim3(kT), 0, s, p);

@@ -97,6 +97,32 @@ def test_stream_units_dropped_duplicate_and_invalid(gpu, stream_path, small_laye
             assert not got[0, 1].any() and not got[1, 2].any()
 
 
+@pytest.mark.parametrize("T,k", [(1, 2), (33, 1), (17, 5), (301, 8)])
+def test_stream_slot_rows(gpu, stream_path, small_layer, small_dev, T, k):
+    """Every row of a per-slot output, written over NaN: tokens from 1e-6 to 1e6
+    (exponents of both signs), dropped and out-of-range slots at both ends."""
+    import torch
+
+    rng = np.random.default_rng(T)
+    x = (rng.standard_normal((T, 1024)) * 10.0 ** rng.integers(-6, 7, (T, 1))).astype(np.float32)
+    ids, w = routing.softmax_topk(rng.standard_normal((T, 12)), k)
+    ids[0, 0], ids[-1, -1] = -1, 12
+    ids[rng.random(ids.shape) < 0.05] = -7
+    xt = torch.from_numpy(x).cuda()
+    it, wt = torch.from_numpy(ids.astype(np.int32)).cuda(), torch.from_numpy(w.astype(np.float32)).cuda()
+    for wbd in (False, True):
+        out = torch.full((T, k, 1024), float("nan"), device="cuda")
+        gpu.moe_forward(xt, it, wt, small_dev, weight_before_down=wbd, out_mode=1, out=out)
+        got = out.cpu().numpy()
+        want = ref.moe_forward(x, np.where(ids >= 12, -1, ids), w, small_layer, weight_before_down=wbd, out_mode=1)
+        live = (ids >= 0) & (ids < 12)
+        assert not got[~live].any() and np.isfinite(got).all()
+        # Each row by its own size: the tokens span twelve decades.
+        if live.any():
+            err = np.linalg.norm((got - want)[live], axis=-1) / np.linalg.norm(want[live], axis=-1)
+            assert err.max() <= 2 * TOL
+
+
 def test_stream_all_dropped(gpu, stream_path, small_dev):
     import torch
 
