@@ -561,7 +561,12 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) bc_kernel(Params p) {
 // ---------------------------------------------------------------------------
 // Phase D: d_lat . B_d over 512 columns of d, weighted into out
 // ---------------------------------------------------------------------------
-template <int MB, bool kInt8>
+// kAdd: weighted into the reduced output by atomics.  Otherwise into rows of
+// their own (y, or the per-slot output), each lane its eight columns: through
+// LDS, a row at a time like the atomics, the stores of 98 MB of y rows (11,994
+// pairs, d 2048) took the phase 67 us, from the registers 38 (with 10 % INT8
+// groups, one pair block a pass, both ways level).
+template <int MB, bool kInt8, bool kAdd>
 __global__ void __launch_bounds__(kT, waves_for(MB)) d_kernel(Params p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ int rexp[16 * MB];
@@ -588,7 +593,27 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) d_kernel(Params p) {
     lds_barrier();
     float4v acc[MB][8];
     walk.run(lut, acc);
-    // Eight rows of every wave's products at a time.
+    if constexpr (!kAdd) {
+      const int col = ct + n * 8;
+#pragma unroll
+      for (int b = 0; b < MB; ++b) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int row = 16 * b + 4 * kq + v;
+          if (row >= m || col >= p.d) continue;
+          const int pair = s0 + tb + row;
+          const int64_t orow = p.y ? pair : static_cast<int64_t>(p.pair_tok[pair]) * p.K + p.pair_slot[pair];
+          float4v* dst = reinterpret_cast<float4v*>((p.y ? p.y : p.out) + orow * p.d + col);
+          const float sc = ldexpf(1.0f, -rexp[row]);
+          dst[0] = sc * float4v{acc[b][0][v], acc[b][1][v], acc[b][2][v], acc[b][3][v]};
+          dst[1] = sc * float4v{acc[b][4][v], acc[b][5][v], acc[b][6][v], acc[b][7][v]};
+        }
+      }
+      lds_barrier();  // the latents are read
+      continue;
+    }
+    // Eight rows of every wave's products at a time, one row at a time over the
+    // workgroup: a wave's atomics cover consecutive columns.
     const uint32_t at = L_lat + wave * kHalfSlot + static_cast<uint32_t>((kq & 1) * 4 * kTileStr + n * 8) * 4u;
 #pragma unroll
     for (int half = 0; half < 2 * MB; ++half) {
@@ -596,27 +621,18 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) d_kernel(Params p) {
       lds_barrier();  // the latents (or the last rows' products) are read
       if ((kq >> 1) == (half & 1)) store_tile(at, acc[half >> 1]);
       lds_barrier();
-      // One row at a time over the workgroup: a wave's stores and atomics
-      // cover consecutive columns.
       const int rows = min(8, m - half * 8);
       for (int r = 0; r < rows; ++r) {
-        const int pair = s0 + tb + half * 8 + r, tok = p.pair_tok[pair];
+        const int pair = s0 + tb + half * 8 + r;
         const float sc = ldexpf(1.0f, -rexp[half * 8 + r]);
-        const bool add = p.out_mode == LATENT_OUT_REDUCED && !p.y;
-        const float w = add && !p.wbd ? p.pair_w[pair] * sc : sc;
-        float* dst = p.y ? p.y + static_cast<int64_t>(pair) * p.d
-                   : add ? p.out + static_cast<int64_t>(tok) * p.d
-                         : p.out + (static_cast<int64_t>(tok) * p.K + p.pair_slot[pair]) * p.d;
+        const float w = p.wbd ? sc : p.pair_w[pair] * sc;
+        float* dst = p.out + static_cast<int64_t>(p.pair_tok[pair]) * p.d;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const int col = c0 + t * 256 + tid;
-          if (col >= p.d) continue;
-          const float y = w * lds_ld<float>(L_lat + (2 * t + (tid >> 7)) * kHalfSlot +
-                                            static_cast<uint32_t>(r * kTileStr + (tid & 127)) * 4u);
-          if (add)
-            atomic_add_f32(dst + col, y);
-          else
-            dst[col] = y;
+          if (col < p.d)
+            atomic_add_f32(dst + col, w * lds_ld<float>(L_lat + (2 * t + (tid >> 7)) * kHalfSlot +
+                                                        static_cast<uint32_t>(r * kTileStr + (tid & 127)) * 4u));
         }
       }
     }
@@ -656,7 +672,10 @@ int launch_phases(const Params& p, hipStream_t s) {
   const unsigned groups = static_cast<unsigned>((p.a_max + 7) / 8 * p.n_pass);
   hipLaunchKernelGGL((a_kernel<MB, kInt8>), dim3(8 * groups * p.n_a), dim3(kT), lds_a(), s, p);
   hipLaunchKernelGGL((bc_kernel<MB, kInt8>), dim3(8 * groups * p.n_bc), dim3(kT), lds_bc<MB>(p.R), s, p);
-  hipLaunchKernelGGL((d_kernel<MB, kInt8>), dim3(8 * groups * p.n_d), dim3(kT), lds_d<MB>(p.R), s, p);
+  if (!p.y && p.out_mode == LATENT_OUT_REDUCED)
+    hipLaunchKernelGGL((d_kernel<MB, kInt8, true>), dim3(8 * groups * p.n_d), dim3(kT), lds_d<MB>(p.R), s, p);
+  else
+    hipLaunchKernelGGL((d_kernel<MB, kInt8, false>), dim3(8 * groups * p.n_d), dim3(kT), lds_d<MB>(p.R), s, p);
   if (p.y) hipLaunchKernelGGL(combine_kernel, dim3((p.d / 4 + kT - 1) / kT, p.T), dim3(kT), 0, s, p);
   return hipGetLastError() == hipSuccess ? LATENT_OK : LATENT_E_HIP;
 }
