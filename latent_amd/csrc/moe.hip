@@ -1043,8 +1043,8 @@ int choose_path(const latent_moe_args& a) {
 // Whether a prefill call on the row layout takes the row-layout MFMA phases
 // rather than the grouped GEMMs, whose 128-pair tiles need a tile on every CU
 // (us, phases / GEMMs): E 64, d 2048, ff 1408, rank 128, top-6: 200 tokens 89
-// / 221, 1999 tokens (128 tiles) 252 / 291; E 16, d 4096, ff 2048, rank 128:
-// 2000 tokens 261 / 424; DeepSeek-V3 shape: 512 tokens 481 / 866, 1280 (208
+// / 221, 1999 tokens (128 tiles) 217 / 291; E 16, d 4096, ff 2048, rank 128:
+// 2000 tokens 236 / 424; DeepSeek-V3 shape: 512 tokens 481 / 866, 1280 (208
 // tiles) 822 / 875, 1536 (224) 1,010 / 897, 4096 (384) 2,186 / 1,510.
 // LATENT_MOE_PATH=prefill keeps the GEMMs.
 bool rows_prefill(const latent_moe_args& a) {
