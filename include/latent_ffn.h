@@ -144,7 +144,11 @@ int latent_version(void);
 /* Static text for a status code. */
 const char* latent_status_string(int status);
 
-/* Workspace bytes required by latent_moe_ffn_forward for these dims. */
+/*
+ * Workspace bytes for latent_moe_ffn_forward with these dims.  A call given
+ * less runs where its kernels have a form that needs less (row-layout prefill:
+ * the grouped GEMMs) and returns LATENT_E_WORKSPACE otherwise.
+ */
 int latent_moe_workspace_size(const latent_moe_args* args, size_t* bytes);
 
 /*
@@ -160,8 +164,8 @@ int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream_t stream);
  * harnesses that forbid hipMalloc).  No counterpart in the reference.
  * args->workspace and args->workspace_bytes are ignored: scratch comes from a
  * library-owned array of LATENT_NOALLOC_SCRATCH_BYTES on each GPU (held until
- * the process ends); a call whose latent_moe_workspace_size exceeds that
- * returns LATENT_E_WORKSPACE.  No call allocates.  Every call on one GPU
+ * the process ends); a call that cannot run in that many bytes returns
+ * LATENT_E_WORKSPACE.  No call allocates.  Every call on one GPU
  * shares that GPU's array: calls that overlap on one GPU (other streams,
  * other host threads) race; calls in order on one stream do not.
  */
@@ -220,7 +224,8 @@ int latent_moe_check(void* workspace, size_t workspace_bytes, latent_stream_t st
  *       it streams 64-pair units of one expert, on the row layout (n_embd /
  *       n_ff / max_rank multiples of 128, n_ff and max_rank <= 2048, 16-byte
  *       aligned codes) it runs grouped GEMMs, or the kernels of path 4 where
- *       the GEMMs' 128-pair tiles would not fill the chip;
+ *       the GEMMs' 128-pair tiles would not fill the chip and the workspace
+ *       holds their sums; on the row layout bit-reproducible;
  *   3 = streaming fp16-MFMA decode: the factors are in the tile layout, 1 to
  *       4096 routed pairs, 16-byte aligned x;
  *   4 = multi-kernel fp16-MFMA path on the row layout, taken here when a

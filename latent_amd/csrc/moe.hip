@@ -905,6 +905,7 @@ constexpr size_t kOwn = LATENT_NOALLOC_SCRATCH_BYTES - LATENT_NOALLOC_CONTROL_BY
 
 struct Layout {
   size_t meta, act_expert, act_start, act_count, pair_tok, pair_slot, pair_w, hist, units, gu, dl, xh, xexp, pos_of, y, total;
+  bool ordered;  // y holds an ordered row-layout call's planes, then its y rows
 };
 
 // Pairs per chunk of the multi-workgroup grouping: multiples of the block
@@ -923,9 +924,45 @@ int64_t xh_cols(const latent_moe_args& a) {
   return a.layout == LATENT_LAYOUT_ROWS && a.max_rank <= 512 ? a.n_embd : 0;
 }
 
-Layout layout_for(int64_t T, int64_t K, int64_t E, int64_t R, int64_t d, bool roomy) {
+// The shape and work split of a row-layout MFMA call.
+rows::Params rows_shape(const latent_moe_args& a, bool int8, bool ordered) {
+  rows::Params r{};
+  r.T = static_cast<int>(a.n_tokens);
+  r.d = static_cast<int>(a.n_embd);
+  r.ff = static_cast<int>(a.n_ff);
+  r.E = static_cast<int>(a.n_expert);
+  r.K = static_cast<int>(a.n_expert_used);
+  r.R = static_cast<int>(a.max_rank);
+  r.out_mode = a.out_mode;
+  r.a_max = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(a.n_expert, a.n_tokens * a.n_expert_used)));
+  r.ordered = ordered ? 1 : 0;
+  rows::plan(r, int8);
+  return r;
+}
+
+// Whether a prefill call on the row layout is one for the row-layout MFMA phases
+// rather than the grouped GEMMs.  The GEMMs' 128-pair tiles need a tile on every
+// CU, and what the phases save there (the factors in fp16) is less the more
+// pairs share a factor and the higher its rank (us, phases / GEMMs):
+//   E 64, d 2048, ff 1408, rank 128, top-6: 200 tokens 70 / 220, 1999 (125
+//     tiles) 208 / 295, 4000 (219) 372 / 372
+//   E 16, d 4096, ff 2048, rank 128, top-4: 500 tokens 104 / 390, 5000 490 / 546
+//   E 256, d 7168, ff 2048, rank 256, top-8: 512 tokens 417 / 832, 1280 (208
+//     tiles) 722 / 899
+//   E 64, d 4096, ff 2048, top-8: rank 256 400 tokens 231 / 435, 2000 (pairs x
+//     rank 4.1 M) 700 / 622; rank 384 400 tokens 292 / 385, 1000 (3.1 M) 558 /
+//     502; rank 512 400 tokens 377 / 418, 1000 (4.1 M) 652 / 543
+bool few_tiles(const latent_moe_args& a) {
+  const int64_t P = a.n_tokens * a.n_expert_used;
+  return a.layout == LATENT_LAYOUT_ROWS && rows::supported(a) && prefill::supported(a) &&
+         P / 128 + std::min(a.n_expert, P) / 2 < 212 && P * a.max_rank < 2800000;
+}
+
+// extra: with what a call can do without (see moe_workspace_bytes).
+Layout layout_for(const latent_moe_args& a, bool extra) {
   Layout L{};
-  const int64_t P = T * K;
+  const int64_t T = a.n_tokens, E = a.n_expert, R = a.max_rank, P = T * a.n_expert_used;
+  const int64_t d = xh_cols(a);
   const int64_t amax = std::max<int64_t>(1, std::min(E, P));
   size_t off = 0;
   L.meta = off;       off = align_up(off + 64 * sizeof(int));
@@ -942,23 +979,26 @@ Layout layout_for(int64_t T, int64_t K, int64_t E, int64_t R, int64_t d, bool ro
   // x as fp16 rows x 2^xexp for the row-layout MFMA phases (d = 0: none).
   L.xh = off;         off = align_up(off + T * d * 2);
   L.xexp = off;       off = align_up(off + T * sizeof(int));
-  // Their y rows, summed per token at the end, from 2048 pairs (25 M fp32
-  // atomics into out took 75 us of a call's 113 in phase D); not where they
-  // alone (another path of the call needing no more: not roomy) would take it
-  // past the library's own scratch array.
   L.pos_of = L.y = 0;
-  const size_t with_y = align_up(off + P * sizeof(int)) + align_up(static_cast<size_t>(P) * d * sizeof(float));
-  if (d > 0 && P >= 2048 && (with_y <= kOwn || off > kOwn || roomy)) {
+  auto place_y = [&](size_t bytes) {
     L.pos_of = off;   off = align_up(off + P * sizeof(int));
-    L.y = off;        off = align_up(off + static_cast<size_t>(P) * d * sizeof(float));
+    L.y = off;        off = align_up(off + bytes);
+  };
+  if (few_tiles(a)) {
+    if (extra) {
+      L.ordered = true;
+      place_y(rows::sums_bytes(rows_shape(a, false, true)));
+    }
+  } else if (d > 0 && P >= 2048) {
+    // y rows, summed per token at the end, from 2048 pairs (25 M fp32 atomics
+    // into out took 75 us of a call's 113 in phase D); not where they alone
+    // would take the call past the library's own scratch array.
+    const size_t bytes = static_cast<size_t>(P) * d * sizeof(float);
+    const bool roomy = a.layout == LATENT_LAYOUT_ROWS && prefill::supported(a) && prefill::layout_for(a).total > kOwn;
+    if (align_up(off + P * sizeof(int)) + align_up(bytes) <= kOwn || off > kOwn || roomy) place_y(bytes);
   }
   L.total = off;
   return L;
-}
-
-Layout layout_for(const latent_moe_args& a) {
-  const bool roomy = a.layout == LATENT_LAYOUT_ROWS && prefill::supported(a) && prefill::layout_for(a).total > kOwn;
-  return layout_for(a.n_tokens, a.n_expert_used, a.n_expert, a.max_rank, xh_cols(a), roomy);
 }
 
 int validate(const latent_moe_args& a) {
@@ -1040,20 +1080,6 @@ int choose_path(const latent_moe_args& a) {
   return kPathGeneral;
 }
 
-// Whether a prefill call on the row layout takes the row-layout MFMA phases
-// rather than the grouped GEMMs, whose 128-pair tiles need a tile on every CU
-// (us, phases / GEMMs): E 64, d 2048, ff 1408, rank 128, top-6: 200 tokens 89
-// / 221, 1999 tokens (128 tiles) 217 / 291; E 16, d 4096, ff 2048, rank 128:
-// 2000 tokens 236 / 424; DeepSeek-V3 shape: 512 tokens 481 / 866, 1280 (208
-// tiles) 822 / 875, 1536 (224) 1,010 / 897, 4096 (384) 2,186 / 1,510.
-// LATENT_MOE_PATH=prefill keeps the GEMMs.
-bool rows_prefill(const latent_moe_args& a) {
-  if (a.layout != LATENT_LAYOUT_ROWS || !rows::supported(a)) return false;
-  const char* env = std::getenv("LATENT_MOE_PATH");
-  if (env && !std::strcmp(env, "prefill")) return false;
-  return a.n_tokens * a.n_expert_used / 128 + std::min(a.n_expert, a.n_tokens * a.n_expert_used) / 2 < 212;
-}
-
 template <int MB, bool kInt8>
 int launch_phases(const MoeParams& p, hipStream_t s) {
   const unsigned a_groups = static_cast<unsigned>((p.a_max + 7) / 8);
@@ -1122,17 +1148,26 @@ extern "C" const char* latent_status_string(int status) {
   }
 }
 
-// Workspace: [fused control block, zero between calls][scratch shared by both paths]
+namespace latent {
+// Workspace bytes of a valid call: control block (zero between calls), scratch
+// the paths share, INT8 word offsets.  extra: with the planes of row-layout
+// prefill in place of its GEMMs; a call given less runs the GEMMs.
+size_t moe_workspace_bytes(const latent_moe_args& a, bool extra) {
+  const Layout L = layout_for(a, extra);
+  size_t scratch = L.total;
+  if (prefill::supported(a)) scratch = std::max(scratch, L.gu + prefill::layout_for(a).total);
+  if (chain32::supported(a)) scratch = std::max(scratch, L.gu + chain32::layout_for(a).total);
+  if (stream::supported(a)) scratch = std::max(scratch, L.gu + stream::layout_for(a).total);
+  return kControlBytes + align_up(scratch) + int8_word_offset_bytes(a);
+}
+int moe_validate(const latent_moe_args& a) { return validate(a); }
+}  // namespace latent
+
 extern "C" int latent_moe_workspace_size(const latent_moe_args* args, size_t* bytes) {
   if (!args || !bytes) return LATENT_E_INVALID;
   const int st = validate(*args);
   if (st != LATENT_OK) return st;
-  const Layout L = layout_for(*args);
-  size_t scratch = L.total;
-  if (prefill::supported(*args)) scratch = std::max(scratch, L.gu + prefill::layout_for(*args).total);
-  if (chain32::supported(*args)) scratch = std::max(scratch, L.gu + chain32::layout_for(*args).total);
-  if (stream::supported(*args)) scratch = std::max(scratch, L.gu + stream::layout_for(*args).total);
-  *bytes = kControlBytes + align_up(scratch) + int8_word_offset_bytes(*args);
+  *bytes = moe_workspace_bytes(*args, true);
   return LATENT_OK;
 }
 
@@ -1199,8 +1234,9 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
   if (a.n_tokens == 0) return LATENT_OK;
   if (!a.x || !a.ids || !a.weights || !a.out) return LATENT_E_INVALID;
   if ((reinterpret_cast<uintptr_t>(a.out) & 15u) != 0) return LATENT_E_INVALID;
-  size_t need = 0;
-  latent_moe_workspace_size(&a, &need);
+  size_t need = moe_workspace_bytes(a, true);
+  const bool extra = a.workspace_bytes >= need;
+  if (!extra) need = moe_workspace_bytes(a, false);
   if (!a.workspace || a.workspace_bytes < need) return LATENT_E_WORKSPACE;
   if ((reinterpret_cast<uintptr_t>(a.workspace) & (kAlign - 1)) != 0) return LATENT_E_WORKSPACE;
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
@@ -1215,13 +1251,10 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
     any_int8 = any_int8 || fs[i]->int8_bitmap != nullptr;
   }
   if (any_int8) {
-    // The tail of the workspace (after the largest path's scratch).
-    size_t total = 0;
-    latent_moe_workspace_size(&a, &total);
-    char* tail = static_cast<char*>(a.workspace) + total - int8_word_offset_bytes(a);
-    set_int8_word_offsets(a, tail, p);
+    // The workspace's tail, after the largest path's scratch.
+    set_int8_word_offsets(a, static_cast<char*>(a.workspace) + need - int8_word_offset_bytes(a), p);
   }
-  const Layout L = layout_for(a);
+  const Layout L = layout_for(a, extra);
   char* ws = static_cast<char*>(a.workspace) + kControlBytes;
   p.x = a.x;
   p.ids = a.ids;
@@ -1249,7 +1282,8 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
   p.out_mode = a.out_mode;
   const int64_t P = a.n_tokens * a.n_expert_used;
   p.a_max = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(a.n_expert, P)));
-  const bool use_prefill = path == kPathPrefill && !rows_prefill(a);
+  const char* env = std::getenv("LATENT_MOE_PATH");  // "prefill" keeps the GEMMs
+  const bool use_prefill = path == kPathPrefill && !(L.ordered && !(env && !std::strcmp(env, "prefill")));
   const bool use_stream = path == kPathStream;
   if (use_stream && stream::lite_applies(a)) {
     static_assert(stream::kLiteCtrlOffset + stream::kLiteCtrlBytes <= kControlBytes, "control block");
@@ -1285,11 +1319,13 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
     p.xexp = reinterpret_cast<int*>(ws + L.xexp);
     p.longest_first = 1;
   }
+  const bool ordered = use_rows && L.ordered;
   const bool y_rows = use_rows && L.y != 0 && a.out_mode == LATENT_OUT_REDUCED;
   if (y_rows) p.pos_of = reinterpret_cast<int*>(ws + L.pos_of);
   // The MFMA paths write their intermediates whole, and every output row
-  // (per-token combine); the row-layout MFMA phases accumulate like the fp32 ones.
-  p.zero_floats = use_prefill || use_stream ? 0 : P * 3 * a.max_rank;
+  // (per-token combine), and so do ordered row-layout calls; the others of the
+  // row-layout MFMA phases accumulate like the fp32 ones.
+  p.zero_floats = use_prefill || use_stream || ordered ? 0 : P * 3 * a.max_rank;
   p.zero_out = use_prefill || use_stream || y_rows ? 0 : 1;
   p.clear = use_stream ? 0 : 1;
 
@@ -1337,7 +1373,7 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
     return stream::forward(a, g, ws + L.gu, s);
   }
   if (use_rows) {
-    rows::Params rp{};
+    rows::Params rp = rows_shape(a, any_int8, ordered);
     for (int i = 0; i < 6; ++i) rp.fac[i] = p.fac[i];
     rp.ranks = p.ranks;
     rp.meta = p.meta;
@@ -1352,21 +1388,13 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
     rp.gu = p.gu;
     rp.dl = p.dl;
     rp.out = p.out;
+    rp.sums = reinterpret_cast<float*>(ws + L.y);
     rp.y = y_rows ? reinterpret_cast<float*>(ws + L.y) : nullptr;
     rp.pos_of = p.pos_of;
     rp.ids = p.ids;
     rp.weights = p.weights;
     rp.w_dtype = p.w_dtype;
-    rp.E = p.E;
-    rp.T = p.T;
-    rp.d = p.d;
-    rp.ff = p.ff;
-    rp.K = p.K;
-    rp.R = p.R;
     rp.wbd = p.wbd;
-    rp.out_mode = p.out_mode;
-    rp.a_max = p.a_max;
-    rows::plan(rp, any_int8);
     return rows::launch(rp, any_int8, s);
   }
   if (MB == 1)

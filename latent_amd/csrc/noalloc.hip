@@ -17,6 +17,11 @@
 #include <mutex>
 
 namespace latent {
+
+// moe.hip
+int moe_validate(const latent_moe_args& a);
+size_t moe_workspace_bytes(const latent_moe_args& a, bool extra);
+
 namespace {
 
 static_assert(LATENT_NOALLOC_CONTROL_BYTES == kControlBytes, "control block size");
@@ -64,10 +69,9 @@ extern "C" int latent_moe_ffn_forward_noalloc(const latent_moe_args* args, laten
   latent_moe_args a = *args;
   a.workspace = nullptr;
   a.workspace_bytes = 0;
-  size_t need = 0;
-  const int st = latent_moe_workspace_size(&a, &need);
+  const int st = latent::moe_validate(a);
   if (st != LATENT_OK) return st;
-  if (need > LATENT_NOALLOC_SCRATCH_BYTES) return LATENT_E_WORKSPACE;
+  if (latent::moe_workspace_bytes(a, false) > LATENT_NOALLOC_SCRATCH_BYTES) return LATENT_E_WORKSPACE;
   if (a.n_tokens == 0) return LATENT_OK;
   void* p = nullptr;
   const int sp = latent::noalloc_scratch(reinterpret_cast<hipStream_t>(stream), &p);

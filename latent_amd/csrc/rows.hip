@@ -37,6 +37,11 @@
 // multi-kernel path with atomics (gu, dl; out for the reduced output), which
 // its prep kernel zeroes.  A pass takes MB blocks of 16 pairs of one expert;
 // an expert with more pairs takes several passes.
+//
+// Ordered calls (row-layout prefill) repeat bit for bit: a range of d (phase
+// A) or of ff (BC) stores its sums to a plane of its own, sum_planes_kernel
+// adds the planes in order, and the reduced output comes from y rows.  E 64, d
+// 2048, ff 1408, rank 128, 1999 tokens: 226 us with atomics, 224 so.
 #include "common.hpp"
 #include "rowblock.hpp"
 #include "rows.hpp"
@@ -329,12 +334,13 @@ __device__ __forceinline__ void store_tile(uint32_t at, const float4v (&acc)[CPL
                       float4v{acc[c][v], acc[c + 1][v], acc[c + 2][v], acc[c + 3][v]});
 }
 // Products of 32 nblk rows (from row0 of the factor) with `cols` columns for
-// m pairs, times 2^-exp of their rows, added to dst[row][0 .. cols) (rows
-// `stride` floats apart).  The waves share K where the columns are fewer than
-// four tiles.  ready(): the level table and the activations are in LDS (the
-// first factor loads are issued before it).  red: LDS address of kRedBytes the
-// table, the meta slots and the activations may overlap.
-template <int MB, bool kInt8, class Act, typename Ready>
+// m pairs, times 2^-exp of their rows, added to (kStore: stored to)
+// dst[row][0 .. cols) (rows `stride` floats apart).  The waves share K where
+// the columns are fewer than four tiles.  ready(): the level table and the
+// activations are in LDS (the first factor loads are issued before it).  red:
+// LDS address of kRedBytes the table, the meta slots and the activations may
+// overlap.
+template <int MB, bool kInt8, bool kStore, class Act, typename Ready>
 __device__ __forceinline__ void rank_gemm(const Factor& f, int e, int row0, int nblk, int cols, int m, uint32_t lut,
                                           uint32_t meta, uint32_t red, const int* rexp, const Act& act, Ready&& ready,
                                           float* dst, int stride) {
@@ -356,13 +362,28 @@ __device__ __forceinline__ void rank_gemm(const Factor& f, int e, int row0, int 
       if ((kq >> 1) == (half & 1)) store_tile(at, acc[half >> 1]);
       lds_barrier();
       const int rows = min(8, m - half * 8);
-      for (int i = tid; i < rows * cols; i += kT) {
-        const int r = i / cols, c = i - r * cols, t = c / (16 * CPL);
-        const uint32_t src = red + t * kHalfSlot + static_cast<uint32_t>(r * kTileStr + c - t * 16 * CPL) * 4u;
-        float s = lds_ld<float>(src);
+      if constexpr (kStore) {
+        for (int i = tid; i < rows * cols / 4; i += kT) {
+          const int r = i * 4 / cols, c = i * 4 - r * cols, t = c / (16 * CPL);
+          const uint32_t src = red + t * kHalfSlot + static_cast<uint32_t>(r * kTileStr + c - t * 16 * CPL) * 4u;
+          float* to = dst + static_cast<int64_t>(half * 8 + r) * stride + c;
+          const int ex = -rexp[half * 8 + r];
+          float4v s = lds_ld<float4v>(src);
 #pragma unroll
-        for (int k = 1; k < KP; ++k) s += lds_ld<float>(src + k * NT * kHalfSlot);
-        atomic_add_f32(dst + static_cast<int64_t>(half * 8 + r) * stride + c, ldexpf(s, -rexp[half * 8 + r]));
+          for (int k = 1; k < KP; ++k) s += lds_ld<float4v>(src + k * NT * kHalfSlot);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) s[q] = ldexpf(s[q], ex);
+          *reinterpret_cast<float4v*>(to) = s;
+        }
+      } else {
+        for (int i = tid; i < rows * cols; i += kT) {
+          const int r = i / cols, c = i - r * cols, t = c / (16 * CPL);
+          const uint32_t src = red + t * kHalfSlot + static_cast<uint32_t>(r * kTileStr + c - t * 16 * CPL) * 4u;
+          float s = lds_ld<float>(src);
+#pragma unroll
+          for (int k = 1; k < KP; ++k) s += lds_ld<float>(src + k * NT * kHalfSlot);
+          atomic_add_f32(dst + static_cast<int64_t>(half * 8 + r) * stride + c, ldexpf(s, -rexp[half * 8 + r]));
+        }
       }
     }
   });
@@ -436,7 +457,7 @@ constexpr int waves_for(int mb) { return mb == 1 ? 3 : 2; }
 // ---------------------------------------------------------------------------
 // Phase A: x . A_g, x . A_u over a range of d rows
 // ---------------------------------------------------------------------------
-template <int MB, bool kInt8>
+template <int MB, bool kInt8, bool kOrdered>
 __global__ void __launch_bounds__(kT, waves_for(MB)) a_kernel(Params p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ int rexp[16 * MB];
@@ -448,13 +469,15 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) a_kernel(Params p) {
   const int kind = item & 1, split = item >> 1;
   const int e = p.act_expert[a], s0 = p.act_start[a], mtot = p.act_count[a];
   const int cols = (rank_of(p, e, kind) + kGroup - 1) / kGroup * kGroup;
-  // Ranges of d in proportion to the expert's rank, so that items are alike.
-  const int pieces = (p.na_split * max(cols, 128) + p.R - 1) / max(p.R, 128), nblk = p.d / 32;
+  // Ranges of d in proportion to the expert's rank, so that items are alike;
+  // every plane of an ordered call is written.
+  const int pieces = kOrdered ? p.na_split : (p.na_split * max(cols, 128) + p.R - 1) / max(p.R, 128), nblk = p.d / 32;
   if (split >= pieces) return;
   const int blk0 = split * nblk / pieces, blk1 = (split + 1) * nblk / pieces;
   if (blk0 == blk1) return;
   const uint32_t lut0 = lds_addr(smem), lut = lut0 + (lane & (kCopies - 1)) * 4;
   const uint32_t meta = lut0 + kLutBytes + uniform(tid >> 6) * kMetaBytes;
+  float* gu = kOrdered && p.na_split > 1 ? p.sums + static_cast<int64_t>(split) * p.T * p.K * (2 * p.R) : p.gu;
   for (int tb = 16 * MB * pass; tb < mtot; tb += 16 * MB * p.n_pass) {
     const int m = min(16 * MB, mtot - tb);
     ActX<MB> act;
@@ -468,8 +491,8 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) a_kernel(Params p) {
       lut_fill(lut0, tid);  // the sums take the table's place
       lds_barrier();
     };
-    rank_gemm<MB, kInt8>(p.fac[kind ? F_UP_A : F_GATE_A], e, 32 * blk0, blk1 - blk0, cols, m, lut, meta, lut0, rexp,
-                         act, ready, p.gu + static_cast<int64_t>(s0 + tb) * (2 * p.R) + kind * p.R, 2 * p.R);
+    rank_gemm<MB, kInt8, kOrdered>(p.fac[kind ? F_UP_A : F_GATE_A], e, 32 * blk0, blk1 - blk0, cols, m, lut, meta, lut0,
+                                   rexp, act, ready, gu + static_cast<int64_t>(s0 + tb) * (2 * p.R) + kind * p.R, 2 * p.R);
     lds_barrier();  // the sums and exponents are read
   }
 }
@@ -478,7 +501,7 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) a_kernel(Params p) {
 // Phase BC: g . B_g and u . B_u over 256 columns of ff, h = SiLU(g) u in
 // LDS, then h . A_d (those 256 rows of A_d)
 // ---------------------------------------------------------------------------
-template <int MB, bool kInt8>
+template <int MB, bool kInt8, bool kOrdered>
 __global__ void __launch_bounds__(kT, waves_for(MB)) bc_kernel(Params p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ int rexp[2][16 * MB], hexp[16 * MB];
@@ -502,6 +525,7 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) bc_kernel(Params p) {
   const int kind = wave & 1, tile = wave >> 1;
   const int nb = tile * 128 < ncol ? ((kind ? ru : rg) + 31) / 32 : 0;
   const int cols = (rd + kGroup - 1) / kGroup * kGroup;
+  float* dl = kOrdered && p.n_bc > 1 ? p.sums + static_cast<int64_t>(item) * p.T * p.K * p.R : p.dl;
   for (int tb = 16 * MB * pass; tb < mtot; tb += 16 * MB * p.n_pass) {
     const int m = min(16 * MB, mtot - tb);
     Walk<8, MB, kInt8, ActLds> walk(
@@ -551,9 +575,9 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) bc_kernel(Params p) {
       }
     }
     if (cols != 0)
-      rank_gemm<MB, kInt8>(p.fac[F_DOWN_A], e, c0, ncol / 32, cols, m, lut, meta, L_red, hexp,
-                           ActLds{L_h + static_cast<uint32_t>(n * kHStr + 8 * kq) * 2u, 16u * kHStr * 2},
-                           [] { lds_barrier(); }, p.dl + static_cast<int64_t>(s0 + tb) * p.R, p.R);
+      rank_gemm<MB, kInt8, kOrdered>(p.fac[F_DOWN_A], e, c0, ncol / 32, cols, m, lut, meta, L_red, hexp,
+                                     ActLds{L_h + static_cast<uint32_t>(n * kHStr + 8 * kq) * 2u, 16u * kHStr * 2},
+                                     [] { lds_barrier(); }, dl + static_cast<int64_t>(s0 + tb) * p.R, p.R);
     lds_barrier();
   }
 }
@@ -640,6 +664,19 @@ __global__ void __launch_bounds__(kT, waves_for(MB)) d_kernel(Params p) {
   }
 }
 
+// dst = the planes' sum, in plane order; one float4 per thread.  Columns past an
+// expert's rank and rows past the routed pairs were never written: no one
+// reads their sums.
+__global__ void __launch_bounds__(kT) sum_planes_kernel(const float* planes, int n, int64_t n4, float* dst) {
+  const int64_t i = blockIdx.x * static_cast<int64_t>(kT) + threadIdx.x;
+  if (i >= n4) return;
+  const float4v* src = reinterpret_cast<const float4v*>(planes) + i;
+  float4v s = src[0];
+#pragma unroll 8
+  for (int k = 1; k < n; ++k) s += src[k * n4];
+  reinterpret_cast<float4v*>(dst)[i] = s;
+}
+
 // Reduced output from y rows: the weighted sum over a token's slots in slot
 // order, one float4 per thread.
 __global__ void __launch_bounds__(kT) combine_kernel(Params p) {
@@ -667,11 +704,20 @@ size_t lds_d(int R) {
   return static_cast<size_t>(kFixBytes + std::max(16 * MB * (R + 8) * 2, kRedBytes));
 }
 
-template <int MB, bool kInt8>
+template <int MB, bool kInt8, bool kOrdered = false>
 int launch_phases(const Params& p, hipStream_t s) {
   const unsigned groups = static_cast<unsigned>((p.a_max + 7) / 8 * p.n_pass);
-  hipLaunchKernelGGL((a_kernel<MB, kInt8>), dim3(8 * groups * p.n_a), dim3(kT), lds_a(), s, p);
-  hipLaunchKernelGGL((bc_kernel<MB, kInt8>), dim3(8 * groups * p.n_bc), dim3(kT), lds_bc<MB>(p.R), s, p);
+  const int64_t P = static_cast<int64_t>(p.T) * p.K;
+  auto sum_planes = [&](int n, int64_t width, float* dst) {
+    if (!kOrdered || n == 1) return;
+    const int64_t n4 = P * width / 4;
+    hipLaunchKernelGGL(sum_planes_kernel, dim3(static_cast<unsigned>((n4 + kT - 1) / kT)), dim3(kT), 0, s, p.sums, n, n4,
+                       dst);
+  };
+  hipLaunchKernelGGL((a_kernel<MB, kInt8, kOrdered>), dim3(8 * groups * p.n_a), dim3(kT), lds_a(), s, p);
+  sum_planes(p.na_split, 2 * p.R, p.gu);
+  hipLaunchKernelGGL((bc_kernel<MB, kInt8, kOrdered>), dim3(8 * groups * p.n_bc), dim3(kT), lds_bc<MB>(p.R), s, p);
+  sum_planes(p.n_bc, p.R, p.dl);
   if (!p.y && p.out_mode == LATENT_OUT_REDUCED)
     hipLaunchKernelGGL((d_kernel<MB, kInt8, true>), dim3(8 * groups * p.n_d), dim3(kT), lds_d<MB>(p.R), s, p);
   else
@@ -715,15 +761,28 @@ void plan(Params& p, bool int8) {
   // Phase A ranges per expert and factor at the full rank (a smaller rank has
   // fewer): about 4096 items in all, of eight blocks of 32 rows or more; with
   // 64 pairs a pass the items are eight times as long, and their sums cost as
-  // many atomics per range.
-  const int64_t want = step == 64 ? 512 : 4096;
-  int s = step == 64 ? 1 : 4;
-  while (s < 32 && 2ll * p.a_max * p.n_pass * s < want && p.d / 32 >= 16 * s) s *= 2;
+  // many atomics per range.  Ordered calls, one plane per range: some 512 items
+  // and at most four ranges (E 256, d 7168, rank 256, 512 tokens: 417 us at one,
+  // 433 at four; E 64, d 4096, rank 256, 150 tokens 121 and 98).
+  const bool few = step == 64 || p.ordered;
+  const int64_t want = few ? 512 : 4096;
+  int s = few ? 1 : 4;
+  while (s < (p.ordered ? 4 : 32) && 2ll * p.a_max * p.n_pass * s < want && p.d / 32 >= 16 * s) s *= 2;
   p.na_split = s;
   p.n_a = 2 * s;
 }
 
+size_t sums_bytes(const Params& p) {
+  const size_t P = static_cast<size_t>(p.T) * p.K;
+  size_t n = p.out_mode == LATENT_OUT_REDUCED ? P * p.d : 0;
+  if (p.na_split > 1) n = std::max(n, P * 2 * p.R * p.na_split);
+  if (p.n_bc > 1) n = std::max(n, P * p.R * p.n_bc);
+  return n * sizeof(float);
+}
+
 int launch(const Params& p, bool int8, hipStream_t s) {
+  if (p.ordered)  // at least 16 pairs an expert, no INT8 groups
+    return pair_blocks(p, false) == 4 ? launch_phases<4, false, true>(p, s) : launch_phases<2, false, true>(p, s);
   if (int8) return launch_phases<1, true>(p, s);
   switch (pair_blocks(p, false)) {
     case 4: return launch_phases<4, false>(p, s);

@@ -1,6 +1,7 @@
 // Host interface of the MFMA phases over the row layout (rows.hip).
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 #include <hip/hip_runtime.h>
@@ -38,6 +39,8 @@ struct Params {
   int na_split;  // phase A: K ranges per factor
   int n_a, n_bc, n_d;  // items per active expert
   int n_pass;          // workgroups that share an item's passes
+  int ordered;  // sums in a fixed order through the planes of `sums`
+  float* sums;  // sums_bytes() of them; y takes their place
 };
 
 // The row-layout shapes the kernels take (d, ff multiples of 32, max_rank at
@@ -45,6 +48,9 @@ struct Params {
 bool supported(const latent_moe_args& a);
 // Sets the work split (na_split, n_a, n_bc, n_d, n_pass) of p from its shape.
 void plan(Params& p, bool int8);
+// Bytes of an ordered call's planes and y rows (p planned).  Ordered calls have
+// 16 pairs or more per expert and no INT8 groups.
+size_t sums_bytes(const Params& p);
 int launch(const Params& p, bool int8, hipStream_t s);
 
 }  // namespace rows

@@ -183,3 +183,61 @@ def test_rows_large_batches(gpu, monkeypatch, T, E, d, ff, R, mode):
         monkeypatch.setenv("LATENT_MOE_PATH", "prefill")
         gemm = gpu.moe_forward(x, it, wt, dev, out_mode=mode).cpu().numpy()
         assert ref.rel_l2(gemm, got) <= TOL
+
+
+@pytest.mark.parametrize("T,E,d,ff,R,k,mode", [
+    (300, 12, 256, 640, 128, 2, 0),    # four pair blocks, three planes of down latents, one of gate and up
+    (130, 16, 1024, 256, 256, 2, 0),   # two pair blocks, four planes of gate and up, one of down latents
+    (130, 16, 1024, 896, 384, 2, 1),   # the same with planes of both, per-slot output
+    (2100, 7, 640, 512, 512, 2, 0),    # several workgroups group 4200 pairs
+])
+def test_row_layout_prefill_repeats_bit_for_bit(gpu, monkeypatch, T, E, d, ff, R, k, mode):
+    """Row-layout prefill in these kernels: every sum has a fixed order, so calls
+    repeat their bits (their latents used to meet in atomics), also on a
+    workspace that another call left full of its own sums."""
+    import torch
+
+    monkeypatch.delenv("LATENT_MOE_PATH")
+    ranks = [max(1, R - 37 * (i % 5)) for i in range(E)]
+    host = synth.make_layer(seed=R, n_expert=E, d=d, ff=ff, max_rank=R, ranks=ranks)
+    dev = _rows_layer(host)
+    rng = np.random.default_rng(T + R)
+    x = torch.from_numpy(rng.standard_normal((T, d)).astype(np.float32)).cuda()
+    ids, w = routing.softmax_topk(rng.standard_normal((T, E)) + np.linspace(1.5, 0, E), k)
+    ids[rng.random(ids.shape) < 0.03] = -1
+    it, wt = torch.from_numpy(ids.astype(np.int32)).cuda(), torch.from_numpy(w.astype(np.float32)).cuda()
+    assert gpu.moe_path(dev, x, k) == "prefill"
+    got = gpu.moe_forward(x, it, wt, dev, out_mode=mode)
+    for _ in range(4):
+        gpu.moe_forward(x.flip(0), it, wt, dev, out_mode=mode)
+        assert torch.equal(got, gpu.moe_forward(x, it, wt, dev, out_mode=mode))
+    pick = np.array(sorted(set(range(0, T, T // 30)) | {T - 1}))
+    want = ref.moe_forward(x.cpu().numpy()[pick], ids[pick], w[pick], host, out_mode=mode)
+    assert ref.rel_l2(want, got.cpu().numpy()[pick]) <= TOL
+
+
+def test_row_layout_prefill_in_less_workspace(gpu, monkeypatch):
+    """Given less than the queried size, row-layout prefill runs the GEMMs, whose
+    need is that of a call in which they were chosen."""
+    import torch
+
+    from latent_amd._lib import LatentError
+
+    monkeypatch.delenv("LATENT_MOE_PATH")
+    host = synth.make_layer(seed=5, n_expert=8, d=512, ff=384, max_rank=128)
+    dev = _rows_layer(host)
+    rng = np.random.default_rng(8)
+    T, k = 400, 2
+    x = torch.from_numpy(rng.standard_normal((T, 512)).astype(np.float32)).cuda()
+    ids, w = routing.softmax_topk(rng.standard_normal((T, 8)), k)
+    it, wt = torch.from_numpy(ids.astype(np.int32)).cuda(), torch.from_numpy(w.astype(np.float32)).cuda()
+    full = gpu.workspace_size(dev, T, k)
+    ws = torch.zeros(full, dtype=torch.uint8, device="cuda")
+    phases = gpu.moe_forward(x, it, wt, dev, workspace=ws)
+    monkeypatch.setenv("LATENT_MOE_PATH", "prefill")
+    gemms = gpu.moe_forward(x, it, wt, dev, workspace=ws)
+    monkeypatch.delenv("LATENT_MOE_PATH")
+    assert not torch.equal(phases, gemms)
+    assert torch.equal(gemms, gpu.moe_forward(x, it, wt, dev, workspace=ws[:full - 256]))
+    with pytest.raises(LatentError):
+        gpu.moe_forward(x, it, wt, dev, workspace=ws[:full // 3])
