@@ -59,11 +59,14 @@ struct WordOffsets {
   int64_t rows;
   int words;
 };
+struct OffsetList {
+  int n;
+  WordOffsets f[6];
+};
+struct NoOffsets {};
 
 struct MoeParams {
   Factor fac[6];
-  WordOffsets off[6];
-  int n_off;
   const void* x;
   const int32_t* ids;
   const void* weights;
@@ -78,8 +81,8 @@ struct MoeParams {
   float* pair_w;
   float* gu;  // [P][2R]
   float* dl;  // [P][R]
-  int4* unit_info;  // work units {expert, first pair, pairs, 0} (NULL: not built)
-  int unit_shift;   // a unit holds at most 1 << unit_shift pairs of one expert
+  int4* unit_info;  // work units {expert, first pair, pairs, 0}
+  int unit_shift;   // a unit holds at most 1 << unit_shift pairs of one expert (0: no units)
   int* unit_tok;    // [units][1 << unit_shift] token of each unit row (0 past the unit's pairs)
   int* pos_of;      // [T*K] grouped position of each routed slot (with units)
   _Float16* xh;     // streaming path: x as fp16 rows * 2^xexp (NULL: not converted)
@@ -124,30 +127,32 @@ constexpr int kCached = 4;  // pairs per thread held in registers by route_block
 constexpr int kOrderedExperts = 1024;  // route_block places pairs in index order up to this many experts
 
 // Place routed pair i (expert e, weight w) at the expert's next position and
-// in its streaming unit's row tables.  start[e] is the expert's first
+// in its unit's row tables (kShift > 0).  start[e] is the expert's first
 // position; fill[e] its running insert position.
+template <int kShift>
 __device__ __forceinline__ void place_pair(const MoeParams& p, const int* start, const int* ubase, int i, int e,
                                            float w, int pos) {
   const int tok = i / p.K, slot = i - tok * p.K;
   p.pair_tok[pos] = tok;
   p.pair_slot[pos] = slot;
   p.pair_w[pos] = w;
-  if (p.unit_info) {
+  if (kShift > 0) {
     const int rel = pos - start[e];
-    p.unit_tok[(ubase[e] << p.unit_shift) + rel] = tok;
+    p.unit_tok[(ubase[e] << kShift) + rel] = tok;
   }
-  if (p.pos_of) p.pos_of[i] = pos;
+  if (kShift > 0 || p.pos_of) p.pos_of[i] = pos;
 }
 
 // Same, at the expert's next free position (the order among one expert's
 // pairs then depends on timing).
+template <int kShift>
 __device__ __forceinline__ void scatter_pair(const MoeParams& p, const int* start, int* fill, const int* ubase, int i,
                                              int e, float w) {
   if (e < 0 || e >= p.E) return;
-  place_pair(p, start, ubase, i, e, w, atomicAdd(&fill[e], 1));
+  place_pair<kShift>(p, start, ubase, i, e, w, atomicAdd(&fill[e], 1));
 }
 
-template <bool kRows>
+template <bool kRows, int kShift>
 __device__ void route_block(const MoeParams& p) {
   __shared__ int cnt[kMaxExperts];  // pairs per expert, then the expert's first position
   __shared__ int fill[kMaxExperts];
@@ -192,12 +197,12 @@ __device__ void route_block(const MoeParams& p) {
   // Block scan over experts: each thread owns a contiguous run of experts.
   const int per = (p.E + kRouteThreads - 1) / kRouteThreads;
   const int e0 = min(p.E, tid * per), e1 = min(p.E, e0 + per);
-  const int um = 1 << p.unit_shift;
+  constexpr int um = 1 << kShift;
   int sc = 0, sa = 0, su = 0;
   for (int e = e0; e < e1; ++e) {
     sc += cnt[e];
     sa += cnt[e] > 0;
-    su += (cnt[e] + um - 1) >> p.unit_shift;
+    su += (cnt[e] + um - 1) >> kShift;
   }
   // Inclusive scan: within the wave by shuffles, then across the waves'
   // totals.
@@ -252,7 +257,7 @@ __device__ void route_block(const MoeParams& p) {
       p.act_expert[act] = e;
       p.act_start[act] = start;
       p.act_count[act] = c;
-      if (p.unit_info) {  // units of one expert; rows past the pairs are padding
+      if (kShift > 0) {  // units of one expert; rows past the pairs are padding
         for (int j = 0; j < c; j += um, ++unit) {
           const int m = min(um, c - j);
           p.unit_info[unit] = make_int4(e, start + j, m, 0);
@@ -282,6 +287,21 @@ __device__ void route_block(const MoeParams& p) {
     uint32_t* mask = ordered_counts;  // [E][stride]
     // No more words than the call has pairs for (64 pairs: 2 of them to clear).
     const int words = min(p.E <= kOrderedExperts / 2 ? 32 : 16, (P + 31) / 32), stride = words | 1, round = 32 * words;
+    if (P <= round) {  // one round
+      for (int x = tid; x < p.E * stride; x += kRouteThreads) mask[x] = 0u;
+      __syncthreads();
+      const int e = my_e[0];
+      const bool ok = e >= 0 && e < p.E;
+      if (ok) atomicOr(&mask[e * stride + (tid >> 5)], 1u << (tid & 31));
+      __syncthreads();
+      if (ok) {
+        const uint32_t* m = mask + e * stride;
+        int pos = cnt[e] + __builtin_popcount(m[tid >> 5] & ((1u << (tid & 31)) - 1u));
+        for (int x = 0; x < (tid >> 5); ++x) pos += __builtin_popcount(m[x]);
+        place_pair<kShift>(p, cnt, ubase, tid, e, my_w[0], pos);
+      }
+      return;
+    }
     for (int base = 0, r = 0; base < P; base += round, ++r) {
       for (int x = tid; x < p.E * stride; x += kRouteThreads) mask[x] = 0u;
       const int i = base + tid;
@@ -312,7 +332,7 @@ __device__ void route_block(const MoeParams& p) {
         const uint32_t* m = mask + e * stride;
         int pos = fill[e] + __builtin_popcount(m[tid >> 5] & ((1u << (tid & 31)) - 1u));
         for (int x = 0; x < (tid >> 5); ++x) pos += __builtin_popcount(m[x]);
-        place_pair(p, cnt, ubase, i, e, w, pos);
+        place_pair<kShift>(p, cnt, ubase, i, e, w, pos);
       }
       if (base + round >= P) break;
       __syncthreads();
@@ -326,26 +346,28 @@ __device__ void route_block(const MoeParams& p) {
     return;
   }
 #pragma unroll
-  for (int j = 0; j < kCached; ++j) scatter_pair(p, cnt, fill, ubase, tid + j * kRouteThreads, my_e[j], my_w[j]);
+  for (int j = 0; j < kCached; ++j) scatter_pair<kShift>(p, cnt, fill, ubase, tid + j * kRouteThreads, my_e[j], my_w[j]);
   for (int i = tid + kCached * kRouteThreads; i < P; i += kRouteThreads) {
     const int e = p.ids[i];
-    if (e >= 0 && e < p.E) scatter_pair(p, cnt, fill, ubase, i, e, load_act(p.weights, p.w_dtype, i));
+    if (e >= 0 && e < p.E) scatter_pair<kShift>(p, cnt, fill, ubase, i, e, load_act(p.weights, p.w_dtype, i));
   }
 }
 
 // What the workgroups beside the grouping do: word offsets of INT8 factors, x
 // as fp16 rows, cleared accumulators.
-template <bool kRows>
-__device__ void prep_rest(const MoeParams& p, int64_t blk, int64_t nblk) {
+template <class Offsets>
+__device__ void prep_rest(const MoeParams& p, const Offsets& offsets, int64_t blk, int64_t nblk) {
   const int64_t t0 = blk * static_cast<int64_t>(kRouteThreads) + threadIdx.x;
   const int64_t stride = nblk * kRouteThreads;
-  for (int f = 0; kRows && f < p.n_off; ++f) {  // index of each bitmap word's first INT8 group
-    const WordOffsets& w = p.off[f];
-    for (int64_t r = t0; r < w.rows; r += stride) {
-      int run = w.row_offset[r];
-      for (int i = 0; i < w.words; ++i) {
-        w.out[r * w.words + i] = run;
-        run += popc(w.bitmap[r * w.words + i]);
+  if constexpr (std::is_same_v<Offsets, OffsetList>) {
+    for (int f = 0; f < offsets.n; ++f) {  // index of each bitmap word's first INT8 group
+      const WordOffsets& w = offsets.f[f];
+      for (int64_t r = t0; r < w.rows; r += stride) {
+        int run = w.row_offset[r];
+        for (int i = 0; i < w.words; ++i) {
+          w.out[r * w.words + i] = run;
+          run += popc(w.bitmap[r * w.words + i]);
+        }
       }
     }
   }
@@ -416,9 +438,10 @@ __device__ void prep_rest(const MoeParams& p, int64_t blk, int64_t nblk) {
 // its expert, so results do not depend on it.
 constexpr int kHistInts = 16384;  // (E + 1) * nchunk bound: the scan holds the histograms in LDS
 
-__global__ void __launch_bounds__(kRouteThreads) group_count_kernel(MoeParams p, int* hist, int chunk, int nchunk) {
+__global__ void __launch_bounds__(kRouteThreads) group_count_kernel(MoeParams p, OffsetList off, int* hist, int chunk,
+                                                                    int nchunk) {
   if (static_cast<int>(blockIdx.x) >= nchunk) {
-    prep_rest<true>(p, blockIdx.x - nchunk, gridDim.x - nchunk);
+    prep_rest(p, off, blockIdx.x - nchunk, gridDim.x - nchunk);
     return;
   }
   __shared__ int cnt[kMaxExperts + 1];
@@ -513,21 +536,32 @@ __global__ void __launch_bounds__(kRouteThreads) group_scatter_kernel(MoeParams 
 }
 
 // kRows: with the row-layout MFMA phases' expert order and the INT8 word
-// offsets.  A kernel without their code is shorter to fetch: 64 pairs of 256
-// experts 5.4 -> 4.9 us.
-template <bool kRows>
-__global__ void __launch_bounds__(kRouteThreads) prep_kernel(MoeParams p) {
+// offsets.  A kernel without their code and arguments (256 bytes) is shorter to
+// fetch: 64 pairs of 256 experts 5.4 -> 4.7 us.  kShift: a unit holds 1 <<
+// kShift pairs (0: no units).
+template <bool kRows, int kShift>
+__global__ void __launch_bounds__(kRouteThreads) prep_kernel(MoeParams p,
+                                                             std::conditional_t<kRows, OffsetList, NoOffsets> off) {
   if (blockIdx.x == 0)
-    route_block<kRows>(p);
+    route_block<kRows, kShift>(p);
   else
-    prep_rest<kRows>(p, blockIdx.x - 1, gridDim.x - 1);
+    prep_rest(p, off, blockIdx.x - 1, gridDim.x - 1);
 }
 
-void launch_prep(const MoeParams& p, unsigned blocks, hipStream_t s) {
-  if (p.n_off || p.longest_first)
-    hipLaunchKernelGGL(prep_kernel<true>, dim3(blocks), dim3(kRouteThreads), 0, s, p);
+void launch_prep(const MoeParams& p, const OffsetList& off, unsigned blocks, hipStream_t s) {
+  static_assert(stream::kMaxM == 16 && chain32::kUnitPairs == 4, "unit shifts");
+  const dim3 grid(blocks), block(kRouteThreads);
+  const bool rows = off.n || p.longest_first;
+  if (p.unit_shift == 4)
+    hipLaunchKernelGGL((prep_kernel<false, 4>), grid, block, 0, s, p, NoOffsets{});
+  else if (p.unit_shift == 2 && rows)
+    hipLaunchKernelGGL((prep_kernel<true, 2>), grid, block, 0, s, p, off);
+  else if (p.unit_shift == 2)
+    hipLaunchKernelGGL((prep_kernel<false, 2>), grid, block, 0, s, p, NoOffsets{});
+  else if (rows)
+    hipLaunchKernelGGL((prep_kernel<true, 0>), grid, block, 0, s, p, off);
   else
-    hipLaunchKernelGGL(prep_kernel<false>, dim3(blocks), dim3(kRouteThreads), 0, s, p);
+    hipLaunchKernelGGL((prep_kernel<false, 0>), grid, block, 0, s, p, NoOffsets{});
 }
 
 // ---------------------------------------------------------------------------
@@ -1110,7 +1144,7 @@ size_t int8_word_offset_bytes(const latent_moe_args& a) {
 // Set `word_offset` of every INT8 factor: the workspace tail for factors of
 // more than one bitmap word (filled beside the grouping, see prep_rest),
 // row_offset for the others.
-void set_int8_word_offsets(const latent_moe_args& a, char* tail, MoeParams& p) {
+void set_int8_word_offsets(const latent_moe_args& a, char* tail, MoeParams& p, OffsetList& list) {
   const latent_factor* fs[6] = {&a.gate_a, &a.gate_b, &a.up_a, &a.up_b, &a.down_a, &a.down_b};
   size_t off = 0;
   for (int i = 0; i < 6; ++i) {
@@ -1123,7 +1157,7 @@ void set_int8_word_offsets(const latent_moe_args& a, char* tail, MoeParams& p) {
     }
     int32_t* dst = reinterpret_cast<int32_t*>(tail + off);
     const int64_t rows = a.n_expert * f.rows;
-    p.off[p.n_off++] = WordOffsets{f.int8_bitmap, f.int8_row_offset, dst, rows, static_cast<int>(words)};
+    list.f[list.n++] = WordOffsets{f.int8_bitmap, f.int8_row_offset, dst, rows, static_cast<int>(words)};
     p.fac[i].ext.word_offset = dst;
     off += align_up(static_cast<size_t>(rows * words) * sizeof(int32_t));
   }
@@ -1244,6 +1278,7 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
   const int path = choose_path(a);
   if (path < 0) return path;
   MoeParams p{};
+  OffsetList off{};
   const latent_factor* fs[6] = {&a.gate_a, &a.gate_b, &a.up_a, &a.up_b, &a.down_a, &a.down_b};
   bool any_int8 = false;
   for (int i = 0; i < 6; ++i) {
@@ -1252,7 +1287,7 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
   }
   if (any_int8) {
     // The workspace's tail, after the largest path's scratch.
-    set_int8_word_offsets(a, static_cast<char*>(a.workspace) + need - int8_word_offset_bytes(a), p);
+    set_int8_word_offsets(a, static_cast<char*>(a.workspace) + need - int8_word_offset_bytes(a), p, off);
   }
   const Layout L = layout_for(a, extra);
   char* ws = static_cast<char*>(a.workspace) + kControlBytes;
@@ -1292,19 +1327,17 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
   }
   if (path == kPathFused) {
     const chain32::Layout CL = chain32::layout_for(a);
-    static_assert(chain32::kUnitPairs == 4, "unit_shift");
     p.unit_shift = 2;
     p.unit_info = reinterpret_cast<int4*>(ws + L.gu + CL.units);
     p.unit_tok = reinterpret_cast<int*>(p.unit_info + chain32::max_units(a));
     p.pos_of = reinterpret_cast<int*>(ws + L.gu + CL.pos_of);
-    launch_prep(p, p.n_off ? 257 : 1, s);
+    launch_prep(p, off, off.n ? 257 : 1, s);
     if (hipGetLastError() != hipSuccess) return LATENT_E_HIP;
     const chain32::Grouping g{p.meta, p.unit_info, p.unit_tok, p.pos_of, p.pair_w};
     return chain32::forward(a, p.fac, g, ws + L.gu, s);
   }
   if (use_stream) {
     const int64_t mu = stream::max_units(P, a.n_expert);
-    static_assert(stream::kMaxM == 16, "unit_shift");
     p.unit_shift = 4;
     p.unit_info = reinterpret_cast<int4*>(ws + L.units);
     p.unit_tok = reinterpret_cast<int*>(p.unit_info + mu);
@@ -1347,7 +1380,7 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
   // workgroup per token.
   const int64_t conv_blocks = use_stream || use_rows ? a.n_tokens : 1;
   const int zero_blocks = static_cast<int>(std::min<int64_t>(
-      512, std::max<int64_t>(std::max<int64_t>(conv_blocks, p.n_off ? 256 : 0), zero_work / (kRouteThreads * 8))));
+      512, std::max<int64_t>(std::max<int64_t>(conv_blocks, off.n ? 256 : 0), zero_work / (kRouteThreads * 8))));
   // Large batches: the multi-workgroup grouping, for the row-layout MFMA phases
   // from 4096 pairs (64 experts, 11,994 pairs: 37 us in one workgroup), with
   // the other preparations beside its first kernel; prefill has none.
@@ -1355,12 +1388,12 @@ extern "C" int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream
     int* hist = reinterpret_cast<int*>(ws + L.hist);
     const int chunk = static_cast<int>(group_chunk(P, a.n_expert));
     const int nchunk = static_cast<int>(group_chunks(P, a.n_expert));
-    hipLaunchKernelGGL(group_count_kernel, dim3(nchunk + (use_rows ? zero_blocks : 0)), dim3(kRouteThreads), 0, s, p, hist,
-                       chunk, nchunk);
+    hipLaunchKernelGGL(group_count_kernel, dim3(nchunk + (use_rows ? zero_blocks : 0)), dim3(kRouteThreads), 0, s, p, off,
+                       hist, chunk, nchunk);
     hipLaunchKernelGGL(group_scan_kernel, dim3(1), dim3(kRouteThreads), 0, s, p, hist, nchunk);
     hipLaunchKernelGGL(group_scatter_kernel, dim3(nchunk), dim3(kRouteThreads), 0, s, p, hist, chunk);
   } else {
-    launch_prep(p, 1 + zero_blocks, s);
+    launch_prep(p, off, 1 + zero_blocks, s);
   }
   if (hipGetLastError() != hipSuccess) return LATENT_E_HIP;
   if (use_prefill) {

@@ -120,10 +120,9 @@ struct Params {
   int* dexp;           // [P]
   float* ybuf;         // [P][d]
   int T, K, E, d, ff, P, wbd, out_mode;
-  int direct;            // phase D writes the per-slot output itself
   int nka, nb, nkc, nd;  // tiles per unit and factor: A (d/256), B (ff/128), C (ff/256), D (d/256)
   int G;                 // workgroups the tile ranges are cut for
-  const int* pair_tok;    // [P] token of each grouped pair (bulk launches, direct)
+  const int* pair_tok;    // [P] token of each grouped pair (bulk launches, kSlots)
   const int* pair_slot;   // [P] slot of each grouped pair
   // Bulk (prefill) launches only.
   const float* pair_w;    // [P] router weight of each grouped pair
@@ -832,8 +831,10 @@ constexpr int kRemPieces = 2;  // rest pieces per workgroup range (<= per_key ti
 // at most kRows pairs (partial blocks of kRows rows).
 // kPerItem: phase C's partials are one per item (bc_kernel), row (pair * nkc
 // + j) for item j of a unit, summed in item order.  kByKey: the bulk launches' slots (Deal): a whole
-// key's one partial, or a rest key's pieces in workgroup order.
-template <int kPhase, int kRows, bool kPerItem = false, bool kByKey = false>
+// key's one partial, or a rest key's pieces in workgroup order.  kSlots (phase
+// C): see item_kernel; a pair's output row beside its exponent, zeros for the
+// dropped slots.
+template <int kPhase, int kRows, bool kPerItem = false, bool kByKey = false, bool kSlots = false>
 __global__ void __launch_bounds__(kT) reduce_kernel(Params p) {
   const int lane = threadIdx.x & (kWave - 1);
   const int per_unit = tiles_per_unit<kPhase>(p), per_key = tiles_per_key<kPhase>(p);
@@ -945,11 +946,11 @@ __global__ void __launch_bounds__(kT) reduce_kernel(Params p) {
     if (kPhase == kPhaseA)
       finish_row(s, p.lat + (static_cast<int64_t>(f) * p.P + pair) * kK, p.lexp + f * p.P + pair, lane);
     else
-      finish_row(s, p.dlat + pair * kK, p.dexp + pair, lane, p.direct ? p.pair_tok[pair] * p.K + p.pair_slot[pair] : -1);
+      finish_row(s, p.dlat + pair * kK, p.dexp + pair, lane, kSlots ? p.pair_tok[pair] * p.K + p.pair_slot[pair] : -1);
   }
-  if constexpr (kPhase == kPhaseC && kPerItem) {
+  if constexpr (kSlots) {
     // Phase D writes no dropped slot's row.
-    for (int r = blockIdx.x; p.direct && r < p.P; r += gridDim.x) {
+    for (int r = blockIdx.x; r < p.P; r += gridDim.x) {
       const int e = p.ids[r];
       if (e >= 0 && e < p.E) continue;
       float4* o = reinterpret_cast<float4*>(p.out + static_cast<int64_t>(r) * p.d);
@@ -959,8 +960,8 @@ __global__ void __launch_bounds__(kT) reduce_kernel(Params p) {
 }
 
 // out from the y rows of the routed slots, in slot order: reduced mode sums
-// w * y over the token's slots; per-slot mode with the weight before
-// the down projection writes w * y (y is linear in h) and zero for a dropped slot.
+// w * y over the token's slots; per-slot mode writes y (times w when the weight
+// goes before the down projection: y is linear in h) and zero for a dropped slot.
 // d % 256 == 0, so the 64 float4 columns of a wave lie in one output row: the
 // slot's id, weight and grouped position are wave-uniform (scalar loads), and
 // the y rows of kCombineBatch slots are loaded before any is added.
@@ -997,8 +998,10 @@ __global__ void __launch_bounds__(kT) combine_kernel(Params p) {
       const int e = p.ids[r];
       if (e >= 0 && e < p.E) {
         s = reinterpret_cast<const float4*>(p.ybuf + static_cast<int64_t>(p.pos_of[r]) * p.d)[c4];
-        const float w = load_act(p.weights, p.w_dtype, r);
-        s.x *= w; s.y *= w; s.z *= w; s.w *= w;
+        if (p.wbd) {
+          const float w = load_act(p.weights, p.w_dtype, r);
+          s.x *= w; s.y *= w; s.z *= w; s.w *= w;
+        }
       }
     }
     reinterpret_cast<float4*>(p.out)[i] = s;
@@ -2774,7 +2777,7 @@ int forward(const latent_moe_args& a, const Grouping& g, char* scratch, hipStrea
   p.out_mode = a.out_mode;
   // reduce_kernel tags a pair's exponent with its output row (T * K rows).
   static_assert(kMaxPairs < (1 << 23), "output row in 23 bits");
-  p.direct = p.out_mode == LATENT_OUT_PER_SLOT && !p.wbd ? 1 : 0;
+  const bool slots = p.out_mode == LATENT_OUT_PER_SLOT && !p.wbd;
   p.pair_tok = g.pair_tok;
   p.pair_slot = g.pair_slot;
   p.nka = p.d / kK;
@@ -2792,12 +2795,13 @@ int forward(const latent_moe_args& a, const Grouping& g, char* scratch, hipStrea
   hipLaunchKernelGGL((reduce_kernel<kPhaseA, kMaxM>), dim3(blocks((U * 2 * kMaxM + rows_per_block - 1) / rows_per_block)),
                      dim3(kT), 0, s, p);
   hipLaunchKernelGGL(bc_kernel, dim3(item_grid(p.nkc)), dim3(kT), 0, s, p);
-  hipLaunchKernelGGL((reduce_kernel<kPhaseC, kMaxM, true>), dim3(blocks((U * kMaxM + rows_per_block - 1) / rows_per_block)),
-                     dim3(kT), 0, s, p);
-  if (p.direct) {
+  const dim3 c_grid(blocks((U * kMaxM + rows_per_block - 1) / rows_per_block));
+  if (slots) {
+    hipLaunchKernelGGL((reduce_kernel<kPhaseC, kMaxM, true, false, true>), c_grid, dim3(kT), 0, s, p);
     hipLaunchKernelGGL((item_kernel<kPhaseD, true>), dim3(item_grid(p.nd)), dim3(kT), 0, s, p);
     return hipGetLastError() == hipSuccess ? LATENT_OK : LATENT_E_HIP;
   }
+  hipLaunchKernelGGL((reduce_kernel<kPhaseC, kMaxM, true>), c_grid, dim3(kT), 0, s, p);
   hipLaunchKernelGGL(item_kernel<kPhaseD>, dim3(item_grid(p.nd)), dim3(kT), 0, s, p);
   const int64_t out4 = (a.out_mode == LATENT_OUT_REDUCED ? p.T : static_cast<int64_t>(p.P)) * p.d / 4;
   hipLaunchKernelGGL(combine_kernel, dim3(blocks((out4 + kT - 1) / kT)), dim3(kT), 0, s, p);

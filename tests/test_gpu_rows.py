@@ -128,6 +128,7 @@ def test_rows_pair_blocks(gpu, T, k, mode, wbd):
 
 @pytest.mark.parametrize("E,T,k", [
     (512, 700, 3),   # rounds of 1024 pairs: two and a part, the most experts they take
+    (512, 256, 4),   # exactly one of them
     (513, 260, 4),   # rounds of 512 pairs: two and 16 pairs
     (1024, 128, 4),  # one whole round, the most experts placed in order
     (1025, 129, 4),  # more experts: placed as the threads come
