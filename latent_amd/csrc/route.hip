@@ -572,10 +572,12 @@ int64_t split_tiles(const latent_route_args& a, int64_t tok) {
 
 // Slices of d (and, for the split kernel, their rows).
 int64_t n_slices(const latent_route_args& a, int* slice_rows) {
-  if (!split_applies(a)) return (a.n_embd + kRows - 1) / kRows;
-  // About two workgroups per CU, at most kFewSlices slices of whole steps.
+  const int64_t slices = (a.n_embd + kRows - 1) / kRows;
+  if (!split_applies(a)) return slices;
+  // About two workgroups per CU, at most kFewSlices slices of whole steps, and
+  // no more than the other route's (the workspace callers know).
   const int64_t tiles = split_tiles(a, kSTok);
-  const int64_t want = std::max<int64_t>(1, std::min<int64_t>(kFewSlices, 512 / tiles));
+  const int64_t want = std::max<int64_t>(1, std::min({int64_t{kFewSlices}, slices, 512 / tiles}));
   const int64_t rows = ((a.n_embd + want - 1) / want + kSStep - 1) / kSStep * kSStep;
   if (slice_rows) *slice_rows = static_cast<int>(rows);
   return (a.n_embd + rows - 1) / rows;
@@ -598,16 +600,17 @@ int validate(const latent_route_args& a) {
 
 size_t workspace_bytes(const latent_route_args& a) {
   if (a.logits_in) return 0;
-  // Partial rows.  A workspace sized for a batch also serves every smaller
-  // one: the split kernel's slices x tokens are bounded by an expression that
-  // grows with the tokens, and a batch just below its range needs ceil(d / 64)
-  // rows a token.
+  // Partial rows: ceil(d / 64) a token, fewer for the split kernel's batches.  A
+  // workspace sized for a batch also serves every smaller one: the split
+  // kernel's slices x tokens are bounded by an expression that grows with the
+  // tokens, and a batch just below its range needs ceil(d / 64) rows a token.
   const int64_t slices = (a.n_embd + kRows - 1) / kRows;
   if (a.n_embd % kSStep != 0) return static_cast<size_t>(slices * a.n_tokens) * a.n_expert * sizeof(float);
   int64_t rows = slices * std::min(a.n_tokens, split_tokens(a) - 1);
   if (split_applies(a)) {
     const int64_t neb = (a.n_expert + kSExp - 1) / kSExp;
     rows = std::max(rows, std::min(kFewSlices * a.n_tokens, std::max(a.n_tokens, 512 * kSTok / neb)));
+    rows = std::min(rows, slices * a.n_tokens);
   }
   return static_cast<size_t>(rows) * a.n_expert * sizeof(float);
 }

@@ -261,3 +261,21 @@ def test_tiles_repack_argument_checks(L):
     for factor, src, dst, status in bad:
         assert L.lib.latent_tiles_repack(factor, ctypes.byref(src), ctypes.byref(dst), 4, 1, None) == status
     assert L.lib.latent_tiles_repack(0, None, ctypes.byref(g), 4, 1, None) == L.LATENT_E_INVALID
+
+
+@pytest.mark.parametrize("d", [64, 96, 1024, 1408, 2048, 7168])
+@pytest.mark.parametrize("E", [8, 128, 160, 256, 1000])
+def test_route_workspace_is_at_most_one_partial_row_per_64_rows_of_d(L, d, E):
+    """T * E * 4 * ceil(d / 64) bytes hold any call (callers allocate by it), and
+    the workspace of a batch holds every smaller batch."""
+    a = L.LatentRouteArgs()
+    a.n_embd, a.n_expert, a.n_expert_used = d, E, min(8, E)
+    a.x_dtype = a.router_dtype = L.LATENT_F32
+    last = 0
+    for T in sorted({1, 2, 31, 64, 200, 285, 512, 1000, 2047, 2048, 3051, 3052, 4096, 8191, 16384, 65537} |
+                    {max(1, 400000000 // (d * E) + i) for i in (-1, 0, 1, 2)}):
+        a.n_tokens = T
+        n = ctypes.c_size_t(0)
+        assert L.lib.latent_route_workspace_size(ctypes.byref(a), ctypes.byref(n)) == L.LATENT_OK
+        assert last <= n.value <= T * E * 4 * -(-d // 64), (T, n.value)
+        last = n.value

@@ -81,6 +81,22 @@ def test_route_long_batches_against_float64(gpu, T, d, E, k, x_dtype, r_dtype, s
     np.testing.assert_allclose(w.cpu().numpy(), want_w, rtol=2e-6, atol=1e-7)
 
 
+def test_route_in_the_documented_workspace(gpu):
+    """A workspace of T E 4 ceil(d / 64) bytes holds a long batch of a small d
+    (its query once asked for more)."""
+    import torch
+
+    T, d, E = 3052, 1024, 128
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn((T, d), generator=gen, device="cuda")
+    W = torch.randn((d, E), generator=gen, device="cuda") / d ** 0.5
+    logits = torch.empty((T, E), dtype=torch.float32, device="cuda")
+    ws = torch.empty(T * E * 4 * -(-d // 64), dtype=torch.uint8, device="cuda")
+    gpu.route(6, x=x, router=W, logits_out=logits, workspace=ws)
+    want = x.double() @ W.double()
+    assert float((logits.double() - want).norm() / want.norm()) <= 3e-7
+
+
 def test_route_long_batches_non_finite(gpu):
     """A non-finite operand spoils its own tokens or experts only, as a plain
     fp32 sum has it: inf stays inf, inf - inf and NaN are NaN and never chosen."""
