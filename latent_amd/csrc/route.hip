@@ -142,12 +142,14 @@ __global__ void __launch_bounds__(kThreads) logits_kernel(Params p) {
 
 // ---- split_logits_kernel -------------------------------------------------------
 // Logits of longer batches.  A product of fp32 values is the sum of products of
-// their bf16 parts: v = v1 + v2 + v3 exactly, each part the leading 8
-// significant bits of what the earlier ones left (bf16 x is one part, f16 x
-// two), and bf16 products are exact in fp32.  Three bf16 MFMAs (bf16 x, fp32
-// router) replace the eight v_mfma_f32_16x16x4_f32 of the same 16x16x32 block
-// at a sixteenth of their cycles each.  Terms below 2^-24 of the leading one (x2 w3,
-// x3 w2, x3 w3) are left out: the rounding of one fp32 product is as large.
+// their bf16 parts: v = v1 + v2 + v3 exactly, each part what the earlier ones
+// left rounded to the nearest bf16 (bf16 x is one part, f16 x two), and bf16
+// products are exact in fp32.  Three bf16 MFMAs (bf16 x, fp32 router) replace
+// the eight v_mfma_f32_16x16x4_f32 of the same 16x16x32 block at a sixteenth of
+// their cycles each.  x2 w3, x3 w2 and x3 w3 are left out: |v2| <= 2^-8 |v| and
+// |v3| <= 2^-16 |v|, so each is at most 2^-24 of the product, the rounding of one
+// fp32 product, and of either sign (parts cut off instead of rounded leave terms
+// up to 2^-22, all of the product's sign: on positive data a bias).
 //
 // Workgroup: 128 tokens (two workgroups per CU) or 256 (one) x 128 experts,
 // waves of 64 x 64, one slice of d in steps of 32 rows, the next two steps'
@@ -159,9 +161,12 @@ __global__ void __launch_bounds__(kThreads) logits_kernel(Params p) {
 // tiles.  The terms below x1 w1 are summed in accumulators of their own: added
 // to the leading sums they would round at those sums' magnitude.
 //
-// A non-finite operand has no such parts (inf - inf): its logits come out NaN,
-// and topk_kernel computes every NaN logit again in fp32.
+// A non-finite operand, or one that rounds to infinity, has no such parts (inf -
+// inf): its logits come out NaN, and topk_kernel computes every NaN logit again
+// in fp32.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float float2v __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kSTok = 128, kSExp = 128, kSStep = 32;  // kSTok: the smaller token tile
 constexpr int kSPitch = kSStep + 8;  // bf16 per LDS row: 16-byte reads of 16 rows on distinct banks
@@ -176,11 +181,10 @@ __device__ __forceinline__ void split8(const float (&v)[8], u32x4 (&part)[N]) {
   for (int n = 0; n < N; ++n) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const uint32_t a = __float_as_uint(r[2 * j]), b = __float_as_uint(r[2 * j + 1]);
-      part[n][j] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+      part[n][j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(float2v{r[2 * j], r[2 * j + 1]}, bf16x2));
       if (n + 1 < N) {
-        r[2 * j] -= __uint_as_float(a & 0xFFFF0000u);
-        r[2 * j + 1] -= __uint_as_float(b & 0xFFFF0000u);
+        r[2 * j] -= __uint_as_float(part[n][j] << 16);
+        r[2 * j + 1] -= __uint_as_float(part[n][j] & 0xFFFF0000u);
       }
     }
   }

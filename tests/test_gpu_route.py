@@ -81,6 +81,32 @@ def test_route_long_batches_against_float64(gpu, T, d, E, k, x_dtype, r_dtype, s
     np.testing.assert_allclose(w.cpu().numpy(), want_w, rtol=2e-6, atol=1e-7)
 
 
+@pytest.mark.parametrize("x_dtype", ["f32", "f16"])
+@pytest.mark.parametrize("lo,hi", [(2 ** -7 - 2 ** -12, 2 ** -7), (2 ** -8 - 2 ** -12, 2 ** -8), (0.0, 2 ** -7), (-1.0, 0.0)])
+def test_route_long_batches_have_no_bias_on_positive_data(gpu, x_dtype, lo, hi):
+    """Positive operands 1 + u, u in [lo, hi): what the split leaves out of a
+    product has either sign, so the mean error over all logits is far below one
+    rounding (2^-24); parts cut off instead of rounded had 2^-22 of it."""
+    import torch
+
+    T, d, E = 1536, 2048, 128
+    gen = torch.Generator(device="cuda").manual_seed(5)
+
+    def draw(*shape):
+        return 1 + lo + (hi - lo) * torch.rand(shape, generator=gen, device="cuda", dtype=torch.float64)
+
+    x = draw(T, d).to({"f32": torch.float32, "f16": torch.float16}[x_dtype])
+    W = draw(d, E).float()
+    logits = torch.empty((T, E), dtype=torch.float32, device="cuda")
+    gpu.route(6, x=x, router=W, logits_out=logits)
+    want = x.double() @ W.double()
+    err = (logits.double() - want) / want
+    # f16 values in [1 + 2^-7 - 2^-12, 1 + 2^-7) are one or two numbers: their
+    # sums repeat, and so does the sums' own rounding.
+    assert float(err.mean().abs()) <= 2.0 ** -26
+    assert float(err.abs().max()) <= 8 * 2.0 ** -24
+
+
 def test_route_in_the_documented_workspace(gpu):
     """A workspace of T E 4 ceil(d / 64) bytes holds a long batch of a small d
     (its query once asked for more)."""
