@@ -354,19 +354,6 @@ __global__ void __launch_bounds__(2 * kTok, 2) split_logits_kernel(Params p) {
     }
 }
 
-// x[t] . router[:, e] in fp32 over 64-row slices, as logits_kernel sums it.
-__device__ __noinline__ float plain_logit(const Params& p, int t, int e) {
-  float v = 0.f;
-  for (int k0 = 0; k0 < p.d; k0 += kRows) {
-    float s = 0.f;
-    for (int k = k0; k < min(k0 + kRows, p.d); ++k)
-      s = fmaf(load_act(p.x, p.x_dtype, static_cast<int64_t>(t) * p.d + k),
-               load_act(p.router, p.router_dtype, static_cast<int64_t>(k) * p.E + e), s);
-    v += s;
-  }
-  return v;
-}
-
 // Wave arg-max of (v, idx) pairs: larger v wins, equal v -> smaller idx.
 // Each pair is one 64-bit key whose unsigned order is that order (the
 // float's bits made monotonic above, the complemented index below; -0 is
@@ -524,13 +511,62 @@ __global__ void __launch_bounds__(kThreads) topk_kernel(Params p) {
 // one token per workgroup (three of its four waves idle in the selection) took
 // 36 us.
 constexpr int kTopkWaves = 4;
+
+// Workgroup: x . router of tokens t0 .. t0 + 3 in fp32 over 64-row slices, as
+// logits_kernel sums it, into lg[token][expert].  A wave takes a quarter of the
+// experts for all four tokens, a batch of router rows in flight.
+template <int NJ, bool kWF32>
+__device__ __forceinline__ void plain_logits(const Params& p, int t0, float (&xs)[kTopkWaves][kRows],
+                                             float (&lg)[kTopkWaves][NJ * kWave]) {
+  constexpr int kJ = NJ / kTopkWaves, kAhead = kSStep / kJ;
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+  const int64_t xrow = static_cast<int64_t>(min(t0 + wave, p.T - 1)) * p.d;
+  int e[kJ];
+  float acc[kJ][kTopkWaves] = {};
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) e[j] = min((wave * kJ + j) * kWave + lane, p.E - 1);
+  for (int k0 = 0; k0 < p.d; k0 += kRows) {
+    const int rows = min(kRows, p.d - k0);  // a multiple of kSStep
+    __syncthreads();
+    xs[wave][lane] = load_act(p.x, p.x_dtype, xrow + k0 + min(lane, rows - 1));
+    __syncthreads();
+    float s[kJ][kTopkWaves] = {};
+    for (int r = 0; r < rows; r += kAhead) {
+      float w[kAhead][kJ];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+        for (int j = 0; j < kJ; ++j)
+          w[i][j] = load_act(p.router, kWF32 ? LATENT_F32 : LATENT_BF16, static_cast<int64_t>(k0 + r + i) * p.E + e[j]);
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+        for (int t = 0; t < kTopkWaves; ++t) {
+          const float x = xs[t][r + i];
+#pragma unroll
+          for (int j = 0; j < kJ; ++j) s[j][t] = fmaf(x, w[i][j], s[j][t]);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < kJ; ++j)
+#pragma unroll
+      for (int t = 0; t < kTopkWaves; ++t) acc[j][t] += s[j][t];
+  }
+#pragma unroll
+  for (int j = 0; j < kJ; ++j)
+#pragma unroll
+    for (int t = 0; t < kTopkWaves; ++t) lg[t][(wave * kJ + j) * kWave + lane] = acc[j][t];
+  __syncthreads();
+}
+
 template <int NJ>
 __global__ void __launch_bounds__(kTopkWaves * kWave) topk_wave_kernel(Params p) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int t = blockIdx.x * kTopkWaves + (threadIdx.x >> 6);
-  if (t >= p.T) return;
+  __shared__ float xs[kTopkWaves][kRows];
+  __shared__ float lg[kTopkWaves][NJ * kWave];
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+  const int t = blockIdx.x * kTopkWaves + wave;
   const int64_t stride = static_cast<int64_t>(p.T) * p.E;
-  const float* row = p.partial + static_cast<int64_t>(t) * p.E;
+  const float* row = p.partial + static_cast<int64_t>(min(t, p.T - 1)) * p.E;
   float l[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) l[j] = 0.f;
@@ -540,18 +576,31 @@ __global__ void __launch_bounds__(kTopkWaves * kWave) topk_wave_kernel(Params p)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) l[j] += src[min(j * kWave + lane, p.E - 1)];
   }
+  bool nan = false;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) nan = nan || l[j] != l[j];
+  if (__syncthreads_or(nan)) {
+    // NaN logits in fp32, the workgroup's four tokens together: 4096 tokens of
+    // one NaN each, d 7168, 256 experts 0.48 ms a call, finite 59 us.  A lane
+    // summing a token's d alone took 10 ms, and its call's stack made the finite
+    // ones 66.
+    if (p.router_dtype == LATENT_F32)
+      plain_logits<NJ, true>(p, blockIdx.x * kTopkWaves, xs, lg);
+    else
+      plain_logits<NJ, false>(p, blockIdx.x * kTopkWaves, xs, lg);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      if (l[j] != l[j]) l[j] = lg[wave][j * kWave + lane];
+  }
+  if (t >= p.T) return;
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
     const int e = j * kWave + lane;
-    if (e < p.E) {
-      if (l[j] != l[j]) l[j] = plain_logit(p, t, e);
-      if (p.logits_out) p.logits_out[static_cast<int64_t>(t) * p.E + e] = l[j];
-    }
+    if (e < p.E && p.logits_out) p.logits_out[static_cast<int64_t>(t) * p.E + e] = l[j];
     l[j] = e >= p.E || l[j] != l[j] ? -INFINITY : l[j];  // NaN never wins a slot
   }
   select_topk<NJ>(p, t, lane, l);
 }
-
 
 // split_logits_kernel from this many multiply-adds (T E d).  Both routes in us,
 // MI355X, logits and top-k, bf16 x and fp32 router:

@@ -150,6 +150,69 @@ def test_route_long_batches_non_finite(gpu):
     assert not chosen[rows].any() and (got[rows] >= 0).all()
 
 
+@pytest.mark.parametrize("T,d,E,k,x_dtype,r_dtype", [
+    (1534, 2080, 130, 6, "f32", "f32"),    # two tokens in the last workgroup, d ends in half a slice
+    (301, 1408, 1000, 9, "bf16", "bf16"),  # 16 experts a lane
+    (2049, 3072, 64, 6, "f16", "f32"),
+])
+def test_route_long_batches_recompute(gpu, T, d, E, k, x_dtype, r_dtype):
+    """Logits without bf16 parts come from the fp32 sum: tokens of inf and NaN
+    beside finite ones, a router value that rounds to infinity in bf16 (finite
+    logits), one that is infinite."""
+    import torch
+
+    tdt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn((T, d), generator=gen, device="cuda").to(tdt[x_dtype])
+    W = (torch.randn((d, E), generator=gen, device="cuda") / d ** 0.5).to(tdt[r_dtype])
+    x[2, 5] = float("nan")
+    x[3, d - 1] = float("inf")
+    x[T - 1, 0] = float("-inf")
+    W[d - 1, E - 1] = torch.finfo(W.dtype).max
+    x[:, d - 1] = x[:, d - 1].clamp(-0.5, 0.5)
+    x[3, d - 1] = float("inf")
+    W[7, 3] = float("inf")
+    logits = torch.empty((T, E), dtype=torch.float32, device="cuda")
+    ids, _ = gpu.route(k, x=x, router=W, logits_out=logits)
+    want = x.double() @ W.double()
+    assert torch.equal(torch.isnan(logits), torch.isnan(want))
+    assert torch.equal(torch.isinf(logits), torch.isinf(want))
+    inf = torch.isinf(want)
+    assert torch.equal(logits[inf].double(), want[inf])
+    fin = torch.isfinite(want)
+    scale = x.double().abs() @ W.double().abs()
+    assert float(((logits.double() - want).abs() / scale)[fin].max()) <= 8 * 2.0 ** -24
+    rows = torch.isnan(want).sum(1) < E - k
+    assert not torch.gather(torch.isnan(want), 1, ids.long().clamp(min=0))[rows].any()
+
+
+def test_route_of_nan_tokens_stays_bounded(gpu):
+    """A batch with a NaN in every token takes some 8 times a finite one's time
+    (140 times when a lane summed a token alone)."""
+    import torch
+
+    T, d, E = 4096, 7168, 256
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.randn((T, d), generator=gen, device="cuda").bfloat16()
+    r = gpu.Router(torch.randn((d, E), generator=gen, device="cuda") / d ** 0.5, 8)
+
+    def best(x):
+        times = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(5):
+                r(x)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    finite = best(x)
+    x[:, -1] = float("nan")
+    assert best(x) < 30 * finite
+
+
 @pytest.mark.parametrize("drop,param", [("none", 0.0), ("below", 0.05), ("below", 0.2), ("inclusive", 0.95),
                                         ("inclusive", 0.5)])
 def test_route_from_logits_drop_rules(gpu, drop, param):
