@@ -147,7 +147,8 @@ const char* latent_status_string(int status);
 /*
  * Workspace bytes for latent_moe_ffn_forward with these dims.  A call given
  * less runs where its kernels have a form that needs less (row-layout prefill:
- * the grouped GEMMs) and returns LATENT_E_WORKSPACE otherwise.
+ * the grouped GEMMs; path 4 below: atomics into the output) and returns
+ * LATENT_E_WORKSPACE otherwise.
  */
 int latent_moe_workspace_size(const latent_moe_args* args, size_t* bytes);
 

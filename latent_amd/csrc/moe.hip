@@ -958,6 +958,18 @@ int64_t xh_cols(const latent_moe_args& a) {
   return a.layout == LATENT_LAYOUT_ROWS && a.max_rank <= 512 ? a.n_embd : 0;
 }
 
+// Workspace tail holding the per-word INT8 offsets of the factors whose rows
+// span more than one bitmap word (factors of one word use row_offset).
+size_t int8_word_offset_bytes(const latent_moe_args& a) {
+  const latent_factor* fs[6] = {&a.gate_a, &a.gate_b, &a.up_a, &a.up_b, &a.down_a, &a.down_b};
+  size_t n = 0;
+  for (const latent_factor* f : fs) {
+    const int64_t words = (f->cols / kGroup + 31) / 32;
+    if (f->int8_bitmap && words > 1) n += align_up(static_cast<size_t>(a.n_expert * f->rows * words) * sizeof(int32_t));
+  }
+  return n;
+}
+
 // The shape and work split of a row-layout MFMA call.
 rows::Params rows_shape(const latent_moe_args& a, bool int8, bool ordered) {
   rows::Params r{};
@@ -1023,13 +1035,13 @@ Layout layout_for(const latent_moe_args& a, bool extra) {
       L.ordered = true;
       place_y(rows::sums_bytes(rows_shape(a, false, true)));
     }
-  } else if (d > 0 && P >= 2048) {
+  } else if (extra && d > 0 && P >= 2048) {
     // y rows, summed per token at the end, from 2048 pairs (25 M fp32 atomics
     // into out took 75 us of a call's 113 in phase D); not where they alone
     // would take the call past the library's own scratch array.
-    const size_t bytes = static_cast<size_t>(P) * d * sizeof(float);
+    const size_t bytes = static_cast<size_t>(P) * d * sizeof(float), tail = int8_word_offset_bytes(a);
     const bool roomy = a.layout == LATENT_LAYOUT_ROWS && prefill::supported(a) && prefill::layout_for(a).total > kOwn;
-    if (align_up(off + P * sizeof(int)) + align_up(bytes) <= kOwn || off > kOwn || roomy) place_y(bytes);
+    if (align_up(align_up(off + P * sizeof(int)) + bytes) + tail <= kOwn || off + tail > kOwn || roomy) place_y(bytes);
   }
   L.total = off;
   return L;
@@ -1129,18 +1141,6 @@ int launch_phases(const MoeParams& p, hipStream_t s) {
   return LATENT_OK;
 }
 
-// Workspace tail holding the per-word INT8 offsets of the factors whose rows
-// span more than one bitmap word (factors of one word use row_offset).
-size_t int8_word_offset_bytes(const latent_moe_args& a) {
-  const latent_factor* fs[6] = {&a.gate_a, &a.gate_b, &a.up_a, &a.up_b, &a.down_a, &a.down_b};
-  size_t n = 0;
-  for (const latent_factor* f : fs) {
-    const int64_t words = (f->cols / kGroup + 31) / 32;
-    if (f->int8_bitmap && words > 1) n += align_up(static_cast<size_t>(a.n_expert * f->rows * words) * sizeof(int32_t));
-  }
-  return n;
-}
-
 // Set `word_offset` of every INT8 factor: the workspace tail for factors of
 // more than one bitmap word (filled beside the grouping, see prep_rest),
 // row_offset for the others.
@@ -1185,7 +1185,8 @@ extern "C" const char* latent_status_string(int status) {
 namespace latent {
 // Workspace bytes of a valid call: control block (zero between calls), scratch
 // the paths share, INT8 word offsets.  extra: with the planes of row-layout
-// prefill in place of its GEMMs; a call given less runs the GEMMs.
+// prefill in place of its GEMMs and the y rows of the other row-layout MFMA
+// calls; a call given less runs the GEMMs, or adds into its output.
 size_t moe_workspace_bytes(const latent_moe_args& a, bool extra) {
   const Layout L = layout_for(a, extra);
   size_t scratch = L.total;

@@ -279,3 +279,49 @@ def test_route_workspace_is_at_most_one_partial_row_per_64_rows_of_d(L, d, E):
         assert L.lib.latent_route_workspace_size(ctypes.byref(a), ctypes.byref(n)) == L.LATENT_OK
         assert last <= n.value <= T * E * 4 * -(-d // 64), (T, n.value)
         last = n.value
+
+
+def _int8_args(L, T, d, ff, E, k, R):
+    """A layer with INT8 groups in every factor; host pointers that are never read."""
+    buf = np.zeros(64, np.uint8)
+    base = buf.ctypes.data + (-buf.ctypes.data) % 16
+    a = L.LatentMoeArgs()
+
+    def fac(rows, cols):
+        return L.LatentFactor(codes=base, scales=base, rows=rows, cols=cols, int8_bitmap=base, int8_row_offset=base,
+                              int8_data=base)
+
+    a.gate_a, a.gate_b, a.up_a, a.up_b = fac(d, R), fac(R, ff), fac(d, R), fac(R, ff)
+    a.down_a, a.down_b = fac(ff, R), fac(R, d)
+    a.n_tokens, a.n_embd, a.n_ff, a.n_expert, a.n_expert_used, a.max_rank = T, d, ff, E, k, R
+    a.x_dtype, a.weights_dtype, a.out_mode = L.LATENT_BF16, L.LATENT_F32, L.LATENT_OUT_REDUCED
+    return a, buf
+
+
+def _fits_noalloc(L, a):
+    """Whether the allocation-free entry point takes the call: without a GPU it
+    then goes on to the device and fails there."""
+    return L.lib.latent_moe_ffn_forward_noalloc(ctypes.byref(a), None) != L.LATENT_E_WORKSPACE
+
+
+@pytest.mark.parametrize("d,ff,E,k,R,Ts", [
+    (7168, 2048, 256, 8, 128, (255, 256, 257, 260, 400)),
+    (5120, 1536, 128, 2, 512, (1000, 1020, 1024, 1040, 1200)),
+    (4096, 2048, 256, 8, 512, (300, 332, 333, 345, 354, 355, 400)),
+    (2048, 1408, 64, 6, 512, (700, 731, 732, 740, 741, 800)),
+])
+def test_optional_scratch_refuses_no_allocation_free_call(L, d, ff, E, k, R, Ts):
+    """The library's own scratch array takes every batch up to the largest whose
+    accumulators it holds: y rows, which a call can do without, and the INT8 word
+    offsets behind them never push one over it."""
+    import torch
+
+    if torch.cuda.is_available():
+        pytest.skip("host pointers: only where the call ends before a launch")
+    for T in Ts:
+        a, keep = _int8_args(L, T, d, ff, E, k, R)
+        assert _fits_noalloc(L, a), T
+        st, size = _ws(L, a)
+        assert st == L.LATENT_OK and size <= L.LATENT_NOALLOC_SCRATCH_BYTES, (T, size)
+    a, keep = _int8_args(L, 65536, d, ff, E, k, R)
+    assert not _fits_noalloc(L, a)

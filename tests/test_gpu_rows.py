@@ -242,3 +242,33 @@ def test_row_layout_prefill_in_less_workspace(gpu, monkeypatch):
     assert torch.equal(gemms, gpu.moe_forward(x, it, wt, dev, workspace=ws[:full - 256]))
     with pytest.raises(LatentError):
         gpu.moe_forward(x, it, wt, dev, workspace=ws[:full // 3])
+
+
+def test_rows_in_less_workspace(gpu):
+    """Given less than the queried size, a call of 2048 pairs or more adds into its
+    output instead of combining y rows; INT8 word offsets (two bitmap words a row)
+    follow whichever scratch it has."""
+    import torch
+
+    from latent_amd._lib import LatentError
+
+    host = synth.make_layer(seed=6, n_expert=6, d=1056, ff=1088, max_rank=96, int8_fraction=0.1)
+    dev = _rows_layer(host)
+    rng = np.random.default_rng(9)
+    T, k = 700, 3
+    x = rng.standard_normal((T, host.d)).astype(np.float32)
+    ids, w = routing.softmax_topk(rng.standard_normal((T, 6)), k)
+    xt, wt = torch.from_numpy(x).cuda(), torch.from_numpy(w.astype(np.float32)).cuda()
+    it = torch.from_numpy(ids.astype(np.int32)).cuda()
+    full = gpu.workspace_size(dev, T, k)
+    ws = torch.zeros(full, dtype=torch.uint8, device="cuda")
+    y_rows = gpu.moe_forward(xt, it, wt, dev, workspace=ws)
+    least = full - T * k * (host.d + 1) * 4 // 256 * 256  # without y rows and their positions
+    added = gpu.moe_forward(xt, it, wt, dev, workspace=ws[:least + 256])
+    pick = np.arange(0, T, 17)
+    want = ref.moe_forward(x[pick], ids[pick], w[pick], host)
+    for got in (y_rows, added):
+        assert ref.rel_l2(want, got.cpu().numpy()[pick]) <= TOL
+    assert ref.rel_l2(y_rows.cpu().numpy(), added.cpu().numpy()) <= 1e-5
+    with pytest.raises(LatentError):
+        gpu.moe_forward(xt, it, wt, dev, workspace=ws[:least // 2])
