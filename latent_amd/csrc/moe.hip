@@ -934,9 +934,6 @@ __global__ void __launch_bounds__(kThreads) phase_d_kernel(MoeParams p) {
 constexpr size_t kAlign = 256;
 inline size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
-// Scratch of the library's own array (latent_moe_ffn_forward_noalloc).
-constexpr size_t kOwn = LATENT_NOALLOC_SCRATCH_BYTES - LATENT_NOALLOC_CONTROL_BYTES;
-
 struct Layout {
   size_t meta, act_expert, act_start, act_count, pair_tok, pair_slot, pair_w, hist, units, gu, dl, xh, xexp, pos_of, y, total;
   bool ordered;  // y holds an ordered row-layout call's planes, then its y rows
@@ -1035,13 +1032,16 @@ Layout layout_for(const latent_moe_args& a, bool extra) {
       L.ordered = true;
       place_y(rows::sums_bytes(rows_shape(a, false, true)));
     }
-  } else if (extra && d > 0 && P >= 2048) {
+  } else if (extra && d > 0 && P >= 2048 && a.out_mode == LATENT_OUT_REDUCED && !prefill::supported(a)) {
     // y rows, summed per token at the end, from 2048 pairs (25 M fp32 atomics
-    // into out took 75 us of a call's 113 in phase D); not where they alone
-    // would take the call past the library's own scratch array.
-    const size_t bytes = static_cast<size_t>(P) * d * sizeof(float), tail = int8_word_offset_bytes(a);
-    const bool roomy = a.layout == LATENT_LAYOUT_ROWS && prefill::supported(a) && prefill::layout_for(a).total > kOwn;
-    if (align_up(align_up(off + P * sizeof(int)) + bytes) + tail <= kOwn || off + tail > kOwn || roomy) place_y(bytes);
+    // into out took 75 us of a call's 113 in phase D) to 256 MiB of them: they
+    // are most of such a call's workspace.  Us with y rows / atomics: E 64, d
+    // 2048, ff 1408, rank 64, top-6: 350 tokens 72 / 80, 2000 179 / 235; E 128,
+    // d 4096, ff 2048, rank 192, top-8: 256 tokens 188 / 195, 2048 (256 MiB) 617
+    // / 716, 4096 1,045 / 1,230; d 7168, ranks 64..512, 10 % INT8 groups: 256
+    // tokens 487 / 495, 4096 (896 MiB) 3,974 / 3,982.
+    const size_t bytes = static_cast<size_t>(P) * d * sizeof(float);
+    if (bytes <= size_t{256} << 20) place_y(bytes);
   }
   L.total = off;
   return L;

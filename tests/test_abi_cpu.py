@@ -321,7 +321,31 @@ def test_optional_scratch_refuses_no_allocation_free_call(L, d, ff, E, k, R, Ts)
     for T in Ts:
         a, keep = _int8_args(L, T, d, ff, E, k, R)
         assert _fits_noalloc(L, a), T
-        st, size = _ws(L, a)
-        assert st == L.LATENT_OK and size <= L.LATENT_NOALLOC_SCRATCH_BYTES, (T, size)
     a, keep = _int8_args(L, 65536, d, ff, E, k, R)
     assert not _fits_noalloc(L, a)
+
+
+@pytest.mark.parametrize("int8", [False, True])
+def test_optional_scratch_is_bounded_and_only_where_it_is_used(L, int8):
+    """What a row-layout call can do without is at most 256 MiB of y rows, in the
+    reduced mode, on the path that writes them; prefill calls that run the GEMMs
+    and per-slot calls reserve none."""
+    d, ff, E, k, R = 7168, 2048, 256, 8, 512
+    for T in (256, 1024, 4096, 16384, 65536):
+        a, keep = _int8_args(L, T, d, ff, E, k, R)
+        if not int8:
+            for name in ("gate_a", "gate_b", "up_a", "up_b", "down_a", "down_b"):
+                getattr(a, name).int8_bitmap = None
+        reduced = _ws(L, a)[1]
+        a.out_mode = L.LATENT_OUT_PER_SLOT
+        slots = _ws(L, a)[1]
+        P = T * k
+        # Accumulators, fp16 x rows and grouping; GEMMs: fp16 intermediates and y.
+        least = P * 12 * R + T * d * 2
+        gemms = P * (3 * R + ff + d) * 2 + T * d * 2
+        rest = (32 << 20) + 256 * P
+        if int8:
+            assert least <= slots <= least + rest
+            assert slots <= reduced <= least + rest + min(4 * P * (d + 1), 256 << 20)
+        elif T >= 4096:
+            assert reduced <= max(least, gemms) + rest

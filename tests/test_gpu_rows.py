@@ -269,6 +269,9 @@ def test_rows_in_less_workspace(gpu):
     want = ref.moe_forward(x[pick], ids[pick], w[pick], host)
     for got in (y_rows, added):
         assert ref.rel_l2(want, got.cpu().numpy()[pick]) <= TOL
-    assert ref.rel_l2(y_rows.cpu().numpy(), added.cpu().numpy()) <= 1e-5
+    # The latents' sums differ in their last bits from call to call (atomics, a few
+    # 2^-24); about 2^-11 of them then round to another fp16 value, 2^-11 away:
+    # 2^-11 sqrt(2^-11) = 1e-5 of a row, ten times that allowed.
+    assert ref.rel_l2(y_rows.cpu().numpy(), added.cpu().numpy()) <= 1e-4
     with pytest.raises(LatentError):
         gpu.moe_forward(xt, it, wt, dev, workspace=ws[:least // 2])
