@@ -678,9 +678,11 @@ __global__ void __launch_bounds__(kT) sum_planes_kernel(const float* planes, int
 }
 
 // Reduced output from y rows: the weighted sum over a token's slots in slot
-// order, one float4 per thread.
+// order, one float4 per thread.  One grid dimension: a call may have more tokens
+// than the 65,535 workgroups of another.
 __global__ void __launch_bounds__(kT) combine_kernel(Params p) {
-  const int d4 = p.d / 4, t = blockIdx.y, c = blockIdx.x * kT + threadIdx.x;
+  const int d4 = p.d / 4, per = (d4 + kT - 1) / kT;
+  const int t = blockIdx.x / per, c = (blockIdx.x - t * per) * kT + threadIdx.x;
   if (c >= d4) return;
   float4v s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
@@ -722,7 +724,8 @@ int launch_phases(const Params& p, hipStream_t s) {
     hipLaunchKernelGGL((d_kernel<MB, kInt8, true>), dim3(8 * groups * p.n_d), dim3(kT), lds_d<MB>(p.R), s, p);
   else
     hipLaunchKernelGGL((d_kernel<MB, kInt8, false>), dim3(8 * groups * p.n_d), dim3(kT), lds_d<MB>(p.R), s, p);
-  if (p.y) hipLaunchKernelGGL(combine_kernel, dim3((p.d / 4 + kT - 1) / kT, p.T), dim3(kT), 0, s, p);
+  const unsigned per_token = (p.d / 4 + kT - 1) / kT;
+  if (p.y) hipLaunchKernelGGL(combine_kernel, dim3(per_token * p.T), dim3(kT), 0, s, p);
   return hipGetLastError() == hipSuccess ? LATENT_OK : LATENT_E_HIP;
 }
 

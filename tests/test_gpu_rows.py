@@ -275,3 +275,22 @@ def test_rows_in_less_workspace(gpu):
     assert ref.rel_l2(y_rows.cpu().numpy(), added.cpu().numpy()) <= 1e-4
     with pytest.raises(LatentError):
         gpu.moe_forward(xt, it, wt, dev, workspace=ws[:least // 2])
+
+
+def test_rows_more_tokens_than_a_grid_dimension(gpu):
+    """70,000 tokens, y rows and their combine: beyond the 65,535 workgroups of a
+    launch's second dimension."""
+    import torch
+
+    host = synth.make_layer(seed=4, n_expert=3, d=64, ff=64, max_rank=32)
+    dev = _rows_layer(host)
+    rng = np.random.default_rng(1)
+    T = 70000
+    x = rng.standard_normal((T, host.d)).astype(np.float32)
+    ids = rng.integers(-1, 3, (T, 1)).astype(np.int32)
+    w = rng.random((T, 1)).astype(np.float32)
+    got = gpu.moe_forward(torch.from_numpy(x).cuda(), torch.from_numpy(ids).cuda(), torch.from_numpy(w).cuda(), dev)
+    got = got.cpu().numpy()
+    pick = np.array([0, 1, 65534, 65535, 65536, T - 1])
+    assert ref.rel_l2(ref.moe_forward(x[pick], ids[pick], w[pick], host), got[pick]) <= TOL
+    assert not got[ids[:, 0] < 0].any() and got[ids[:, 0] >= 0].any(1).all()
