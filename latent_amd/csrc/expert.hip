@@ -128,6 +128,7 @@ constexpr int kC = 64;        // columns per tile: one per lane
 constexpr int kWaves = kT / kWave;
 constexpr int kBT = 512, kBWaves = kBT / kWave;  // chain_bc: two products and their sums in one workgroup
 constexpr int kMaxSlices = 16, kMaxRanges = 32;
+constexpr int kRangeBlocks = 2048;  // chain_bc workgroups beyond which ranges only repeat the latents' sums
 constexpr int kChainRank = 256, kChainD = 2048, kChainFf = 4096;
 static_assert(kMT == 8 && kC == kWave, "activation rows of two float4, one column per lane");
 
@@ -356,17 +357,30 @@ struct Layout {
   size_t gl, ul, g, u, dl, part, part_a, part_c, total;
 };
 
-// Experts whose latents fit the chain's LDS and whose factors do not want more
-// than 16 slices of d and 32 ranges of ff.
-bool chain_applies(const Dims& m) {
-  return std::max({m.rg, m.ru, m.rd}) <= kChainRank && m.d <= kChainD && m.ff <= kChainFf && m.T <= 65535 * kMT;
-}
+// The split of a chain.  chain_bc's workgroups each sum all slices' latents, so
+// ranges of ff beyond what fills the chip only repeat that: d 2048, ff 4096, rank
+// 256, 4096 tokens 2,356 us at 32 ranges, 2,119 at four (and 256 -> 144 MiB).
 void chain_split(const Dims& m, Chain& c) {
   c.ks = static_cast<int>(std::max<int64_t>(32, (m.d + kMaxSlices - 1) / kMaxSlices));
   c.n_slice = static_cast<int>((m.d + c.ks - 1) / c.ks);
-  const int64_t tiles = (m.ff + kC - 1) / kC;
-  c.sub = static_cast<int>((tiles + kMaxRanges - 1) / kMaxRanges);
+  const int64_t tiles = (m.ff + kC - 1) / kC, token_tiles = std::max<int64_t>(1, (m.T + kMT - 1) / kMT);
+  const int64_t ranges = std::max<int64_t>(1, std::min<int64_t>(kMaxRanges, kRangeBlocks / token_tiles));
+  c.sub = static_cast<int>((tiles + ranges - 1) / ranges);
   c.n_range = static_cast<int>((tiles + c.sub - 1) / c.sub);
+}
+
+// Experts whose latents fit the chain's LDS and whose factors do not want more
+// than 16 slices of d and 32 ranges of ff.  Many tokens at a high rank keep a
+// launch per product: their latents (n_slice x ranks a token) are most of the
+// traffic.  Us, chain / products: d 2048, ff 4096, rank 256: 768 tokens 440 /
+// 559, 1024 596 / 545, 4096 2,119 / 1,807; d 512, ff 4096, rank 256: 1024 462 /
+// 451, 4096 1,612 / 1,363; d 2048, ff 4096, rank 192: 1024 308 / 421, 16,384
+// 4,387 / 5,688; d 512, ff 1408, rank 64: 4 21 / 119, 16,384 706 / 1,010.
+bool chain_applies(const Dims& m) {
+  if (std::max({m.rg, m.ru, m.rd}) > kChainRank || m.d > kChainD || m.ff > kChainFf || m.T > 65535 * kMT) return false;
+  Chain c{};
+  chain_split(m, c);
+  return m.T < 1024 || c.n_slice * (m.rg + m.ru) <= 16 * 2 * 192;
 }
 
 size_t part_floats(const Dims& m, int64_t K, int64_t N) {

@@ -138,6 +138,10 @@ def test_weight_ignored_without_weight_before_down(gpu):
     (4, 2049, 70, (40, 40, 40), "nf4"),     # one past the chain's d, ff and rank: a launch per product
     (5, 64, 4100, (40, 33, 40), "int8"),
     (3, 70, 96, (40, 40, 257), "nf4"),
+    (1023, 512, 96, (256, 256, 30), "nf4"),  # the most tokens of a chain at 16 slices of high ranks
+    (1024, 512, 96, (256, 256, 30), "nf4"),  # a launch per product
+    (2100, 96, 700, (64, 40, 33), "int8"),   # fewer ranges of ff than column tiles: 263 token tiles
+    (16500, 33, 130, (5, 7, 64), "nf4"),     # one range
 ])
 def test_chain_limits(gpu, T, d, ff, ranks, kind):
     """Both sides of the three-launch chain's limits, against fp32 sums of the
