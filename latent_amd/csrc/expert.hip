@@ -189,7 +189,7 @@ __device__ __forceinline__ void wave_rows(const Flat& f, int N, int n, int base,
 }
 
 __global__ void __launch_bounds__(kT) chain_a(Chain p) {
-  __shared__ float act[kChainD / kMaxSlices * kMT];
+  __shared__ __attribute__((aligned(16))) float act[kChainD / kMaxSlices * kMT];
   __shared__ float red[kWaves][kMT][kC];
   __shared__ float lv[16];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
@@ -236,7 +236,7 @@ __device__ __forceinline__ void sum_latents(const float* part, int n, int T, int
 }
 
 __global__ void __launch_bounds__(kBT) chain_bc(Chain p) {
-  __shared__ float lat[2 * kChainRank * kMT];
+  __shared__ __attribute__((aligned(16))) float lat[2 * kChainRank * kMT];
   __shared__ float dacc[kMT][kChainRank];
   __shared__ float red[kBWaves][kMT][kC];
   __shared__ __attribute__((aligned(16))) float hs[kC * kMT];
@@ -280,7 +280,7 @@ __global__ void __launch_bounds__(kBT) chain_bc(Chain p) {
 }
 
 __global__ void __launch_bounds__(kT) chain_d(Chain p) {
-  __shared__ float lat[kChainRank * kMT];
+  __shared__ __attribute__((aligned(16))) float lat[kChainRank * kMT];
   __shared__ float red[kWaves][kMT][kC];
   __shared__ float lv[16];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
