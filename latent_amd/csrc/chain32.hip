@@ -127,7 +127,7 @@ __device__ __forceinline__ void block_mfma(const Block<CPL>& b, const float (&ac
       float v[CPL];
 #pragma unroll
       for (int j = 0; j < CPL / 2; ++j) {
-        const uint32_t byte = (b.c[i][j >> 2] >> (8 * (j & 3))) & 0xFFu;
+        const uint32_t byte = (b.c[i] >> (8 * j)) & 0xFFu;
         const float2v lv = lds_ld<float2v>(lut + byte * (kCopies * 8));
         v[2 * j] = lv[0];
         v[2 * j + 1] = lv[1];

@@ -54,7 +54,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, 
 // One lane's codes and scales of a block (rows 8 kq + i).
 template <int CPL>
 struct Block {
-  uint32_t c[8][(CPL + 7) / 8];
+  uint32_t c[8];
   u16x2 s[4];  // rows 2 i, 2 i + 1
 };
 
@@ -87,19 +87,14 @@ __device__ __forceinline__ Src<CPL> make_src(const Factor& f, int e, int col0, i
 // Rows 2 h and 2 h + 1 of the lane in the block whose first row is `row` (uniform).
 template <int CPL>
 __device__ __forceinline__ void load_rows(const Src<CPL>& s, int row, int h, Block<CPL>& b) {
-  static_assert(CPL == 4 || CPL == 8 || CPL == 16, "columns per lane");
+  static_assert(CPL == 4 || CPL == 8, "columns per lane");
   const int oc = row * s.cs, os = row * s.ss;
 #pragma unroll
   for (int i = 2 * h; i < 2 * h + 2; ++i) {
-    if (CPL == 16) {
-      const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(s.rc, s.vc, oc + i * s.cs, 0));
-      b.c[i][0] = v[0];
-      b.c[i][(CPL + 7) / 8 - 1] = v[1];
-    } else if (CPL == 8) {
-      b.c[i][0] = __builtin_amdgcn_raw_buffer_load_b32(s.rc, s.vc, oc + i * s.cs, 0);
-    } else {
-      b.c[i][0] = __builtin_amdgcn_raw_buffer_load_b16(s.rc, s.vc, oc + i * s.cs, 0);
-    }
+    if (CPL == 8)
+      b.c[i] = __builtin_amdgcn_raw_buffer_load_b32(s.rc, s.vc, oc + i * s.cs, 0);
+    else
+      b.c[i] = __builtin_amdgcn_raw_buffer_load_b16(s.rc, s.vc, oc + i * s.cs, 0);
     b.s[i >> 1][i & 1] = __builtin_amdgcn_raw_buffer_load_b16(s.rs, s.vs, os + i * s.ss, 0);
   }
 }

@@ -119,7 +119,7 @@ struct Walk {
   uint32_t vm, vw, bit, byte, gsc;
   int wstride;
   Act act;
-  uint32_t c[8][(CPL + 7) / 8];  // codes of the block
+  uint32_t c[8];  // codes of the block
   uint32_t q[kInt8 ? 8 : 1][kQ];  // its INT8 bytes
   uint32_t flags;                 // bit i: row i is INT8
   uint32_t msc[kG], mw, mo;       // meta of the block after the next
@@ -151,15 +151,10 @@ struct Walk {
     const int oc = row * src.cs;
 #pragma unroll
     for (int i = 2 * h; i < 2 * h + 2; ++i) {
-      if (CPL == 16) {
-        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(src.rc, src.vc, oc + i * src.cs, 0));
-        c[i][0] = v[0];
-        c[i][(CPL + 7) / 8 - 1] = v[1];
-      } else if (CPL == 8) {
-        c[i][0] = __builtin_amdgcn_raw_buffer_load_b32(src.rc, src.vc, oc + i * src.cs, 0);
-      } else {
-        c[i][0] = __builtin_amdgcn_raw_buffer_load_b16(src.rc, src.vc, oc + i * src.cs, 0);
-      }
+      if (CPL == 8)
+        c[i] = __builtin_amdgcn_raw_buffer_load_b32(src.rc, src.vc, oc + i * src.cs, 0);
+      else
+        c[i] = __builtin_amdgcn_raw_buffer_load_b16(src.rc, src.vc, oc + i * src.cs, 0);
     }
   }
   __device__ __forceinline__ void load_meta(int row) {
@@ -192,11 +187,7 @@ struct Walk {
       const bool is8 = (w[j] & bit) != 0u;
       const uint32_t off = is8 ? (o[j] + popc(w[j] & (bit - 1u))) * kGroup + byte : 0x80000000u;
       fl |= is8 ? 1u << (2 * h + j) : 0u;
-      if (CPL == 16) {
-        const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rd, off, 0, 0));
-#pragma unroll
-        for (int t = 0; t < kQ; ++t) q[i][t] = v[t & 3];
-      } else if (CPL == 8) {
+      if (CPL == 8) {
         const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rd, off, 0, 0));
 #pragma unroll
         for (int t = 0; t < kQ; ++t) q[i][t] = v[t & 1];
@@ -229,60 +220,54 @@ struct Walk {
       for (int mb = 0; mb < MB; ++mb) a[mb] = act.get(b, mb);
       act.load(max(0, min(b + 1, b1 - 1)));
       uint32_t fl = 0u;
-      constexpr int kHalf = CPL < 8 ? CPL : 8;
+      // Every level pair of the block first (the scheduling fence keeps the
+      // reads together: left alone, the compiler waited for each one).
+      uint32_t v[4][CPL];
 #pragma unroll
-      for (int hc = 0; hc < CPL; hc += kHalf) {  // eight columns at a time
-        // Every level pair of the block first (the scheduling fence keeps the
-        // reads together: left alone, the compiler waited for each one).
-        uint32_t v[4][kHalf];
+      for (int h = 0; h < 4; ++h) {
+        const uint32_t d0 = c[2 * h], d1 = c[2 * h + 1];
+        // Bytes of (row 2h, row 2h + 1) nibbles: even columns, odd columns.
+        const uint32_t even = (d0 & 0x0F0F0F0Fu) | ((d1 << 4) & 0xF0F0F0F0u);
+        const uint32_t odd = ((d0 >> 4) & 0x0F0F0F0Fu) | (d1 & 0xF0F0F0F0u);
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const uint32_t d0 = c[2 * h][hc / 8], d1 = c[2 * h + 1][hc / 8];
-          // Bytes of (row 2h, row 2h + 1) nibbles: even columns, odd columns.
-          const uint32_t even = (d0 & 0x0F0F0F0Fu) | ((d1 << 4) & 0xF0F0F0F0u);
-          const uint32_t odd = ((d0 >> 4) & 0x0F0F0F0Fu) | (d1 & 0xF0F0F0F0u);
+        for (int j = 0; j < CPL; ++j)
+          v[h][j] = lds_ld<uint32_t>(lut + ((((j & 1) ? odd : even) >> (8 * (j >> 1))) & 0xFFu) * (kCopies * 4));
+      }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int j = 0; j < kHalf; ++j)
-            v[h][j] = lds_ld<uint32_t>(lut + ((((j & 1) ? odd : even) >> (8 * (j >> 1))) & 0xFFu) * (kCopies * 4));
+      for (int h = 0; h < 4; ++h) {
+        half2v s = __builtin_bit_cast(half2v, static_cast<uint32_t>(sc[h])), s8 = {};
+        if (kInt8) {
+          const uint32_t m = ((flags >> (2 * h)) & 1u ? 0xFFFFu : 0u) | ((flags >> (2 * h)) & 2u ? 0xFFFF0000u : 0u);
+          s8 = __builtin_bit_cast(half2v, __builtin_bit_cast(uint32_t, s) & m);
+          s = __builtin_bit_cast(half2v, __builtin_bit_cast(uint32_t, s) & ~m);
         }
-        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          half2v s = __builtin_bit_cast(half2v, static_cast<uint32_t>(sc[h])), s8 = {};
+        for (int j = 0; j < CPL; ++j) {
+          half2v x = __builtin_bit_cast(half2v, v[h][j]);
           if (kInt8) {
-            const uint32_t m = ((flags >> (2 * h)) & 1u ? 0xFFFFu : 0u) | ((flags >> (2 * h)) & 2u ? 0xFFFF0000u : 0u);
-            s8 = __builtin_bit_cast(half2v, __builtin_bit_cast(uint32_t, s) & m);
-            s = __builtin_bit_cast(half2v, __builtin_bit_cast(uint32_t, s) & ~m);
+            // q ^ 0x80 under 0x64: 1024 + q + 128 as fp16, exactly.
+            const int t = kInt8 ? j >> 2 : 0;
+            const uint32_t q0 = q[kInt8 ? 2 * h : 0][t] ^ 0x80808080u;
+            const uint32_t q1 = q[kInt8 ? 2 * h + 1 : 0][t] ^ 0x80808080u;
+            const uint32_t pr = __builtin_amdgcn_perm(q1, q0, (j & 2) ? 0x07030602u : 0x05010400u);
+            const half2v bias = {static_cast<_Float16>(-1152.f), static_cast<_Float16>(-1152.f)};
+            const half2v y = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, pr, (j & 1) ? 0x04030402u : 0x04010400u));
+            x = __builtin_elementwise_fma(x, s, (y + bias) * s8);  // one of the two is zero
+          } else {
+            x = x * s;
           }
-#pragma unroll
-          for (int j = 0; j < kHalf; ++j) {
-            half2v x = __builtin_bit_cast(half2v, v[h][j]);
-            if (kInt8) {
-              // q ^ 0x80 under 0x64: 1024 + q + 128 as fp16, exactly.
-              const int t = kInt8 ? (hc + j) >> 2 : 0;
-              const uint32_t q0 = q[kInt8 ? 2 * h : 0][t] ^ 0x80808080u;
-              const uint32_t q1 = q[kInt8 ? 2 * h + 1 : 0][t] ^ 0x80808080u;
-              const uint32_t pr = __builtin_amdgcn_perm(q1, q0, (j & 2) ? 0x07030602u : 0x05010400u);
-              const half2v bias = {static_cast<_Float16>(-1152.f), static_cast<_Float16>(-1152.f)};
-              const half2v y = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, pr, (j & 1) ? 0x04030402u : 0x04010400u));
-              x = __builtin_elementwise_fma(x, s, (y + bias) * s8);  // one of the two is zero
-            } else {
-              x = x * s;
-            }
-            v[h][j] = __builtin_bit_cast(uint32_t, x);
-          }
-          if (hc + kHalf == CPL) {  // the rows are used: reload them from the next block
-            load_codes(row_of(b + 1), h);
-            load_int8(b + 1, h, fl);
-          }
+          v[h][j] = __builtin_bit_cast(uint32_t, x);
         }
+        load_codes(row_of(b + 1), h);  // the rows are used: reload them from the next block
+        load_int8(b + 1, h, fl);
+      }
 #pragma unroll
-        for (int j = 0; j < kHalf; ++j) {
-          const half8 bv = __builtin_bit_cast(half8, u32x4{v[0][j], v[1][j], v[2][j], v[3][j]});
+      for (int j = 0; j < CPL; ++j) {
+        const half8 bv = __builtin_bit_cast(half8, u32x4{v[0][j], v[1][j], v[2][j], v[3][j]});
 #pragma unroll
-          for (int mb = 0; mb < MB; ++mb)
-            acc[mb][hc + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[mb], bv, acc[mb][hc + j], 0, 0, 0);
-        }
+        for (int mb = 0; mb < MB; ++mb)
+          acc[mb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[mb], bv, acc[mb][j], 0, 0, 0);
       }
       flags = fl;
     }
