@@ -734,8 +734,15 @@ bool supported(const latent_moe_args& a) {
 // 4096, ff 1408, rank 64, top-8: 200 tokens (12 pairs an expert) 99 us at one
 // block and 110 at two, 2000 tokens 674 at one and 568 at four; E 64, d 2048,
 // rank 192, 200 tokens (19 pairs): 124 at one, 116 at two.
+// Above rank 256, four blocks' latents leave LDS for one workgroup per CU, which
+// pays from some 64 pairs an expert (E 64, d 4096, ff 1408, top-8, us at one / two
+// / four blocks): rank 480 50 pairs 328 / 439 / 415, 87 pairs 512 / - / 526, 125
+// pairs 691 / 730 / 706; rank 416 302 / 357 / 341, 478 / - / 441, 645 / 588 / 601.
+// Ordered calls (ff 2048): rank 384 50 pairs 308 / 292 / 339, 81 pairs - / 389 /
+// 416; rank 512 348 / 377 / 392, 125 pairs 707 / 745 / 652.
 int pair_blocks(const Params& p, bool int8) {
   const int64_t per = static_cast<int64_t>(p.T) * p.K / p.a_max;
+  if (!int8 && p.R > 256 && per < (p.ordered ? 96 : 64)) return p.ordered ? 2 : 1;
   return int8 || per < 16 ? 1 : per < 24 ? 2 : 4;
 }
 

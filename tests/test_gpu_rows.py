@@ -126,6 +126,21 @@ def test_rows_pair_blocks(gpu, T, k, mode, wbd):
     assert ref.rel_l2(want, got) <= TOL
 
 
+@pytest.mark.parametrize("R", [288, 416, 512])
+@pytest.mark.parametrize("T", [60, 79, 80])
+def test_rows_pair_blocks_of_high_ranks(gpu, R, T):
+    """Pure NF4 layers above rank 256: 48, 63 and 64 pairs an expert (one block of
+    pairs a pass, then four, whose latents and sums take up to 149 KB of LDS)."""
+    host = synth.make_layer(seed=R, n_expert=5, d=544, ff=576, max_rank=R, ranks=[R, R - 31, 100, R, 260])
+    dev = _rows_layer(host)
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T, host.d)).astype(np.float32)
+    ids, w = routing.softmax_topk(rng.standard_normal((T, 5)), 4)
+    for mode in (0, 1):
+        got, want = _run(gpu, host, dev, x, ids, w, mode=mode)
+        assert ref.rel_l2(want, got) <= TOL
+
+
 @pytest.mark.parametrize("E,T,k", [
     (512, 700, 3),   # rounds of 1024 pairs: two and a part, the most experts they take
     (512, 256, 4),   # exactly one of them
