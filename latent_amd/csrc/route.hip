@@ -603,17 +603,20 @@ __global__ void __launch_bounds__(kTopkWaves * kWave) topk_wave_kernel(Params p)
 }
 
 // split_logits_kernel from this many multiply-adds (T E d).  Both routes in us,
-// MI355X, logits and top-k, bf16 x and fp32 router:
-//   E 256, d 7168:  T 200 26 / 31 (64-row slices), 512 32 / 51, 4096 67 / 364;
-//                   T 128 25 / 26 (fp32 x: 29 / 25)
-//   E 160, d 5120:  T 512 26 / 32, 256 23 / 24 (fp32 x: 26 / 23)
-//   E 64, d 2048:   T 2048 29 / 35, 1024 22 / 21
-// Short batches have too few tiles to hide a workgroup's steps; long ones pay
-// the other route for ceil(d / 64) partials of every logit, written and read.
-constexpr int64_t kSplitMacs = 400000000;
+// MI355X, logits and top-k, split / 64-row slices, fp32 router:
+//                   bf16 x                                fp32 x
+//   E 256, d 7168:  T 128 23 / 25, 200 25 / 30,           128 28 / 26, 200 30 / 31,
+//                   512 29 / 51, 4096 58 / 359            512 33 / 51, 4096 95 / 366
+//   E 160, d 5120:  T 200 21 / 22, 350 22 / 27            256 24 / 23, 350 26 / 26, 512 27 / 31
+//   E 64, d 2048:   T 1024 19 / 21, 2048 24 / 34          1024 21 / 21, 2048 27 / 33
+//   E 1000, d 1408: T 100 30 / 33, 200 34 / 39            200 36 / 38
+// Short batches have too few tiles to hide a workgroup's steps (three-part x has
+// twice as many MFMAs in each); long ones pay the other route for ceil(d / 64)
+// partials of every logit, written and read.
+constexpr int64_t kSplitMacs = 250000000, kSplitMacsF32 = 400000000;
 int64_t split_tokens(const latent_route_args& a) {
-  const int64_t per = a.n_expert * a.n_embd;
-  return per > 0 ? (kSplitMacs + per - 1) / per : 0;
+  const int64_t per = a.n_expert * a.n_embd, macs = a.x_dtype == LATENT_F32 ? kSplitMacsF32 : kSplitMacs;
+  return per > 0 ? (macs + per - 1) / per : 0;
 }
 bool split_applies(const latent_route_args& a) {
   return a.n_tokens >= split_tokens(a) && a.n_embd % kSStep == 0;

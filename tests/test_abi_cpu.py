@@ -270,15 +270,19 @@ def test_route_workspace_is_at_most_one_partial_row_per_64_rows_of_d(L, d, E):
     the workspace of a batch holds every smaller batch."""
     a = L.LatentRouteArgs()
     a.n_embd, a.n_expert, a.n_expert_used = d, E, min(8, E)
-    a.x_dtype = a.router_dtype = L.LATENT_F32
-    last = 0
+    a.router_dtype = L.LATENT_F32
+    last = {L.LATENT_F32: 0, L.LATENT_BF16: 0}
     for T in sorted({1, 2, 31, 64, 200, 285, 512, 1000, 2047, 2048, 3051, 3052, 4096, 8191, 16384, 65537} |
-                    {max(1, 400000000 // (d * E) + i) for i in (-1, 0, 1, 2)}):
+                    {max(1, n // (d * E) + i) for n in (250000000, 400000000) for i in (-1, 0, 1, 2)}):
         a.n_tokens = T
-        n = ctypes.c_size_t(0)
-        assert L.lib.latent_route_workspace_size(ctypes.byref(a), ctypes.byref(n)) == L.LATENT_OK
-        assert last <= n.value <= T * E * 4 * -(-d // 64), (T, n.value)
-        last = n.value
+        size = {}
+        for x in last:
+            a.x_dtype = x
+            n = ctypes.c_size_t(0)
+            assert L.lib.latent_route_workspace_size(ctypes.byref(a), ctypes.byref(n)) == L.LATENT_OK
+            assert last[x] <= n.value <= T * E * 4 * -(-d // 64), (T, n.value)
+            size[x] = last[x] = n.value
+        assert size[L.LATENT_BF16] <= size[L.LATENT_F32]  # latent_amd.router queries for fp32 x
 
 
 def _int8_args(L, T, d, ff, E, k, R):

@@ -53,6 +53,7 @@ def test_route_from_x_matches_oracle(gpu, T, d, E, k, x_dtype, r_dtype):
 
 @pytest.mark.parametrize("T,d,E,k,x_dtype,r_dtype,shift", [
     (220, 7168, 256, 8, "bf16", "f32", 0),    # 128-token tiles, last one ragged
+    (137, 7168, 256, 8, "bf16", "f32", 0),    # the fewest tokens of this shape it takes
     (2049, 7168, 256, 8, "f16", "f32", 0),    # 256-token tiles, one token over
     (1500, 2080, 130, 6, "f32", "f32", 0),    # two experts in the last tile, 65 steps of 32 rows
     (4096, 2048, 64, 6, "bf16", "bf16", 0),
