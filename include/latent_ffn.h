@@ -231,10 +231,12 @@ int latent_moe_check(void* workspace, size_t workspace_bytes, latent_stream_t st
  *       4096 routed pairs, 16-byte aligned x;
  *   4 = multi-kernel fp16-MFMA path on the row layout, taken here when a
  *       factor has INT8 groups: at least 16 routed pairs, max_rank <= 512,
- *       16-byte aligned x (per-expert ranks allowed); factors decoded into
- *       LDS chunk by chunk;
- *   1 = fp32 matrix-core chain: row layout, 32 to 512 routed pairs, at most
- *       512 experts, 16-byte aligned x (INT8 groups allowed); bit-reproducible;
+ *       16-byte aligned x (per-expert ranks allowed); factors go through
+ *       registers, decoded, to the matrix cores; sums meet in fp32 atomics, so
+ *       repeated calls agree to rounding;
+ *   1 = fp32 matrix-core chain ("fused" below): row layout, 32 to 512 routed
+ *       pairs, at most 512 experts, 16-byte aligned x (INT8 groups allowed);
+ *       bit-reproducible;
  *   4 = as above, for the pure-NF4 calls path 1 does not take;
  *   0 = multi-kernel fp32 GEMV path: any call on the row layout.
  * A call in the tile layout that neither path 2 nor 3 takes is

@@ -321,11 +321,11 @@ def _fake_int8_args(L, d, E=512, R=256, ff=512, T=8, k=8):
 
 
 def test_int8_side_buffer_beyond_32_bit_offsets_leaves_the_persistent_kernel(gpu, monkeypatch):
-    """The persistent kernel and the row-layout MFMA phases read INT8 groups
+    """The fp32 matrix-core chain and the row-layout MFMA phases read INT8 groups
     with 32-bit byte offsets: a factor whose side buffer could reach 2^31
     bytes (every group INT8) goes to the multi-kernel fp32 path, one just
     below stays on them (the row-layout MFMA phases by default, the
-    persistent kernel when it is asked for)."""
+    fp32 chain when it is asked for)."""
     import ctypes
 
     from latent_amd import _lib as L

@@ -213,7 +213,7 @@ def test_check_after_timeout_rezeros_control_block(gpu, layer, dev):
     ctrl = _lib.LATENT_NOALLOC_CONTROL_BYTES
     ws[36:40] = torch.tensor([1, 0, 0, 0], dtype=torch.uint8)  # the error word
     ws[192 * 1024 + 4] = 3                                     # a small-batch chain counter
-    ws[4096] = 9                                               # a persistent-kernel ticket
+    ws[4096] = 9                                               # a word no path counts in
     assert gpu.workspace_error(ws) == _lib.LATENT_E_TIMEOUT
     assert int(ws[:ctrl].count_nonzero()) == 0
     assert gpu.workspace_error(ws) == _lib.LATENT_OK

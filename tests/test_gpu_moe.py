@@ -209,8 +209,8 @@ def test_dsv3_decode_parity(gpu, dsv3, B, path, monkeypatch):
     x_t = gsynth.bf16_input(seed=2000 + B, n_tokens=B, d=7168)
     out = gpu.moe_forward(x_t, ids_t, w_t, layer)
     torch.cuda.synchronize()
-    # A second call must reproduce the first: bit for bit on the persistent
-    # decode kernel (fixed summation order, control block left as found) and
+    # A second call must reproduce the first: bit for bit on the fp32 chain
+    # (fixed summation order, control block left as found) and
     # the streaming path (fixed-order reductions); the multi-kernel path
     # accumulates with float atomics, so only to rounding.
     again = gpu.moe_forward(x_t, ids_t, w_t, layer)

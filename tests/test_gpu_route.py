@@ -257,7 +257,7 @@ def test_route_rejects_bad_arguments(gpu):
 
 @pytest.mark.parametrize("T", [2, 8])
 def test_graph_stack_matches_eager_and_oracle(gpu, T):
-    """Three small layers (8 routed pairs: multi-kernel path; 32: persistent kernel)."""
+    """Three small layers (8 routed pairs: multi-kernel path; 32: fp32 chain)."""
     import torch
 
     E, d, ff, R, k, n_layers = 16, 256, 256, 64, 4, 3
@@ -288,7 +288,7 @@ def test_graph_stack_matches_eager_and_oracle(gpu, T):
         assert err <= TOL
         np.testing.assert_array_equal(xs[l + 1].cpu().numpy(), x_l + ys[l].cpu().numpy())
     # Graph replays, with eager work and synchronisations between them.
-    # The persistent kernel (>= 32 pairs) sums in a fixed order; the multi-kernel
+    # The fp32 chain (>= 32 pairs) sums in a fixed order; the multi-kernel
     # path adds workgroup partials with float atomics (order not fixed).
     exact = gpu.moe_path(layers[0], x0, k) == "fused"
     assert exact == (T * k >= 32)

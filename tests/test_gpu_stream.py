@@ -194,7 +194,7 @@ def test_reference_rank_table_at_max_rank_256(gpu, tmp_path, monkeypatch, path):
     assert dev.ranks is None
     monkeypatch.setenv("LATENT_MOE_PATH", path)
     rng = np.random.default_rng(5)
-    T = 40 if path == "fused" else 5  # the persistent kernel takes 32..512 routed pairs
+    T = 40 if path == "fused" else 5  # the fp32 chain takes 32..512 routed pairs
     x = rng.standard_normal((T, 256)).astype(np.float32)
     ids, w = routing.softmax_topk(rng.standard_normal((T, 4)), 2)
     xt = torch.from_numpy(x).cuda()

@@ -85,7 +85,7 @@ def test_noalloc_matches_workspace_entry_dsv3(gpu):
 def test_noalloc_small_layer_paths(gpu, monkeypatch):
     host = synth.make_layer(seed=100, n_expert=16, d=256, ff=512, max_rank=64)
     layer = to_device(host)
-    # persistent kernel (32+ pairs, fixed order) then the multi-kernel path (atomics)
+    # fp32 chain (32+ pairs, fixed order) then the multi-kernel path (atomics)
     for T, exact in ((40, True), (5, False)):
         _compare(gpu, layer, T, 4, seed=200 + T, mode=0, exact=exact)
 
