@@ -1107,13 +1107,13 @@ int choose_path(const latent_moe_args& a) {
   // Measured on MI355X at the DeepSeek-V3 shape (d 7168, ff 2048, 256
   // experts, top-8): below the prefill threshold the streaming MFMA path is
   // the fastest wherever it applies (batch 1: 49 vs 52 us for the
-  // multi-kernel path; batch 8 85 and batch 64 208 us against 109 and 361 us
+  // multi-kernel path; batch 8 85 and batch 64 206 us against 109 and 343 us
   // for the fp32 chain on the row layout of the same layer).  On the row layout:
   //   * with INT8 groups (ranks 64..512, 10 % INT8 groups): the row-layout
-  //     MFMA phases from 16 routed pairs (batch 16 / 64 / 256: 219 / 442 /
-  //     509 us against 632 / 1,549 / 3,633 us for the multi-kernel path);
-  //   * pure NF4: the fp32 chain where it applies (rank 256, batch 16 / 32 /
-  //     64: 182 / 272 / 361 us; 64 experts, d 2048, ff 1408, rank 128, top-6, 24 tokens:
+  //     MFMA phases from 16 routed pairs (batch 16 / 64 / 256: 198 / 400 /
+  //     484 us against 632 / 1,549 / 3,633 us for the multi-kernel path);
+  //   * pure NF4: the fp32 chain where it applies (rank 256, batch 16 / 64:
+  //     183 / 343 us; 64 experts, d 2048, ff 1408, rank 128, top-6, 24 tokens:
   //     45 us against 177 us for the persistent fp32 kernel it replaced).
   const bool int8 = a.gate_a.int8_bitmap || a.gate_b.int8_bitmap || a.up_a.int8_bitmap || a.up_b.int8_bitmap ||
                     a.down_a.int8_bitmap || a.down_b.int8_bitmap;

@@ -22,7 +22,8 @@
 // No LDS round trip for a factor and no barrier in the loop: decoding chunks
 // transposed through LDS, as this file once did, spent two barriers and 64
 // scattered LDS stores a thread on every 8 KB.  DeepSeek-V3 shape, ranks 64 to
-// 512, 10 % INT8 groups: batch 16 328 -> 219 us, batch 256 751 -> 509 us.
+// 512, 10 % INT8 groups: batch 16 328 -> 219 us, batch 256 751 -> 509 us (198 and
+// 484 with what came since).
 //
 // What bounds it with INT8 groups: the decode's VALU (about 390 instructions a
 // block of 32 x 128, half of them for the INT8 bytes, which nearly every wave
