@@ -166,9 +166,11 @@ int latent_moe_ffn_forward(const latent_moe_args* args, latent_stream_t stream);
  * args->workspace and args->workspace_bytes are ignored: scratch comes from a
  * library-owned array of LATENT_NOALLOC_SCRATCH_BYTES on each GPU (held until
  * the process ends); a call that cannot run in that many bytes returns
- * LATENT_E_WORKSPACE.  No call allocates.  Every call on one GPU
- * shares that GPU's array: calls that overlap on one GPU (other streams,
- * other host threads) race; calls in order on one stream do not.
+ * LATENT_E_WORKSPACE, one whose latent_moe_workspace_size is larger runs the
+ * form that needs less (results then agree to rounding).  No call allocates.
+ * Every call on one GPU shares that GPU's array: calls that overlap on one GPU
+ * (other streams, other host threads) race; calls in order on one stream do
+ * not.
  */
 #define LATENT_NOALLOC_SCRATCH_BYTES (64u << 20)
 #define LATENT_NOALLOC_CONTROL_BYTES (256u << 10)
